@@ -69,7 +69,7 @@ def build_oracle() -> None:
 
 
 def build_reference() -> bool:
-    if not os.path.isdir("/root/reference"):
+    if not os.path.isdir("/root/reference/interface"):
         return False
     # the reference builds, then the boundary test shim over the product and oracle libraries
     _run(["make", "-s", "-j8", "-C", ROOT, "-f", "oracle/Makefile.ref", "all", "glue"])
