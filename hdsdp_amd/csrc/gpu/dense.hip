@@ -182,94 +182,6 @@ __global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, T alpha,
             }
 }
 
-// Two successive symmetric rank-K updates of a 64 x 64 tile grid,
-//   C = alpha A1 A1(rows j)^T + beta C,  then  C = alpha A2 A2(rows j)^T + beta C,
-// with C read and written once.  Each product runs the k slabs and MFMAs of
-// gemm_kernel (TA = false, TB = true, B = A) and each update rounds as gemm_kernel's
-// epilogue, so the result is that of two gemm_kernel launches with half the traffic
-// on C.  lin as in gemm_kernel (lower products with a square tile grid).
-template <typename T, bool LOWER>
-__global__ __launch_bounds__(256) void gemm_nt2_kernel(int M, int N, int K, T alpha, const T *A1, const T *A2, int lda,
-                                                       T beta, T *C, int ldc, int lin) {
-    typedef typename Mfma<T>::acc_t acc_t;
-    int bx, by;
-    tile_xy(lin, bx, by, 0);
-    const int i0 = bx * TILE, j0 = by * TILE;
-    if (LOWER && i0 + TILE - 1 < j0) return;
-    __shared__ T As[2][KSTEP][TILE + 1];
-    __shared__ T Bs[2][KSTEP][TILE + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
-    const int lr = lane & 15, lk = lane >> 4;
-    T cin[2][2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = i0 + wi + a * 16 + Mfma<T>::row(lk, r);
-                const int j = j0 + wj + b * 16 + lr;
-                const bool ok = i < M && j < N && (!LOWER || i >= j);
-                cin[a][b][r] = (ok && beta != (T) 0) ? C[i + (long) j * ldc] : (T) 0;
-            }
-    const int nslab = K > 0 ? (K + KSTEP - 1) / KSTEP : 0;
-    acc_t acc[2][2];
-    auto product = [&](const T *A) {
-        for (int a = 0; a < 2; ++a)
-            for (int b = 0; b < 2; ++b) acc[a][b] = (acc_t){0, 0, 0, 0};
-        if (nslab == 0) return;
-        T ra[4], rb[4];
-        tile_fetch<T, false, true>(A, lda, A, lda, M, N, K, i0, j0, 0, tid, ra, rb);
-        tile_stash<T, false, true>(As[0], Bs[0], tid, ra, rb);
-        __syncthreads();
-        for (int sl = 0; sl < nslab; ++sl) {
-            const int cur = sl & 1;
-            const bool more = sl + 1 < nslab;
-            if (more) tile_fetch<T, false, true>(A, lda, A, lda, M, N, K, i0, j0, (sl + 1) * KSTEP, tid, ra, rb);
-#pragma unroll
-            for (int kk = 0; kk < KSTEP; kk += 4) {
-                T a0 = As[cur][kk + lk][wi + lr], a1 = As[cur][kk + lk][wi + 16 + lr];
-                T b0 = Bs[cur][kk + lk][wj + lr], b1 = Bs[cur][kk + lk][wj + 16 + lr];
-                acc[0][0] = Mfma<T>::op(a0, b0, acc[0][0]);
-                acc[0][1] = Mfma<T>::op(a0, b1, acc[0][1]);
-                acc[1][0] = Mfma<T>::op(a1, b0, acc[1][0]);
-                acc[1][1] = Mfma<T>::op(a1, b1, acc[1][1]);
-            }
-            if (more) tile_stash<T, false, true>(As[cur ^ 1], Bs[cur ^ 1], tid, ra, rb);
-            __syncthreads();
-        }
-    };
-    product(A1);
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) cin[a][b][r] = alpha * acc[a][b][r] + beta * cin[a][b][r];
-    product(A2);
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = i0 + wi + a * 16 + Mfma<T>::row(lk, r);
-                const int j = j0 + wj + b * 16 + lr;
-                if (i < M && j < N && (!LOWER || i >= j)) C[i + (long) j * ldc] = alpha * acc[a][b][r] + beta * cin[a][b][r];
-            }
-}
-
-template <typename T>
-static void gemm_nt2(hipStream_t s, int M, int N, int K, T alpha, const T *A1, const T *A2, int lda, T beta, T *C,
-                     int ldc) {
-    if (M <= 0 || N <= 0) return;
-    const int mt = (M + TILE - 1) / TILE, nt = (N + TILE - 1) / TILE;
-    const int lin = (mt == nt) ? 1 : 0;
-    dim3 grid(lin ? mt * (mt + 1) / 2 : mt, lin ? 1 : nt, 1);
-    gemm_nt2_kernel<T, true><<<grid, 256, 0, s>>>(M, N, K, alpha, A1, A2, lda, beta, C, ldc, lin);
-}
-
 // 128 x 128 tiles for large products: four waves, each a 64 x 64 quadrant as 4 x 4
 // MFMA 16x16 accumulators; k slabs of 16 double-buffered in LDS so the global
 // loads of slab s + 1 are in flight while slab s is multiplied (one barrier per slab).
@@ -621,282 +533,22 @@ void gemm_splitk(hipStream_t s, bool transA, bool transB, bool lower, int M, int
 template void gemm_splitk<double>(hipStream_t, bool, bool, bool, int, int, int, double, const double *, int,
                                   const double *, int, double, double *, int, double *, size_t);
 
-// ---- Cholesky ----------------------------------------------------------------
-
-// Column r of L^-1 for the 64 x 64 lower factor held column-major in LDS,
-// Ls[c][q] = L(q, c): forward substitution L x = e_r, every lane reading the same
-// entry of column j (an LDS broadcast).
-template <typename T>
-__device__ inline void leaf_inverse(const T (&Ls)[NB][NB], int r, T (&x)[NB]) {
-    // an opaque copy of r: the identity column is formed here rather than merged with
-    // the callers' identical identity padding (which kept 64 values live and spilled)
-    asm volatile("" : "+v"(r));
-#pragma unroll
-    for (int j = 0; j < NB; ++j) x[j] = (j == r) ? (T) 1 : (T) 0;
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        x[j] = x[j] / Ls[j][j];
-#pragma unroll
-        for (int k = j + 1; k < NB; ++k) x[k] -= Ls[j][k] * x[j];
-        // keeps the (read-only) LDS loads of later steps from being hoisted here,
-        // which would hold thousands of values in registers and spill
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// Eight waves factor a kb x kb diagonal block (kb <= 64) and invert its factor.
-// Thread (w, r) holds row r, columns 8 w .. 8 w + 7, in registers; every column
-// is published in LDS once it is final for the step that needs it:
-//   step j: p = a(j, j); row r: t = a(r, j) / p; a(r, c) -= t a(c, j) for c > j;
-//           column j is then scaled by 1 / sqrt(p), a(j, j) = sqrt(p).
-// The wave owning column j + 1 updates that column first and publishes it before its
-// other updates, and the scaling of each column waits until after the last step (no
-// step reads a scaled column), so only one division, one FMA and one LDS round trip
-// lie between consecutive steps.  Entries above the diagonal are scratch.
-// The inverse X = L^-1 follows by forward substitution, lane r computing column r of
-// X with wave w holding its rows 8 w .. 8 w + 7: after row j is published, the
-// owner of row j + 1 finishes that row (x(j+1) -= L(j+1, j) x(j), then the division
-// by L(j+1, j+1)) and publishes it, and every wave updates its other rows
-// k > j by x(k) -= L(k, j) x(j).  Every entry sees the same operations in the same
-// order as in a one-wave sweep.  Rows and columns beyond kb are the identity.  Writes
-// L (lower) in place and X into Dinv (64 x 64, zeros above); sets *info = k0 + j + 1
-// at the first non-positive pivot.  Eight waves of eight columns take 27 us for a
-// 64 x 64 block in FP64 against 41 us for four waves of sixteen (each step between
-// barriers is half as long, two waves per SIMD) and 28 us for sixteen waves of four.
-constexpr int LEAF_W = 8, LEAF_CW = NB / LEAF_W, LEAF_THREADS = LEAF_W * 64;
-
-template <typename T>
-__global__ __launch_bounds__(LEAF_THREADS) void chol_leaf_kernel(T *A, int lda, int k0, int kb, int *info, T *Dinv,
-                                                                 int ldd) {
-    if (*info) return;
-    __shared__ T Ls[NB][NB];      // Ls[c][q] = entry (q, c)
-    __shared__ T Xs[NB][NB + 1];  // Xs[k][c] = X(k, c)
-    const int r = threadIdx.x & 63, w = threadIdx.x >> 6, c0 = w * LEAF_CW;
-    T a[LEAF_CW], sq[LEAF_CW];
-#pragma unroll
-    for (int i = 0; i < LEAF_CW; ++i) {
-        const int c = c0 + i;
-        T v = (r == c) ? (T) 1 : (T) 0;
-        if (r < kb && c < kb && r >= c) v = A[r + (long) c * lda];
-        a[i] = v;
-        sq[i] = (T) 1;
-    }
-    if (w == 0) Ls[0][r] = a[0];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const int wj = j / LEAF_CW, jj = j % LEAF_CW;
-        const int jn = (j + 1) % LEAF_CW;  // the next column's index in its owner wave
-        const bool last = j + 1 == NB;
-        __syncthreads();  // column j is published
-        const T p = Ls[j][j];
-        if (!(p > (T) 0)) {
-            if (threadIdx.x == 0) *info = k0 + j + 1;
-            return;
-        }
-        if (w == wj) {
-            const T t = a[jj] / p;
-            if (jj + 1 < LEAF_CW) {  // the next column is this wave's: update and publish it first
-                a[jj + 1] -= t * Ls[j][j + 1];
-                Ls[j + 1][r] = a[jj + 1];
-            }
-#pragma unroll
-            for (int i = jj + 2; i < LEAF_CW; ++i) a[i] -= t * Ls[j][c0 + i];
-            sq[jj] = sqrt(p);
-        } else if (w > wj) {
-            const T t = Ls[j][r] / p;
-            if (!last && jn == 0 && w == wj + 1) {  // this wave owns the next column
-                a[0] -= t * Ls[j][c0];
-                Ls[j + 1][r] = a[0];
-#pragma unroll
-                for (int i = 1; i < LEAF_CW; ++i) a[i] -= t * Ls[j][c0 + i];
-            } else {
-#pragma unroll
-                for (int i = 0; i < LEAF_CW; ++i) a[i] -= t * Ls[j][c0 + i];
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < LEAF_CW; ++i) a[i] = (r == c0 + i) ? sq[i] : a[i] / sq[i];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < LEAF_CW; ++i) {
-        const int c = c0 + i;
-        Ls[c][r] = a[i];
-        if (r < kb && c < kb && r >= c) A[r + (long) c * lda] = a[i];
-    }
-    __syncthreads();
-    // forward substitution: lane r builds column r of X, wave w its rows c0 .. c0 + 7
-    T dg[LEAF_CW], sub[LEAF_CW];  // L(k, k) and L(k, k - 1) of this wave's rows k
-#pragma unroll
-    for (int i = 0; i < LEAF_CW; ++i) {
-        dg[i] = Ls[c0 + i][c0 + i];
-        sub[i] = (c0 + i > 0) ? Ls[c0 + i - 1][c0 + i] : (T) 0;
-    }
-    int rr = r;
-    asm volatile("" : "+v"(rr));  // identity formed here, not merged with the padding above
-    T x[LEAF_CW];
-#pragma unroll
-    for (int i = 0; i < LEAF_CW; ++i) x[i] = (c0 + i == rr) ? (T) 1 : (T) 0;
-    if (w == 0) {
-        x[0] = x[0] / dg[0];
-        Xs[0][r] = x[0];
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const int wj = j / LEAF_CW, jj = j % LEAF_CW;
-        const int jn = (j + 1) % LEAF_CW;
-        const bool last = j + 1 == NB;
-        __syncthreads();  // row j of X is published
-        if (w == wj) {
-            const T xj = x[jj];
-            if (jj + 1 < LEAF_CW) {  // finish and publish the next row first
-                x[jj + 1] -= sub[jj + 1] * xj;
-                x[jj + 1] = x[jj + 1] / dg[jj + 1];
-                Xs[j + 1][r] = x[jj + 1];
-            }
-#pragma unroll
-            for (int i = jj + 2; i < LEAF_CW; ++i) x[i] -= Ls[j][c0 + i] * xj;
-        } else if (w > wj) {
-            const T xj = Xs[j][r];
-            if (!last && jn == 0 && w == wj + 1) {
-                x[0] -= sub[0] * xj;
-                x[0] = x[0] / dg[0];
-                Xs[j + 1][r] = x[0];
-#pragma unroll
-                for (int i = 1; i < LEAF_CW; ++i) x[i] -= Ls[j][c0 + i] * xj;
-            } else {
-#pragma unroll
-                for (int i = 0; i < LEAF_CW; ++i) x[i] -= Ls[j][c0 + i] * xj;
-            }
-        }
-    }
-    __syncthreads();
-    // Dinv(q, c) = X(q, c) below the diagonal, stored row-coalesced: lane q writes row q
-    for (int c = c0; c < c0 + LEAF_CW; ++c) Dinv[r + (long) c * ldd] = (r >= c) ? Xs[r][c] : (T) 0;
-}
-
-// Right-looking blocked Cholesky.  Per block column k (width NB):
-//   leaf:  factor the diagonal block and invert its factor (work)
-//   panel: P = P L11^-T as a GEMM with that inverse
-//   trail: A22 -= P P^T (lower)
-// With look-ahead the trailing update is split: the next block column's part runs on
-// s (so that the next leaf and panel can start at once), the rest on s2; the next
-// block column's own update waits for s2's previous update through an event.
-template <typename T>
-bool potrf(hipStream_t s, int n, T *A, int lda, T *work, size_t workLen, int *info, const LookAhead *la) {
-    if (workLen < POTRF_WORK) {
-        fprintf(stderr, "[hdsdp_amd] potrf: work of %zu elements, %zu needed\n", workLen, POTRF_WORK);
-        return false;
-    }
-    hipMemsetAsync(info, 0, sizeof(int), s);
-    auto at = [&](int i, int j) { return A + i + (long) j * lda; };
-    auto leaf = [&](int k0) {
-        const int kb = (n - k0 < NB) ? n - k0 : NB;
-        chol_leaf_kernel<T><<<1, LEAF_THREADS, 0, s>>>(at(k0, k0), lda, k0, kb, info, work, NB);
-        if (k0 + kb < n)
-            gemm<T>(s, false, true, false, n - k0 - kb, kb, kb, (T) 1, at(k0 + kb, k0), lda, 0, work, NB, 0, (T) 0,
-                    at(k0 + kb, k0), lda, 0, 1);
-    };
-    if (!la || n <= 4 * NB) {
-        for (int k0 = 0; k0 < n; k0 += NB) {
-            leaf(k0);
-            const int k1 = k0 + NB;
-            if (k1 < n)
-                gemm<T>(s, false, true, true, n - k1, n - k1, NB, (T) -1, at(k1, k0), lda, 0, at(k1, k0), lda, 0,
-                        (T) 1, at(k1, k1), lda, 0, 1);
-        }
-        return true;
-    }
-    // Block columns are taken in pairs (a, b = a + NB): the update of a's panel to the
-    // blocks from a + 2 NB on waits for b's panel, and then both updates run as one pass
-    // over the trailing matrix (gemm_nt2: the two updates in order, C read and written
-    // once; the trailing updates are bound by that traffic).  The next block column is
-    // always updated on s, ahead of its leaf; the rest on s2, overlapping the next leaves.
-    int ring = 0;
-    bool s2dirty = false;  // s2 holds an update that s has not yet waited for
-    hipEvent_t evB = nullptr;
-    int kDef = -1;  // first panel of an open pair
-    leaf(0);
-    for (int k0 = 0;; k0 += NB) {
-        const int k1 = k0 + NB;
-        if (k1 >= n) break;
-        const int nb1 = (n - k1 < NB) ? n - k1 : NB, k2 = k1 + nb1;
-        if (kDef < 0) {
-            if (k2 < n) kDef = k0;  // this panel's update of blocks from k2 on waits for the next panel
-            if (s2dirty) {
-                hipStreamWaitEvent(s, evB, 0);  // the previous pair's update reached block k1
-                s2dirty = false;
-            }
-            gemm<T>(s, false, true, true, n - k1, nb1, NB, (T) -1, at(k1, k0), lda, 0, at(k1, k0), lda, 0, (T) 1,
-                    at(k1, k1), lda, 0, 1);
-        } else {
-            if (k2 < n) {
-                hipEvent_t evP = la->ev[ring++ % LA_EVENTS];
-                hipEventRecord(evP, s);
-                hipStreamWaitEvent(la->s2, evP, 0);
-                gemm_nt2<T>(la->s2, n - k2, n - k2, NB, (T) -1, at(k2, kDef), at(k2, k0), lda, (T) 1, at(k2, k2),
-                            lda);
-                evB = la->ev[ring++ % LA_EVENTS];
-                hipEventRecord(evB, la->s2);
-                s2dirty = true;
-            }
-            gemm_nt2<T>(s, n - k1, nb1, NB, (T) -1, at(k1, kDef), at(k1, k0), lda, (T) 1, at(k1, k1), lda);
-            kDef = -1;
-        }
-        leaf(k1);
-    }
-    if (s2dirty) hipStreamWaitEvent(s, evB, 0);
-    return true;
-}
-
-template bool potrf<double>(hipStream_t, int, double *, int, double *, size_t, int *, const LookAhead *);
-template bool potrf<float>(hipStream_t, int, float *, int, float *, size_t, int *, const LookAhead *);
-
 // ---- triangular inverse ------------------------------------------------------
 
-// Inverse of each 64 x 64 diagonal block of the lower factor (the last one may be
-// smaller, padded with the identity): one wave per block, lane q loads row q and
-// stores it to LDS as column-major L for the broadcast reads of the substitution.
+// Linv = the inverses of the 64 x 64 diagonal blocks, zero elsewhere
 template <typename T>
-__global__ __launch_bounds__(64) void trtri_diag_kernel(int n, const T *L, int ldl, T *Linv, int ldi) {
-    const int o = blockIdx.x * NB;
-    const int kb = (n - o < NB) ? n - o : NB;
-    const int r = threadIdx.x;
-    __shared__ T Ls[NB][NB];
-#pragma unroll
-    for (int c = 0; c < NB; ++c) {
-        T v = (r == c) ? (T) 1 : (T) 0;
-        if (r < kb && c < kb && r >= c) v = L[(o + r) + (long) (o + c) * ldl];
-        Ls[c][r] = v;
-    }
-    __syncthreads();
-    T x[NB];
-    leaf_inverse<T>(Ls, r, x);
-    __syncthreads();
-    // column r of the inverse back into LDS, then stored row by row (lane q writes row q)
-#pragma unroll
-    for (int k = 0; k < NB; ++k) Ls[r][k] = (k >= r) ? x[k] : (T) 0;
-    __syncthreads();
-    for (int c = 0; c < kb; ++c)
-        if (r < kb) Linv[(o + r) + (long) (o + c) * ldi] = Ls[c][r];
-}
-
-template <typename T>
-__global__ void fill_matrix_kernel(int n, T *A, int lda, T v) {
-    long total = (long) n * n;
-    for (long e = blockIdx.x * (long) blockDim.x + threadIdx.x; e < total; e += (long) gridDim.x * blockDim.x) {
-        long i = e % n, j = e / n;
-        A[i + j * lda] = v;
-    }
+__global__ void place_diag_kernel(int n, const double *Dinv, T *Linv, long ldi) {
+    const int j = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const bool in = (i >> 6) == (j >> 6);
+    Linv[i + j * ldi] = in ? (T) Dinv[(long) (j >> 6) * NB * NB + (i & 63) + 64 * (j & 63)] : (T) 0;
 }
 
 // inv([[A, 0], [B, C]]) = [[A^-1, 0], [-C^-1 B A^-1, C^-1]], applied level by level
 // with every pair of one level batched into two GEMMs.
 template <typename T>
-void trtri(hipStream_t s, int n, const T *L, int ldl, T *Linv, int ldi, T *work) {
-    fill_matrix_kernel<T><<<512, 256, 0, s>>>(n, Linv, ldi, (T) 0);
-    int nblk = (n + NB - 1) / NB;
-    trtri_diag_kernel<T><<<nblk, NB, 0, s>>>(n, L, ldl, Linv, ldi);
+void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work) {
+    place_diag_kernel<T><<<dim3((n + 255) / 256, n), 256, 0, s>>>(n, Dinv, Linv, ldi);
     for (int sz = NB; sz < n; sz *= 2) {
         int npair = n / (2 * sz);
         long strideL = 2L * sz * (ldl + 1), strideI = 2L * sz * (ldi + 1), strideW = (long) sz * sz;
@@ -918,8 +570,8 @@ void trtri(hipStream_t s, int n, const T *L, int ldl, T *Linv, int ldi, T *work)
     }
 }
 
-template void trtri<double>(hipStream_t, int, const double *, int, double *, int, double *);
-template void trtri<float>(hipStream_t, int, const float *, int, float *, int, float *);
+template void trtri<double>(hipStream_t, int, const double *, int, const double *, double *, int, double *);
+template void trtri<float>(hipStream_t, int, const float *, int, const double *, float *, int, float *);
 
 // ---- matrix-vector ------------------------------------------------------------
 

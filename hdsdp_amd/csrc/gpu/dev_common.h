@@ -61,21 +61,21 @@ struct LookAhead {
     hipEvent_t ev[LA_EVENTS];
 };
 
-// In-place lower Cholesky of the n x n matrix A (lda), blocked by NB.
-// work: scratch of workLen >= POTRF_WORK elements (the leaf writes the NB x NB inverse
-// of every diagonal block, padded with the identity, whatever n is); info: device int,
-// 0 on success else failing column + 1.  Returns false, launching nothing, when
-// workLen is too small.  With la, the bulk of each trailing update runs on la->s2
-// while the next block column is factored on s; s has waited for s2 when the call
-// returns.
-constexpr size_t POTRF_WORK = (size_t) NB * NB;
+// Lower Cholesky A = L L^T of the n x n matrix A (lower triangle, destroyed), blocked by
+// NB.  L (n x n, lower triangle written) and A are distinct.  Dinv: chol_dinv_len(n)
+// doubles, the inverses of L's 64 x 64 diagonal blocks (column-major, zeros above the
+// diagonal, the last one padded with the identity).  info: device int, set to 0 on
+// success else failing column + 1.  With la, the bulk of each trailing update of a large
+// matrix runs on la->s2 while the next block columns are factored on s; s has waited for
+// s2 when the call returns.
+inline size_t chol_dinv_len(size_t n) { return (n + NB - 1) / NB * NB * NB; }
 template <typename T>
-bool potrf(hipStream_t s, int n, T *A, int lda, T *work, size_t workLen, int *info, const LookAhead *la = nullptr);
+void potrf(hipStream_t s, int n, T *A, int lda, T *L, int ldl, double *Dinv, int *info, const LookAhead *la = nullptr);
 
-// Linv = L^-1 for the lower-triangular n x n factor L (upper of Linv zeroed).
-// work: n * n scratch.
+// Linv = L^-1 for the lower-triangular n x n factor L (upper of Linv zeroed) with the
+// inverses Dinv of its diagonal blocks.  work: n * n scratch.
 template <typename T>
-void trtri(hipStream_t s, int n, const T *L, int ldl, T *Linv, int ldi, T *work);
+void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work);
 
 // In-place LU with partial pivoting, P A = L U (L unit lower, U upper, both in A),
 // blocked by 64 columns.  ipiv (device, m ints): row interchanged with row c at step c,

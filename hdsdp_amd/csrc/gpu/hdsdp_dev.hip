@@ -68,6 +68,7 @@ struct hdsdp_dev {
     size_t splitLen;
 
     double *S[3], *L[2], *Li[2], *LiT[2];
+    double *Ld[2];  // inverses of the factors' 64 x 64 diagonal blocks
     long facVer[2], liVer[2];
     double *W, *W2, *X, *T1, *T2, *work;
     double *coef_d, *vecA_d, *vecB_d, *sc_d;
@@ -84,7 +85,7 @@ struct hdsdp_dev {
     // primal method (interface/hdsdp_psdp.c): the primal iterate is X; Xs its value at the
     // start (the fixed scaling), dXp the direction, XSX the buffer X S X (+ Xs dS Xs), Sold
     // the dual matrix of the iteration, LX / LXi / LXiT the Cholesky factor of X and inverses
-    double *Xs, *dXp, *XSX, *Sold, *LX, *LXi, *LXiT;
+    double *Xs, *dXp, *XSX, *Sold, *LX, *LXi, *LXiT, *LXd;
     double *lzHist;  // (alpha_k, ||w_k||) of every Lanczos step, read at the check steps
     double *symvW;   // tile partials of the lower-triangle product with M (large m), else null
     std::vector<double> Hh;
@@ -93,7 +94,7 @@ struct hdsdp_dev {
     // Schur system; mVer counts changes of M, cholVer is the mVer its FP64 factor
     // (Mchol, MLi, MLiT) was computed from (-1: none)
     long mVer, cholVer;
-    double *M, *Mchol, *MLi, *MLiT;
+    double *M, *Mchol, *MLi, *MLiT, *Md;  // Md: inverses of the diagonal blocks of either factor of M
     float *Mf, *MLif, *MLiTf, *cf1, *cf2, *workf;
     double *jac, *cr, *crn, *cp, *cz, *cMp, *cx, *crhs, *ctmp;
     double *precS;     // Jacobi scaling of the FP32 preconditioner
@@ -216,7 +217,7 @@ hdsdp_retcode prof_end(hdsdp_dev *d, int k) {
 
 hdsdp_retcode ensure_linv(hdsdp_dev *d, int f) {
     if (d->liVer[f] == d->facVer[f]) return HDSDP_RETCODE_OK;
-    hdk::trtri<double>(d->st, d->n, d->L[f], d->n, d->Li[f], d->n, d->work);
+    hdk::trtri<double>(d->st, d->n, d->L[f], d->n, d->Ld[f], d->Li[f], d->n, d->work);
     hdk::transpose<double>(d->st, d->n, d->Li[f], d->n, d->LiT[f], d->n);
     d->liVer[f] = d->facVer[f];
     return check_launch();
@@ -352,17 +353,16 @@ hdsdp_retcode build_chol64(hdsdp_dev *d) {
     if (!d->Mchol) {
         DCALL(dalloc(d, &d->Mchol, (size_t) m * m));
         DCALL(dalloc(d, &d->MLi, (size_t) m * m));
-        DCALL(dalloc(d, &d->MLiT, std::max((size_t) m * m, hdk::POTRF_WORK)));
+        DCALL(dalloc(d, &d->MLiT, (size_t) m * m));
     }
-    HIP_OK(hipMemcpyAsync(d->Mchol, d->M, sizeof(double) * (size_t) m * m, hipMemcpyDeviceToDevice, d->st));
+    if (!d->Md) DCALL(dalloc(d, &d->Md, hdk::chol_dinv_len(m)));
+    HIP_OK(hipMemcpyAsync(d->MLiT, d->M, sizeof(double) * (size_t) m * m, hipMemcpyDeviceToDevice, d->st));
     d->cholVer = -1;
-    if (!hdk::potrf<double>(d->st, m, d->Mchol, m, d->MLiT, std::max((size_t) m * m, hdk::POTRF_WORK), d->info_d,
-                            &d->la))
-        return HDSDP_RETCODE_FAILED;
+    hdk::potrf<double>(d->st, m, d->MLiT, m, d->Mchol, m, d->Md, d->info_d, &d->la);
     HIP_OK(hipMemcpyAsync(d->hinfo, d->info_d, sizeof(int), hipMemcpyDeviceToHost, d->st));
     DCALL(sync(d));
     if (*d->hinfo != 0) return HDSDP_RETCODE_FAILED;
-    hdk::trtri<double>(d->st, m, d->Mchol, m, d->MLi, m, d->MLiT);
+    hdk::trtri<double>(d->st, m, d->Mchol, m, d->Md, d->MLi, m, d->MLiT);
     hdk::transpose<double>(d->st, m, d->MLi, m, d->MLiT, m);
     d->precKind = PREC_CHOL64;
     d->cholVer = d->mVer;
@@ -381,9 +381,10 @@ hdsdp_retcode build_chol32(hdsdp_dev *d, int *ok) {
         DCALL(dalloc(d, &d->MLiTf, (size_t) m * m));
         DCALL(dalloc(d, &d->cf1, (size_t) m));
         DCALL(dalloc(d, &d->cf2, (size_t) m));
-        DCALL(dalloc(d, &d->workf, std::max((size_t) m * m, hdk::POTRF_WORK)));
+        DCALL(dalloc(d, &d->workf, (size_t) m * m));
         DCALL(dalloc(d, &d->precS, (size_t) m));
     }
+    if (!d->Md) DCALL(dalloc(d, &d->Md, hdk::chol_dinv_len(m)));
     *ok = 0;
     hdk::jacobi_scale(d->st, m, d->M, m, d->precS);
     // M only grows more ill-conditioned along the path: start from the shift the
@@ -391,10 +392,8 @@ hdsdp_retcode build_chol32(hdsdp_dev *d, int *ok) {
     const double shifts[] = {0.0, 1e-6, 1e-5, 1e-4, 1e-3, 1e-2};
     for (double shift : shifts) {
         if (shift < d->precShift) continue;
-        hdk::convert_lower_scaled(d->st, m, d->M, m, d->precS, shift, d->Mf, m);
-        if (!hdk::potrf<float>(d->st, m, d->Mf, m, d->workf, std::max((size_t) m * m, hdk::POTRF_WORK), d->info_d,
-                               &d->la))
-            return HDSDP_RETCODE_FAILED;
+        hdk::convert_lower_scaled(d->st, m, d->M, m, d->precS, shift, d->workf, m);
+        hdk::potrf<float>(d->st, m, d->workf, m, d->Mf, m, d->Md, d->info_d, &d->la);
         HIP_OK(hipMemcpyAsync(d->hinfo, d->info_d, sizeof(int), hipMemcpyDeviceToHost, d->st));
         DCALL(sync(d));
         if (*d->hinfo == 0) {
@@ -404,7 +403,7 @@ hdsdp_retcode build_chol32(hdsdp_dev *d, int *ok) {
         }
     }
     if (!*ok) return HDSDP_RETCODE_OK;
-    hdk::trtri<float>(d->st, m, d->Mf, m, d->MLif, m, d->workf);
+    hdk::trtri<float>(d->st, m, d->Mf, m, d->Md, d->MLif, m, d->workf);
     hdk::transpose<float>(d->st, m, d->MLif, m, d->MLiTf, m);
     d->precKind = PREC_CHOL32;
     return check_launch();
@@ -808,13 +807,14 @@ hdsdp_retcode hdsdp_dev_create(hdsdp_dev **pdev, int nRow, int nCol, int precisi
         DCALL(dalloc(d, &d->L[k], nn));
         DCALL(dalloc(d, &d->Li[k], nn));
         DCALL(dalloc(d, &d->LiT[k], nn));
+        DCALL(dalloc(d, &d->Ld[k], hdk::chol_dinv_len(n)));
         d->facVer[k] = 0;
         d->liVer[k] = -1;
     }
     DCALL(dalloc(d, &d->W, nn));
     DCALL(dalloc(d, &d->W2, nn));
     DCALL(dalloc(d, &d->X, nn));
-    DCALL(dalloc(d, &d->T1, std::max(nn, hdk::POTRF_WORK)));
+    DCALL(dalloc(d, &d->T1, nn));
     DCALL(dalloc(d, &d->T2, nn));
     DCALL(dalloc(d, &d->coef_d, m + 1));
     DCALL(dalloc(d, &d->vecA_d, m + 1));
@@ -1309,10 +1309,8 @@ hdsdp_retcode hdsdp_dev_update_buffer(hdsdp_dev *d, double cCoef, double aScal, 
 hdsdp_retcode hdsdp_dev_factorize(hdsdp_dev *d, int which, int *isPsd) {
     const int n = d->n, f = fidx(which);
     prof_begin(d, HDSDP_PROF_SFACTOR);
-    HIP_OK(hipMemcpyAsync(d->L[f], d->S[f], sizeof(double) * (size_t) n * n, hipMemcpyDeviceToDevice, d->st));
-    if (!hdk::potrf<double>(d->st, n, d->L[f], n, d->T1, std::max((size_t) n * n, hdk::POTRF_WORK), d->info_d,
-                            &d->la))
-        return HDSDP_RETCODE_FAILED;
+    HIP_OK(hipMemcpyAsync(d->T1, d->S[f], sizeof(double) * (size_t) n * n, hipMemcpyDeviceToDevice, d->st));
+    hdk::potrf<double>(d->st, n, d->T1, n, d->L[f], n, d->Ld[f], d->info_d, &d->la);
     HIP_OK(hipMemcpyAsync(d->hinfo, d->info_d, sizeof(int), hipMemcpyDeviceToHost, d->st));
     DCALL(prof_end(d, HDSDP_PROF_SFACTOR));
     DCALL(sync(d));
@@ -1723,14 +1721,13 @@ namespace {
 // (HFpLinsysNumeric / HFpLinsysPsdCheck on the dense solver, linalg/hdsdp_linsolver.c:525-560).
 hdsdp_retcode factor_x(hdsdp_dev *d, int *isPsd) {
     const int n = d->n;
-    HIP_OK(hipMemcpyAsync(d->LX, d->X, sizeof(double) * (size_t) n * n, hipMemcpyDeviceToDevice, d->st));
-    if (!hdk::potrf<double>(d->st, n, d->LX, n, d->T1, std::max((size_t) n * n, hdk::POTRF_WORK), d->info_d, &d->la))
-        return HDSDP_RETCODE_FAILED;
+    HIP_OK(hipMemcpyAsync(d->T1, d->X, sizeof(double) * (size_t) n * n, hipMemcpyDeviceToDevice, d->st));
+    hdk::potrf<double>(d->st, n, d->T1, n, d->LX, n, d->LXd, d->info_d, &d->la);
     HIP_OK(hipMemcpyAsync(d->hinfo, d->info_d, sizeof(int), hipMemcpyDeviceToHost, d->st));
     DCALL(sync(d));
     *isPsd = (*d->hinfo == 0);
     if (!*isPsd) return HDSDP_RETCODE_OK;
-    hdk::trtri<double>(d->st, n, d->LX, n, d->LXi, n, d->work);
+    hdk::trtri<double>(d->st, n, d->LX, n, d->LXd, d->LXi, n, d->work);
     hdk::transpose<double>(d->st, n, d->LXi, n, d->LXiT, n);
     return check_launch();
 }
@@ -1748,6 +1745,7 @@ hdsdp_retcode hdsdp_dev_psdp_init(hdsdp_dev *d) {
         DCALL(dalloc(d, &d->LX, nn));
         DCALL(dalloc(d, &d->LXi, nn));
         DCALL(dalloc(d, &d->LXiT, nn));
+        DCALL(dalloc(d, &d->LXd, hdk::chol_dinv_len(n)));
         DCALL(dalloc(d, &d->lwarmP, n));
     }
     HIP_OK(hipMemcpyAsync(d->Xs, d->X, sizeof(double) * nn, hipMemcpyDeviceToDevice, d->st));

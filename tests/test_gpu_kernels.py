@@ -378,3 +378,48 @@ def test_blocked_cholesky_look_ahead(gpu_lib, n):
         assert g.factorize(1) == 0
     finally:
         g.close()
+
+
+def _spd_coeffs(n, rng, flip=None):
+    """C = 4 I + a symmetric part of norm below 2.5 (condition below 5), two diagonal
+    constraints; flip: index of a diagonal entry made negative."""
+    G = rng.standard_normal((n, n)) / np.sqrt(n)
+    S = 4.0 * np.eye(n) + 0.6 * (G + G.T) / np.sqrt(2.0)
+    if flip is not None:
+        S[flip, flip] = -1.0
+    packed = np.concatenate([S[j:, j] for j in range(n)])
+    one = np.ones(1)
+    con = [dt.Coeff(dt.SPARSE, n, row=[k], col=[k], val=one) for k in (0, n - 1)]
+    return S, [dt.Coeff(dt.DENSE, n, val=packed)] + con
+
+
+# block (16), tile (64) and launch (48 tiles) edges of the blocked Cholesky
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 80, 127, 129, 500, 3072, 3073, 3140])
+def test_cholesky_block_edges(gpu_lib, n):
+    """Factor, log det and inverse entries of S at the edges of the blocked Cholesky.
+    Bounds: n-term sums with unit roundoff u = 1.1e-16 and condition kappa < 5 give a
+    relative error of the factor of n u, so |log det| moves by at most 2 n (n u kappa) and
+    entries of S^-1 by (3 n u kappa) |S^-1|."""
+    rng = np.random.default_rng(n)
+    S, coeffs = _spd_coeffs(n, rng)
+    d = dt.Dev(gpu_lib, coeffs)
+    d.update(1.0, 0.0, np.zeros(2), 0.0, 0)
+    assert d.factorize(0) == 1
+    u = 1.1e-16
+    assert abs(d.logdet(0) - np.linalg.slogdet(S)[1]) <= 10.0 * n * n * u + 1e-15
+    a, _, _ = d.schur(1, 0.0)
+    W = np.linalg.inv(S)
+    assert np.max(np.abs(a - np.array([W[0, 0], W[-1, -1]]))) <= (15.0 * n + 20.0) * u
+    d.close()
+
+
+@pytest.mark.parametrize("n,flip", [(1, 0), (16, 15), (64, 0), (64, 16), (64, 63), (65, 64), (200, 137), (3100, 3080)])
+def test_cholesky_flags_a_negative_pivot(gpu_lib, n, flip):
+    """A negative diagonal entry in any 16-column block, tile or outer block of the Cholesky."""
+    _, coeffs = _spd_coeffs(n, np.random.default_rng(n), flip)
+    d = dt.Dev(gpu_lib, coeffs)
+    d.update(1.0, 0.0, np.zeros(2), 0.0, 1)
+    assert d.factorize(1) == 0
+    d.update(1.0, 0.0, np.zeros(2), 8.0, 1)  # the shifted matrix is positive definite
+    assert d.factorize(1) == 1
+    d.close()
