@@ -73,9 +73,18 @@ template <typename T>
 void potrf(hipStream_t s, int n, T *A, int lda, T *L, int ldl, double *Dinv, int *info, const LookAhead *la = nullptr);
 
 // Linv = L^-1 for the lower-triangular n x n factor L (upper of Linv zeroed) with the
-// inverses Dinv of its diagonal blocks.  work: n * n scratch.
+// inverses Dinv of its diagonal blocks.  work: n * n scratch.  With span (a power-of-two
+// multiple of NB), only the diagonal blocks of span rows are inverted, each in its place.
 template <typename T>
-void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work);
+void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work, int span = 0);
+
+// A Cholesky factor L (lower triangle of an m x m matrix, whose upper triangle it may
+// overwrite) as a preconditioner: prepare fills Li and LiT (m x m each, ld as L's), apply
+// computes z = L^-T L^-1 r with tmp of m entries; r, z and tmp distinct.
+template <typename T>
+void solve_prepare(hipStream_t s, int m, T *L, int ld, const double *Dinv, T *Li, T *LiT);
+template <typename T>
+void solve_apply(hipStream_t s, int m, const T *L, int ld, const T *Li, const T *LiT, const T *r, T *z, T *tmp);
 
 // In-place LU with partial pivoting, P A = L U (L unit lower, U upper, both in A),
 // blocked by 64 columns.  ipiv (device, m ints): row interchanged with row c at step c,

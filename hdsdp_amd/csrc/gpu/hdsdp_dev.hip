@@ -92,10 +92,10 @@ struct hdsdp_dev {
     std::vector<double> lzStart, lzPert;  // Lanczos start vector and warm-start perturbation (fixed by n)
 
     // Schur system; mVer counts changes of M, cholVer is the mVer its FP64 factor
-    // (Mchol, MLi, MLiT) was computed from (-1: none)
+    // (Mchol and the inverses of its diagonal blocks, MLi, MLiT) was computed from (-1: none)
     long mVer, cholVer;
     double *M, *Mchol, *MLi, *MLiT, *Md;  // Md: inverses of the diagonal blocks of either factor of M
-    float *Mf, *MLif, *MLiTf, *cf1, *cf2, *workf;
+    float *Mf, *MLif, *MLiTf, *cf1, *cf2, *cf3;
     double *jac, *cr, *crn, *cp, *cz, *cMp, *cx, *crhs, *ctmp;
     double *precS;     // Jacobi scaling of the FP32 preconditioner
     double precShift;  // diagonal shift the FP32 factorisation needed
@@ -347,7 +347,7 @@ hdsdp_retcode lanczos(hdsdp_dev *d, const LzOp &op, double *maxStep) {
     return check_launch();
 }
 
-// FP64 Cholesky preconditioner: M = L L^T, kept as L^-1 and L^-T.
+// FP64 Cholesky preconditioner: M = L L^T, with the inverses of diagonal blocks of L.
 hdsdp_retcode build_chol64(hdsdp_dev *d) {
     const int m = d->m;
     if (!d->Mchol) {
@@ -362,8 +362,7 @@ hdsdp_retcode build_chol64(hdsdp_dev *d) {
     HIP_OK(hipMemcpyAsync(d->hinfo, d->info_d, sizeof(int), hipMemcpyDeviceToHost, d->st));
     DCALL(sync(d));
     if (*d->hinfo != 0) return HDSDP_RETCODE_FAILED;
-    hdk::trtri<double>(d->st, m, d->Mchol, m, d->Md, d->MLi, m, d->MLiT);
-    hdk::transpose<double>(d->st, m, d->MLi, m, d->MLiT, m);
+    hdk::solve_prepare<double>(d->st, m, d->Mchol, m, d->Md, d->MLi, d->MLiT);
     d->precKind = PREC_CHOL64;
     d->cholVer = d->mVer;
     return check_launch();
@@ -381,7 +380,7 @@ hdsdp_retcode build_chol32(hdsdp_dev *d, int *ok) {
         DCALL(dalloc(d, &d->MLiTf, (size_t) m * m));
         DCALL(dalloc(d, &d->cf1, (size_t) m));
         DCALL(dalloc(d, &d->cf2, (size_t) m));
-        DCALL(dalloc(d, &d->workf, (size_t) m * m));
+        DCALL(dalloc(d, &d->cf3, (size_t) m));
         DCALL(dalloc(d, &d->precS, (size_t) m));
     }
     if (!d->Md) DCALL(dalloc(d, &d->Md, hdk::chol_dinv_len(m)));
@@ -392,8 +391,8 @@ hdsdp_retcode build_chol32(hdsdp_dev *d, int *ok) {
     const double shifts[] = {0.0, 1e-6, 1e-5, 1e-4, 1e-3, 1e-2};
     for (double shift : shifts) {
         if (shift < d->precShift) continue;
-        hdk::convert_lower_scaled(d->st, m, d->M, m, d->precS, shift, d->workf, m);
-        hdk::potrf<float>(d->st, m, d->workf, m, d->Mf, m, d->Md, d->info_d, &d->la);
+        hdk::convert_lower_scaled(d->st, m, d->M, m, d->precS, shift, d->MLiTf, m);
+        hdk::potrf<float>(d->st, m, d->MLiTf, m, d->Mf, m, d->Md, d->info_d, &d->la);
         HIP_OK(hipMemcpyAsync(d->hinfo, d->info_d, sizeof(int), hipMemcpyDeviceToHost, d->st));
         DCALL(sync(d));
         if (*d->hinfo == 0) {
@@ -403,8 +402,7 @@ hdsdp_retcode build_chol32(hdsdp_dev *d, int *ok) {
         }
     }
     if (!*ok) return HDSDP_RETCODE_OK;
-    hdk::trtri<float>(d->st, m, d->Mf, m, d->Md, d->MLif, m, d->workf);
-    hdk::transpose<float>(d->st, m, d->MLif, m, d->MLiTf, m);
+    hdk::solve_prepare<float>(d->st, m, d->Mf, m, d->Md, d->MLif, d->MLiTf);
     d->precKind = PREC_CHOL32;
     return check_launch();
 }
@@ -442,12 +440,10 @@ void apply_precond(hdsdp_dev *d, const double *r, double *z, double *p) {
     if (d->precKind == PREC_CHOL32) {
         // z = S (L^-T L^-1) S r with the FP32 factor of S M S
         hdk::d2f_scaled(d->st, m, r, d->precS, d->cf1);
-        hdk::coldot<float>(d->st, m, m, 2, 1.0f, d->MLiTf, m, d->cf1, 0.0f, d->cf2);
-        hdk::coldot<float>(d->st, m, m, 1, 1.0f, d->MLif, m, d->cf2, 0.0f, d->cf1);
-        hdk::f2d_scaled(d->st, m, d->cf1, d->precS, z);
+        hdk::solve_apply<float>(d->st, m, d->Mf, m, d->MLif, d->MLiTf, d->cf1, d->cf3, d->cf2);
+        hdk::f2d_scaled(d->st, m, d->cf3, d->precS, z);
     } else {
-        hdk::coldot<double>(d->st, m, m, 2, 1.0, d->MLiT, m, r, 0.0, d->ctmp);
-        hdk::coldot<double>(d->st, m, m, 1, 1.0, d->MLi, m, d->ctmp, 0.0, z);
+        hdk::solve_apply<double>(d->st, m, d->Mchol, m, d->MLi, d->MLiT, r, z, d->ctmp);
     }
     if (p) hdk::cg_jacobi(d->st, m, z, nullptr, p, nullptr);
 }
@@ -1584,11 +1580,9 @@ hdsdp_retcode hdsdp_dev_kkt_solve(hdsdp_dev *d, const double *rhs, double *sol) 
     return download(d, sol, d->cx, d->m, d->hvecB);
 }
 
-// z = (L L^T)^-1 r with the FP64 factor of M (MLi = L^-1, MLiT = L^-T); tmp: m-vector.
+// z = (L L^T)^-1 r with the FP64 factor of M; tmp: m-vector.
 void apply_chol64(hdsdp_dev *d, const double *r, double *z, double *tmp) {
-    const int m = d->m;
-    hdk::coldot<double>(d->st, m, m, 2, 1.0, d->MLiT, m, r, 0.0, tmp);
-    hdk::coldot<double>(d->st, m, m, 1, 1.0, d->MLi, m, tmp, 0.0, z);
+    hdk::solve_apply<double>(d->st, d->m, d->Mchol, d->m, d->MLi, d->MLiT, r, z, tmp);
 }
 
 // Direct FP64 solve of M x = rhs (FP64 Gram blocks, FP64 Cholesky, two refinement steps

@@ -423,3 +423,36 @@ def test_cholesky_flags_a_negative_pivot(gpu_lib, n, flip):
     d.update(1.0, 0.0, np.zeros(2), 8.0, 1)  # the shifted matrix is positive definite
     assert d.factorize(1) == 1
     d.close()
+
+
+# one diagonal block, the first sizes with two, a ragged last block, and the wider span
+@pytest.mark.parametrize("m", [2048, 2049, 2200, 4097, 10241])
+def test_schur_solve_by_blocks(gpu_lib, m):
+    """kkt_solve_exact (FP64 Cholesky of M, block substitution, two refinement steps) across
+    the block edges of the substitution.  M = (S^-1)_ij^2 for single diagonal constraints
+    plus a diagonal of 1: with S = 2 I + a rank-one part, cond(M) < 3, and a refined solve
+    is accurate to a few m u cond (u = 1.1e-16)."""
+    rng = np.random.default_rng(m)
+    n = 160
+    v = rng.standard_normal(n) / np.sqrt(n)
+    S = 2.0 * np.eye(n) + np.outer(v, v)
+    C = dt.Coeff(dt.DENSE, n, val=np.concatenate([S[j:, j] for j in range(n)]))
+    r, c = np.tril_indices(n)
+    pick = np.sort(rng.choice(len(r), size=m, replace=False))
+    one = np.ones(1)
+    d = dt.Dev(gpu_lib, [C] + [dt.Coeff(dt.SPARSE, n, row=[r[k]], col=[c[k]], val=one) for k in pick])
+    d.update(1.0, 0.0, np.zeros(m), 0.0, 0)
+    assert d.factorize(0) == 1
+    d.schur(0, 0.0)
+    d.add_diag(np.ones(m))
+    W = np.linalg.inv(S)
+    ri, ci = r[pick], c[pick]
+    w = np.where(ri == ci, 1.0, 2.0)
+    M = (W[np.ix_(ri, ri)] * W[np.ix_(ci, ci)] + W[np.ix_(ri, ci)] * W[np.ix_(ci, ri)]) * np.outer(w, w) / 2.0
+    M[np.diag_indices(m)] += 1.0
+    b = rng.standard_normal(m)
+    x = np.zeros(m)
+    assert gpu_lib.hdsdp_dev_kkt_solve_exact(d.h, dt._capi.dptr(b), dt._capi.dptr(x)) == 0
+    d.close()
+    res = np.linalg.norm(M @ x - b) / np.linalg.norm(b)
+    assert res <= 12.0 * m * 1.1e-16
