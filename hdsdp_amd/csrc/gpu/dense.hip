@@ -37,13 +37,15 @@ struct Mfma<float> {
 };
 
 // k range of one output tile when an operand is triangular: tri 1 = op(B) lower
-// (B(k, j) = 0 for k < j), tri 2 = op(A) lower (A(i, k) = 0 for k > i).  Only exact
-// zeros are skipped, so the result is the same as the full product.
+// (B(k, j) = 0 for k < j), tri 2 = op(A) lower (A(i, k) = 0 for k > i), tri 3 = op(B) upper
+// (B(k, j) = 0 for k > j).  Only exact zeros are skipped, so the result is the same as
+// the full product.
 __device__ inline void tri_krange(int tri, int i0, int j0, int tile, int K, int &kLo, int &kHi) {
     kLo = 0;
     kHi = K;
     if (tri == 1) kLo = (j0 / KSTEP) * KSTEP;
     if (tri == 2) kHi = (i0 + tile < K) ? i0 + tile : K;
+    if (tri == 3) kHi = (j0 + tile < K) ? j0 + tile : K;
 }
 
 // Output tile of this workgroup.  With lin != 0 (lower products with as many tile rows
@@ -63,7 +65,8 @@ __device__ inline void tile_xy(int lin, int &bx, int &by, int tri = 0) {
         if (tri == 2) bx = (int) ((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
         return;
     }
-    const int t = blockIdx.x;
+    // a triangular operand makes the later tiles the longer ones: those go first
+    const int t = tri ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
     int x = (int) ((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
     while ((x + 1) * (x + 2) / 2 <= t) ++x;
     while (x * (x + 1) / 2 > t) --x;
@@ -296,10 +299,18 @@ __device__ inline void big_store(T (*As)[BT + BPAD], T (*Bs)[BT + BPAD], int tid
     }
 }
 
-template <typename T, bool TA, bool TB, bool LOWER, bool VEC>
+// PACK 1 (square lower products with beta = 0): the strictly lower part of the result's
+// first ldc rows and columns goes to C packed by columns and the diagonal to dg (stride
+// sDg), as pack_lower stores them.  PACK 2: the same entries in k panels, packed entry e of
+// matrix z at C[(e / 16) slab + 16 z + e % 16].
+// PANEL: both operands are read from k panels of 16, entry (k, i) at (k / 16) slab + 16 i +
+// k % 16, so that a slab of a tile is 16 KB of consecutive memory; K a multiple of 16,
+// rows of whole tiles present.
+template <typename T, bool TA, bool TB, bool LOWER, bool VEC, int PACK = 0, bool PANEL = false>
 __global__ __launch_bounds__(256) void gemm_big_kernel(int M, int N, int K, T alpha, const T *A, int lda, long sA,
                                                        const T *B, int ldb, long sB, T beta, T *C, int ldc,
-                                                       long sC, int tri, int lin, int kLast) {
+                                                       long sC, int tri, int lin, int kLast, T *dg = nullptr,
+                                                       long sDg = 0, long slab = 0) {
     typedef typename Mfma<T>::acc_t acc_t;
     if (kLast > 0 && blockIdx.z == gridDim.z - 1) K = kLast;  // ragged last k part of a split product
     int bx, by;
@@ -331,14 +342,28 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(int M, int N, int K, T al
         }
         big_store<T, TA, TB>(As[buf], Bs[buf], tid, ra, rb);
     };
-    bool vec = big_fetch<T, TA, TB, VEC>(A, lda, B, ldb, M, N, K, i0, j0, kLo, tid, ra, rb);
+    auto fetch = [&](int k0) {
+        if constexpr (PANEL) {
+            const long at = (long) (k0 / KSTEP) * slab;
+            big_load_vec<TA, TB>(A + at, KSTEP, B + at, KSTEP, i0, j0, 0, tid, ra, rb);
+            return true;
+        } else {
+            return big_fetch<T, TA, TB, VEC>(A, lda, B, ldb, M, N, K, i0, j0, k0, tid, ra, rb);
+        }
+    };
+    bool vec = fetch(kLo);
     stash(0, vec);
     __syncthreads();
     const int nslab = (kHi - kLo + KSTEP - 1) / KSTEP;
+    // the quadrants that start a half tile earlier have a triangular operand's zeros in the
+    // last half tile of the k range: those waves skip its products
+    const int kWave = __builtin_amdgcn_readfirstlane((tri == 2 && wi == 0) ? i0 + 64 : (tri == 3 && wj == 0) ? j0 + 64
+                                                                                                             : K);
     for (int sl = 0; sl < nslab; ++sl) {
         const int cur = sl & 1;
         const bool more = sl + 1 < nslab;
-        if (more) vec = big_fetch<T, TA, TB, VEC>(A, lda, B, ldb, M, N, K, i0, j0, kLo + (sl + 1) * KSTEP, tid, ra, rb);
+        if (more) vec = fetch(kLo + (sl + 1) * KSTEP);
+        if (kLo + sl * KSTEP < kWave)
 #pragma unroll
         for (int kk = 0; kk < KSTEP; kk += 4) {
             T af[4], bf[4];
@@ -366,6 +391,20 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(int M, int N, int K, T al
         for (int a = 0; a < 4; ++a)
 #pragma unroll
             for (int r = 0; r < 4; ++r) stage[lr][a * 16 + Mfma<T>::row(lk, r)] = acc[a][b][r];
+        if constexpr (PACK != 0) {
+            const long n = ldc;
+#pragma unroll
+            for (int cc = 0; cc < 16; ++cc) {
+                const long j = j0 + wj + b * 16 + cc;
+                if (i >= n || j >= n || i < j) continue;
+                const T v = alpha * stage[cc][lane];
+                const long e = j * n - j * (j + 1) / 2 + (i - j - 1);
+                if (i == j) dg[(long) blockIdx.z * sDg + i] = v;
+                else if (PACK == 1) C[e] = v;
+                else C[(e >> 4) * slab + 16 * blockIdx.z + (e & 15)] = v;
+            }
+            continue;
+        }
         // all loads of the strip are issued before any store (C may alias nothing,
         // but the compiler cannot know that)
         T cin[16];
@@ -455,6 +494,41 @@ template void gemm<double>(hipStream_t, bool, bool, bool, int, int, int, double,
 template void gemm<float>(hipStream_t, bool, bool, bool, int, int, int, float, const float *, int, long,
                           const float *, int, long, float, float *, int, long, int, int);
 
+// P_z = alpha X_z^T X_z (lower, r x r, ld r, stride r^2) over the k slices z of kc (the
+// last one kLast wide) of the k panels X (PANEL above; slab doubles per 16 k)
+void gram_panels(hipStream_t s, int r, int kc, int kLast, int parts, double alpha, const double *X, long slab,
+                 double *P) {
+    const int nt = (r + BT - 1) / BT;
+    gemm_big_kernel<double, true, false, true, true, 0, true><<<dim3(nt * (nt + 1) / 2, 1, parts), 256, 0, s>>>(
+        r, r, kc, alpha, X, 0, kc / KSTEP * slab, X, 0, kc / KSTEP * slab, 0.0, P, r, (long) r * r, 0, 1, kLast,
+        nullptr, 0, slab);
+}
+
+// C_z = A_z B_z^T for z < batch, lower triangle, packed (PACK above); tri as in gemm
+void gemm_nt_packed(hipStream_t s, int rows, int n, const double *A, int lda, long sA, const double *B, int ldb,
+                    long sB, double *off, long K1, long slab, double *dg, long sDg, int batch, int tri) {
+    const int nt = (rows + BT - 1) / BT;
+    const dim3 grid(nt * (nt + 1) / 2, 1, batch);
+    const bool vec = lda % 2 == 0 && ldb % 2 == 0 && sA % 2 == 0 && sB % 2 == 0 && ((uintptr_t) A % 16) == 0 &&
+                     ((uintptr_t) B % 16) == 0;
+    const int K = std::min(rows, (n + KSTEP - 1) / KSTEP * KSTEP);
+    if (slab > 0)
+        gemm_big_kernel<double, false, true, true, true, 2><<<grid, 256, 0, s>>>(
+            rows, rows, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, 0, tri, 1, 0, dg, sDg, slab);
+    else if (vec)
+        gemm_big_kernel<double, false, true, true, true, 1><<<grid, 256, 0, s>>>(
+            rows, rows, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, K1, tri, 1, 0, dg, sDg);
+    else
+        gemm_big_kernel<double, false, true, true, false, 1><<<grid, 256, 0, s>>>(
+            rows, rows, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, K1, tri, 1, 0, dg, sDg);
+}
+
+// whether a lower n x n product of this batch and depth runs on 128-wide tiles
+bool gemm_lower_is_big(int n, int K, int batch) {
+    const long t = (n + BT - 1) / BT;
+    return t * t * batch / 2 >= 192 && K >= 256;
+}
+
 // ---- split-K ---------------------------------------------------------------------
 
 // C(i, j) = alpha sum_p P_p(i, j) + beta C(i, j) over the P partial products (ld M),
@@ -488,7 +562,7 @@ static int cu_count() {
 // kernel holds two workgroups per CU, so P parts of T output tiles take
 // ceil(T P / (2 CUs)) rounds of a k range K / P each, plus the partial-sum traffic
 // (written by the product, read by the reduction) per part.  Ties go to fewer parts.
-int splitk_parts(int M, int N, int K, bool lower) {
+int splitk_parts(int M, int N, long K, bool lower, int most) {
     const long mt = (M + BT - 1) / BT, nt = (N + BT - 1) / BT;
     const long tiles = std::max<long>(1, lower ? (mt == nt ? mt * (mt + 1) / 2 : mt * nt / 2) : mt * nt);
     const long slots = 2L * cu_count();
@@ -496,7 +570,7 @@ int splitk_parts(int M, int N, int K, bool lower) {
     const double secPerPart = (double) M * N * 8.0 * (lower ? 1.0 : 2.0) / 5e12;  // partials out and in
     int best = 1;
     double tBest = 1e300;
-    for (int P = 1; P <= 32 && P <= K / 1024; ++P) {
+    for (int P = 1; P <= most && P <= K / 1024; ++P) {
         const long kc = ((K + P - 1) / P + KSTEP - 1) / KSTEP * KSTEP;
         const int parts = (int) ((K + kc - 1) / kc);
         const long rounds = (tiles * parts + slots - 1) / slots;

@@ -27,8 +27,9 @@ constexpr int NB = 64;     // Cholesky / triangular-inverse block
 
 // C = alpha * op(A) * op(B) + beta * C over `batch` problems (column-major).
 // lower != 0 restricts the output to i >= j (tiles above the diagonal skipped).
-// tri = 1 when op(B) is lower triangular, 2 when op(A) is: the k ranges that
-// multiply the zero triangle are skipped (the stored zeros must be present).
+// tri = 1 when op(B) is lower triangular, 2 when op(A) is, 3 when op(B) is upper
+// triangular: the k ranges that multiply the zero triangle are skipped (the stored zeros
+// must be present).
 template <typename T>
 void gemm(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int K, T alpha,
           const T *A, int lda, long strideA, const T *B, int ldb, long strideB, T beta, T *C,
@@ -39,10 +40,24 @@ void gemm(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int
 // (128-wide tiles fill the chip only with enough of them).  Falls back to gemm when
 // work is null or too small for two parts.
 // number of k parts gemm_splitk uses for this shape (1: no split)
-int splitk_parts(int M, int N, int K, bool lower);
+int splitk_parts(int M, int N, long K, bool lower, int most = 32);
 template <typename T>
 void gemm_splitk(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int K, T alpha, const T *A,
                  int lda, const T *B, int ldb, T beta, T *C, int ldc, T *work, size_t workLen);
+
+// P_z = alpha X_z^T X_z (lower, r x r, ld r, stride r^2) over `parts` k slices of kc (the
+// last one kLast wide; multiples of 16) of the k panels X: entry (k, p) at (k / 16) slab +
+// 16 p + k % 16, p up to whole tiles of 128.
+void gram_panels(hipStream_t s, int r, int kc, int kLast, int parts, double alpha, const double *X, long slab,
+                 double *P);
+// A_z B_z^T (z < batch) on 128-wide tiles, operands of `rows` >= n rows: of the first n rows
+// and columns the strictly lower part, packed by columns, and the diagonal, into dg + z sDg.
+// slab = 0: packed entries into off + z K1; slab > 0: entry e into off[(e / 16) slab + 16 z +
+// e % 16] (operands 16-byte aligned, even ld, whole tiles of rows).  tri as in gemm.
+void gemm_nt_packed(hipStream_t s, int rows, int n, const double *A, int lda, long sA, const double *B, int ldb,
+                    long sB, double *off, long K1, long slab, double *dg, long sDg, int batch, int tri);
+// whether gemm runs a lower n x n product of this depth and batch on 128-wide tiles
+bool gemm_lower_is_big(int n, int K, int batch);
 
 // C = alpha * X^T Y + beta * C from bf16 split products on the matrix cores: each FP32
 // operand split into `terms` bf16 terms (2: three products, ~16 bits; 3: six products,

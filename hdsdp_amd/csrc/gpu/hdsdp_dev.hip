@@ -40,11 +40,14 @@ struct hdsdp_dev {
     int r1Gram, dnGram, nDn, r1Identity;
     double *H1;              // n x (nR1 + 1): W F
     double *Kr;              // nR1 x nR1 when the slot -> row map is not the identity
-    double *Tall, *Tdg;      // packed strictly-lower T_p (K1 = n (n - 1) / 2 each), diagonals (n each)
-    double *Dbuf, *Ubuf;     // gramBatch x n^2
+    double *Tall, *Tdg;      // packed strictly-lower T_p, diagonals (gramLd apart)
+    double *Dbuf, *Ubuf;     // gramBatch matrices of gramRows columns
     double *Gpart;           // gramParts x nDn^2
     int gramBatch, gramParts;
-    long gramChunk;
+    long gramChunk, gramK1;  // k of a Gram part, entries kept of each packed T_p
+    long gramSlab;           // doubles per k panel of the T_p, 0: one T_p after the other
+    int gramLd, gramRows;    // leading dimension and columns of the batch buffers
+    double *LiPad;           // L^-1 with leading dimension gramLd, null where that is n
     // mixed precision Gram builds (bf16 split products): FP32 copies and products
     float *LiTf;             // n x n, L^-T of the dual factor
     float *Ff, *Gf;          // n x nR1: rank-one factors and G = L^-1 F
@@ -613,34 +616,72 @@ int cg_solve(hdsdp_dev *d) {
 // triangle is formed, and <T_p, T_q> = 2 <off_p, off_q> + <dg_p, dg_q> over the packed
 // strictly-lower parts and the diagonals: a split-K Gram product over n (n - 1) / 2
 // with alpha = 2 (exact) and one over n, summed in a fixed order.
+//
+// From n = GRAM_HALF_MIN: T(i, j) sums U(i, k) L^-1(j, k) over k <= j <= i, so of
+// U = L^-1 A_p the lower triangle is formed only: n^3 / 3 + n^3 / 6 multiply-adds per
+// constraint (n = 1000, 1000 constraints: 15 and 10 ms; <T_p, T_q> 9 ms, 64 TF).  Below,
+// the full U and T_p = L^-1 U^T, n^3 / 2 + n^3 / 3 (26 and 18 ms at that size): there the products are a small share of the build, and the
+// Lanczos step bound that the Schur solutions feed, run without reorthogonalisation to a
+// good part of n steps, turns a last-bit change of M into one of up to 4e-3 (n = 121;
+// 2e-9 at n = 300, 1e-12 at n = 700).  Where the products run on 128-wide tiles, T_p is stored
+// packed by the product itself.
+constexpr int GRAM_HALF_MIN = 512;
+
 void dense_gram(hdsdp_dev *d, const double *Li) {
-    const int n = d->n, r = d->nDn, m = d->m;
-    const long nn = (long) n * n, K1 = (long) n * (n - 1) / 2;
+    const int n = d->n, r = d->nDn, m = d->m, ld = d->gramLd, rows = d->gramRows;
+    const long nl = (long) ld * rows, K1 = d->gramK1, slab = d->gramSlab;
+    const bool half = n >= GRAM_HALF_MIN;
+    if (d->LiPad) {
+        (void) hipMemcpy2DAsync(d->LiPad, sizeof(double) * ld, Li, sizeof(double) * n, sizeof(double) * n, n,
+                                hipMemcpyDeviceToDevice, d->st);
+        Li = d->LiPad;
+    }
     for (int b0 = 0; b0 < r; b0 += d->gramBatch) {
         const int cnt = std::min(d->gramBatch, r - b0);
-        hdk::unpack_dense(d->st, d->c, b0, cnt, d->Dbuf);
-        // U = L^-1 A_p, then the lower triangle of T_p = U L^-T = L^-1 U^T: both products
-        // have the lower-triangular L^-1 on the left, whose zero k ranges are skipped
-        hdk::gemm<double>(d->st, false, false, false, n, n, n, 1.0, Li, n, 0, d->Dbuf, n, nn, 0.0, d->Ubuf, n, nn, cnt,
-                          2);
-        hdk::gemm<double>(d->st, false, true, true, n, n, n, 1.0, Li, n, 0, d->Ubuf, n, nn, 0.0, d->Dbuf, n, nn, cnt,
-                          2);
-        hdk::pack_lower<double>(d->st, n, cnt, d->Dbuf, nn, d->Tall + (size_t) b0 * K1, d->Tdg + (size_t) b0 * n);
+        double *off = d->Tall + (size_t) b0 * (slab > 0 ? 16 : K1), *dg = d->Tdg + (size_t) b0 * ld;
+        hdk::unpack_dense(d->st, d->c, b0, cnt, d->Dbuf, ld, nl);
+        const int K = std::min(rows, (n + 15) / 16 * 16);
+        hdk::gemm<double>(d->st, false, false, half, rows, rows, K, 1.0, Li, ld, 0, d->Dbuf, ld, nl, 0.0, d->Ubuf, ld,
+                          nl, cnt, 2);
+        const double *A = half ? d->Ubuf : Li, *B = half ? Li : d->Ubuf;
+        const long sA = half ? nl : 0, sB = half ? 0 : nl;
+        const int tri = half ? 3 : 2;
+        if (slab > 0 || hdk::gemm_lower_is_big(n, n, cnt)) {
+            hdk::gemm_nt_packed(d->st, rows, n, A, ld, sA, B, ld, sB, off, K1, slab, dg, ld, cnt, tri);
+        } else {
+            hdk::gemm<double>(d->st, false, true, true, n, n, n, 1.0, A, ld, sA, B, ld, sB, 0.0, d->Dbuf, ld, nl, cnt,
+                              tri);
+            hdk::pack_lower<double>(d->st, n, cnt, d->Dbuf, ld, nl, off, K1, dg, ld);
+        }
     }
-    const long kc = d->gramChunk;
-    const int full = (int) (K1 / kc);
-    const long rem = K1 - (long) full * kc;
-    const long rr = (long) r * r;
-    const int nOff = full + (rem > 0 ? 1 : 0);
-    if (full > 0)
-        hdk::gemm<double>(d->st, true, false, true, r, r, (int) kc, 2.0, d->Tall, (int) K1, kc, d->Tall, (int) K1, kc,
-                          0.0, d->Gpart, r, rr, full);
-    if (rem > 0)
-        hdk::gemm<double>(d->st, true, false, true, r, r, (int) rem, 2.0, d->Tall + (long) full * kc, (int) K1, 0,
-                          d->Tall + (long) full * kc, (int) K1, 0, 0.0, d->Gpart + (long) full * rr, r, 0, 1);
-    hdk::gemm<double>(d->st, true, false, true, r, r, n, 1.0, d->Tdg, n, 0, d->Tdg, n, 0, 0.0,
-                      d->Gpart + (long) nOff * rr, r, 0, 1);
-    hdk::gram_reduce(d->st, r, nOff + 1, d->Gpart, r, rr, d->c.denseCon, d->M, m);
+    const long kc = d->gramChunk, rr = (long) r * r;
+    const int parts = (int) ((K1 + kc - 1) / kc);
+    const long rem = K1 - (long) (parts - 1) * kc;
+    if (slab > 0) {
+        hdk::gram_panels(d->st, r, (int) kc, (int) rem, parts, 2.0, d->Tall, slab, d->Gpart);
+    } else {
+        const int full = (rem == kc) ? parts : parts - 1;
+        if (full > 0)
+            hdk::gemm<double>(d->st, true, false, true, r, r, (int) kc, 2.0, d->Tall, (int) K1, kc, d->Tall, (int) K1,
+                              kc, 0.0, d->Gpart, r, rr, full);
+        if (full < parts)
+            hdk::gemm<double>(d->st, true, false, true, r, r, (int) rem, 2.0, d->Tall + (long) full * kc, (int) K1, 0,
+                              d->Tall + (long) full * kc, (int) K1, 0, 0.0, d->Gpart + (long) full * rr, r, 0, 1);
+    }
+    hdk::gemm<double>(d->st, true, false, true, r, r, n, 1.0, d->Tdg, ld, 0, d->Tdg, ld, 0, 0.0,
+                      d->Gpart + (long) parts * rr, r, 0, 1);
+    hdk::gram_reduce(d->st, r, parts + 1, d->Gpart, r, rr, d->c.denseCon, d->M, m);
+}
+
+// buffers of the FP64 build; what the products read beyond the entries written is zero
+hdsdp_retcode alloc_dense_gram(hdsdp_dev *d) {
+    const size_t nl = (size_t) d->gramLd * d->gramRows, r = d->nDn;
+    DCALL(dalloc_zero(d, &d->Tall, d->gramSlab > 0 ? (size_t) d->gramK1 / 16 * d->gramSlab : (size_t) d->gramK1 * r));
+    DCALL(dalloc(d, &d->Tdg, (size_t) d->gramLd * r));
+    DCALL(dalloc_zero(d, &d->Dbuf, nl * d->gramBatch));
+    DCALL(dalloc_zero(d, &d->Ubuf, nl * d->gramBatch));
+    if (d->gramLd != d->n) DCALL(dalloc_zero(d, &d->LiPad, nl));
+    return HDSDP_RETCODE_OK;
 }
 
 // Rebuild the Gram blocks of M in FP64 from the factor of their build, re-apply the
@@ -658,13 +699,7 @@ hdsdp_retcode rebuild_gram_fp64(hdsdp_dev *d) {
         else hdk::r1_schur(d->st, d->c, d->H1, d->Kr, d->c.nR1, d->M, m);
     }
     if (d->dnGram) {
-        if (!d->Tall) {
-            const size_t nn = (size_t) n * n, K1 = (size_t) n * (n - 1) / 2;
-            DCALL(dalloc(d, &d->Tall, K1 * d->nDn));
-            DCALL(dalloc(d, &d->Tdg, (size_t) n * d->nDn));
-            DCALL(dalloc(d, &d->Dbuf, nn * d->gramBatch));
-            DCALL(dalloc(d, &d->Ubuf, nn * d->gramBatch));
-        }
+        if (!d->Tall) DCALL(alloc_dense_gram(d));
         dense_gram(d, d->Lim);
     }
     // the rewritten diagonal entries get back what was added to them after the build
@@ -695,7 +730,7 @@ void dense_gram_mixed_inloop(hdsdp_dev *d) {
         // then packed; column i of the left operand L^-T is zero below row i (tri 2)
         hdk::gemm_bf16s_tn<float>(d->st, BF16_TERMS, true, n, n, n, 1.0, d->LiTf, n, 0, d->Vf, n, nn, 0.0, d->Dbuff, n,
                                   nn, cnt, 2);
-        hdk::pack_lower<float>(d->st, n, cnt, d->Dbuff, nn, d->Tf + (size_t) b0 * K1, d->Tdgf + (size_t) b0 * n);
+        hdk::pack_lower<float>(d->st, n, cnt, d->Dbuff, n, nn, d->Tf + (size_t) b0 * K1, K1, d->Tdgf + (size_t) b0 * n, n);
     }
     const long kc = d->gramChunk;
     const int full = (int) (K1 / kc);
@@ -1088,7 +1123,7 @@ hdsdp_retcode hdsdp_dev_load(hdsdp_dev *d, const hdsdp_coeff_view *cv) {
             DCALL(dalloc(d, &d->splitW, d->splitLen));
         }
     }
-    d->H1 = d->Kr = d->Tall = d->Tdg = d->Dbuf = d->Ubuf = d->Gpart = nullptr;
+    d->H1 = d->Kr = d->Tall = d->Tdg = d->Dbuf = d->Ubuf = d->Gpart = d->LiPad = nullptr;
     if (c.nR1 > 0 || c.cDSR1) DCALL(dalloc(d, &d->H1, (size_t) n * (c.nR1 + 1)));
     if (d->r1Gram && !d->r1Identity) DCALL(dalloc(d, &d->Kr, (size_t) c.nR1 * c.nR1));
     d->LiTf = d->Ff = d->Gf = d->Tf = d->Tdgf = d->Dbuff = d->Vf = nullptr;
@@ -1128,18 +1163,39 @@ hdsdp_retcode hdsdp_dev_load(hdsdp_dev *d, const hdsdp_coeff_view *cv) {
         const size_t nn = (size_t) n * n;
         const int r = d->nDn;
         d->gramBatch = (int) std::max<size_t>(1, std::min<size_t>(r, (size_t) (512u << 20) / (nn * sizeof(double))));
-        // split-K parts of the Gram product: enough 128-wide lower tiles for ~8 rounds over
-        // the CUs, and a part count that divides n^2 where one exists, so that every part
-        // goes into one batched launch (a remainder part runs alone, on too few tiles)
+        // FP64 build, from GRAM_HALF_MIN on with enough 128-wide lower tiles: every operand is
+        // padded with zeros to whole tiles, so that no slab takes the bounds-checked loads (at
+        // n = 1000 a third of the products' work lies in ragged tiles), and the T_p are kept
+        // in k panels of 16: rows of 4 MB between the 128 constraints of a tile's slab held the
+        // Gram product at 26 TF.  Its k is split so that the tiles fill whole rounds of
+        // the CUs.  Otherwise the T_p lie one after the other, and k is split in a part count
+        // near `want` that divides it where one exists (below GRAM_HALF_MIN the order of
+        // summation is kept).
         long tiles = (long) ((r + 127) / 128) * ((r + 127) / 128 + 1) / 2;
         long want = std::min<long>(16, std::max<long>(1, (2048 + tiles - 1) / tiles));
-        long K = (long) n * (n - 1) / 2, parts = want;
-        for (long p = want; p <= 2 * want; ++p)
-            if (K % p == 0 && K / p >= 256) {
-                parts = p;
-                break;
-            }
-        d->gramChunk = std::max<long>(1, (K % parts == 0) ? K / parts : std::max<long>(256, (K + parts - 1) / parts));
+        d->gramK1 = std::max<long>(2, (long) n * (n - 1) / 2);
+        long parts = hdk::splitk_parts(r, r, d->gramK1, true, 16);
+        const bool panels = n >= GRAM_HALF_MIN && tiles * parts >= 192;
+        d->gramRows = panels ? (n + 127) / 128 * 128 : n;
+        d->gramLd = panels ? d->gramRows : (n + 1) & ~1;
+        d->gramSlab = panels ? 16L * ((r + 127) / 128 * 128) : 0;
+        if (panels) {
+            d->gramK1 = (d->gramK1 + 15) / 16 * 16;
+            d->gramChunk = ((d->gramK1 + parts - 1) / parts + 15) / 16 * 16;
+            // a batch of 1 GB: each launch ends with a round of partly filled CUs
+            d->gramBatch = (int) std::max<size_t>(
+                1, std::min<size_t>(r, ((size_t) 1 << 30) / ((size_t) d->gramLd * d->gramRows * sizeof(double))));
+        } else {
+            parts = want;
+            for (long p = want; p <= 2 * want; ++p)
+                if (d->gramK1 % p == 0 && d->gramK1 / p >= 256) {
+                    parts = p;
+                    break;
+                }
+            d->gramChunk = (d->gramK1 % parts == 0) ? d->gramK1 / parts
+                                                    : std::max<long>(256, (d->gramK1 + parts - 1) / parts);
+        }
+        const long K = d->gramK1;
         d->gramParts = (int) ((K + d->gramChunk - 1) / d->gramChunk);
         const size_t K1 = std::max<size_t>(1, (size_t) n * (n - 1) / 2);
         if (mixedGram && d->planes) {
@@ -1178,10 +1234,7 @@ hdsdp_retcode hdsdp_dev_load(hdsdp_dev *d, const hdsdp_coeff_view *cv) {
             DCALL(dalloc(d, &d->Dbuff, nn * d->gramBatch));
             DCALL(dalloc(d, &d->Vf, nn * d->gramBatch));
         } else {
-            DCALL(dalloc(d, &d->Tall, K1 * r));
-            DCALL(dalloc(d, &d->Tdg, (size_t) n * r));
-            DCALL(dalloc(d, &d->Dbuf, nn * d->gramBatch));
-            DCALL(dalloc(d, &d->Ubuf, nn * d->gramBatch));
+            DCALL(alloc_dense_gram(d));
         }
         // split-K parts of the off-diagonal Gram and one for the diagonal Gram
         DCALL(dalloc(d, &d->Gpart, (size_t) r * r * (d->gramParts + 1)));

@@ -369,11 +369,11 @@ void r1_schur(hipStream_t s, const DevCoeffs &c, const double *H, double *K, lon
 // diagonal (lane = row of the mirror, coalesced).  Unpacking element by element read
 // the upper half with a stride of a packed column per lane.
 template <typename T>
-__global__ __launch_bounds__(256) void unpack_dense_kernel(int n, const double *dVal, int slot0, T *out) {
+__global__ __launch_bounds__(256) void unpack_dense_kernel(int n, const double *dVal, int slot0, T *out, long ldo, long stride) {
     __shared__ T tile[64][65];  // tile[c][r] = A(i0 + r, j0 + c)
     const long npk = (long) n * (n + 1) / 2;
     const double *v = dVal + (long) (slot0 + blockIdx.y) * npk;
-    T *o = out + (long) blockIdx.y * n * n;
+    T *o = out + (long) blockIdx.y * stride;
     const int t = blockIdx.x;
     int bi = (int) ((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
     while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(256) void unpack_dense_kernel(int n, const double *
         const long i = i0 + tx, j = j0 + c;
         if (i < n && j < n && i >= j) {
             const T val = (T) v[j * n - j * (j + 1) / 2 + i];
-            o[i + j * n] = val;
+            o[i + j * ldo] = val;
             tile[c][tx] = val;
         }
     }
@@ -392,20 +392,20 @@ __global__ __launch_bounds__(256) void unpack_dense_kernel(int n, const double *
     for (int c = ty; c < 64; c += 4) {
         // mirror entry (j0 + tx, i0 + c) = A(i0 + c, j0 + tx) = tile[tx][c], above the diagonal only
         const long r = j0 + tx, q = i0 + c;
-        if (r < n && q < n && q > r) o[r + q * n] = tile[tx][c];
+        if (r < n && q < n && q > r) o[r + q * ldo] = tile[tx][c];
     }
 }
 
 void unpack_dense_f(hipStream_t s, const DevCoeffs &c, int slot0, int cnt, float *out) {
     if (cnt <= 0) return;
     const int nt = (c.n + 63) / 64;
-    unpack_dense_kernel<float><<<dim3(nt * (nt + 1) / 2, cnt), 256, 0, s>>>(c.n, c.dVal, slot0, out);
+    unpack_dense_kernel<float><<<dim3(nt * (nt + 1) / 2, cnt), 256, 0, s>>>(c.n, c.dVal, slot0, out, c.n, (long) c.n * c.n);
 }
 
-void unpack_dense(hipStream_t s, const DevCoeffs &c, int slot0, int cnt, double *out) {
+void unpack_dense(hipStream_t s, const DevCoeffs &c, int slot0, int cnt, double *out, long ldo, long stride) {
     if (cnt <= 0) return;
     const int nt = (c.n + 63) / 64;
-    unpack_dense_kernel<double><<<dim3(nt * (nt + 1) / 2, cnt), 256, 0, s>>>(c.n, c.dVal, slot0, out);
+    unpack_dense_kernel<double><<<dim3(nt * (nt + 1) / 2, cnt), 256, 0, s>>>(c.n, c.dVal, slot0, out, ldo, stride);
 }
 
 // M(i, j) (lower) = sum over the partial Gram blocks, in block order; i, j index dense slots,
@@ -426,26 +426,28 @@ __global__ void gram_reduce_kernel(int r, int nPart, const double *P, long ldp, 
 // by column into off[p * K1 + j n - j (j + 1) / 2 + (i - j - 1)], i > j, and its diagonal
 // into dg[p * n + i].
 template <typename T>
-__global__ void pack_lower_kernel(int n, const T *Tin, long strideIn, T *off, long K1, T *dg) {
+__global__ void pack_lower_kernel(int n, const T *Tin, long ldt, long strideIn, T *off, long K1, T *dg, long ldg) {
     const int p = blockIdx.y;
     const long nn = (long) n * n;
     const T *src = Tin + p * strideIn;
     for (long e = blockIdx.x * (long) blockDim.x + threadIdx.x; e < nn; e += (long) gridDim.x * blockDim.x) {
         const long i = e % n, j = e / n;
-        if (i > j) off[p * K1 + j * n - j * (j + 1) / 2 + (i - j - 1)] = src[e];
-        else if (i == j) dg[(long) p * n + i] = src[e];
+        if (i > j) off[p * K1 + j * n - j * (j + 1) / 2 + (i - j - 1)] = src[i + j * ldt];
+        else if (i == j) dg[p * ldg + i] = src[i + j * ldt];
     }
 }
 
 template <typename T>
-void pack_lower(hipStream_t s, int n, int cnt, const T *Tin, long strideIn, T *off, T *dg) {
+void pack_lower(hipStream_t s, int n, int cnt, const T *Tin, long ldt, long strideIn, T *off, long K1, T *dg,
+                long ldg) {
     if (cnt <= 0) return;
-    const long K1 = (long) n * (n - 1) / 2;
-    pack_lower_kernel<T><<<dim3(1024, cnt), 256, 0, s>>>(n, Tin, strideIn, off, K1, dg);
+    // a block per 1024 entries, at most 1024 blocks, for each matrix
+    const long blocks = std::min<long>(1024, ((long) n * n + 1023) / 1024);
+    pack_lower_kernel<T><<<dim3((unsigned) blocks, cnt), 256, 0, s>>>(n, Tin, ldt, strideIn, off, K1, dg, ldg);
 }
 
-template void pack_lower<double>(hipStream_t, int, int, const double *, long, double *, double *);
-template void pack_lower<float>(hipStream_t, int, int, const float *, long, float *, float *);
+template void pack_lower<double>(hipStream_t, int, int, const double *, long, long, double *, long, double *, long);
+template void pack_lower<float>(hipStream_t, int, int, const float *, long, long, float *, long, float *, long);
 
 __global__ void add_diag_delta_kernel(int r, const int *con, const double *cur, const double *ref, double *M,
                                       long ldm) {

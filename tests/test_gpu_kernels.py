@@ -456,3 +456,33 @@ def test_schur_solve_by_blocks(gpu_lib, m):
     d.close()
     res = np.linalg.norm(M @ x - b) / np.linalg.norm(b)
     assert res <= 12.0 * m * 1.1e-16
+
+
+# FP64 dense Gram: the largest n of the old order, then the lower-triangle products with the
+# T_p one after the other (few tiles) and in k panels, at ragged and whole tiles
+@pytest.mark.parametrize("n,m", [(511, 20), (512, 20), (515, 530), (640, 513), (513, 1)])
+def test_dense_gram_build(gpu_lib, n, m):
+    """M(p, q) = <A_p, W A_q W> and <A_p, W> of dense constraints against numpy.  With
+    condition kappa < 5 of S, products of n terms and Gram sums of n^2 / 2 terms round to
+    (4 n + n^2 / 2) u kappa^2 |M| at worst (u = 1.1e-16); rounding errors add up as their
+    root, and 25 n u |M| leaves a factor of ten over that."""
+    rng = np.random.default_rng(n + m)
+    S, (C, _, _) = _spd_coeffs(n, rng)
+    d = dt.Dev(gpu_lib, [C] + [dt.rand_dense(rng, n) for _ in range(m)])
+    d.update(1.0, 0.0, np.zeros(m), 0.0, 0)
+    assert d.factorize(0) == 1
+    a, _, _ = d.schur(0, 0.0)
+    M = d.get_schur()
+    W = np.linalg.inv(S)
+    W = 0.5 * (W + W.T)
+    L = np.linalg.cholesky(W)
+    A = np.empty((m, n, n))
+    T = np.empty((m, n * n))
+    for k, c in enumerate(d.coeffs[1:]):
+        A[k] = c.dense()
+        T[k] = (L.T @ A[k] @ L).ravel()
+    ref = T @ T.T
+    d.close()
+    u = 1.1e-16
+    assert np.max(np.abs(M - ref)) <= 25.0 * n * u * np.max(np.abs(ref))
+    assert np.max(np.abs(a - np.einsum("kij,ij->k", A, W))) <= 25.0 * n * u * np.sqrt(n) * np.max(np.abs(W))
