@@ -477,62 +477,116 @@ void schur_apply_exact(hdsdp_dev *d, const double *x, double *y) {
 
 int cg_solve(hdsdp_dev *d);
 
+// The Jacobi-preconditioned part of cg_solve_inner: the iterations are queued in batches
+// and decide on the device whether they go on (cgj_iter), the host looks once per batch.
+// Returns the CgStop reached and the iteration it was reached at, CG_RUNNING after maxIter
+// iterations, -1 on a failed call.
+int cg_jacobi_solve(hdsdp_dev *d, int *pIter) {
+    const int m = d->m, restart = std::max(d->nRestart, 20);
+    // iterations queued between two looks: a look costs about two iterations of a small
+    // system, and half a batch runs for nothing at the end
+    const int batch = (m <= 2048) ? 5 : 3;
+    hdk::cgj_start(d->st, m, d->crhs, d->jac, d->relTol, d->absTol, d->cr, d->cx, d->cz, d->cp, d->sc_d);
+    symv_M(d, d->cp, d->cMp);
+    int iter = 0, stop = hdk::CG_RUNNING;
+    while (iter < d->maxIter) {
+        for (int left = std::min(batch, d->maxIter - iter); left > 0 || iter % restart == 6; --left) {
+            // a batch ends with an iteration that reports, never with a restart
+            if (iter >= d->maxIter) break;
+            if (iter % restart == 5) {
+                hdk::cgj_half(d->st, m, d->cz, d->cr, d->cp, d->cMp, d->cx, d->sc_d);
+                symv_M(d, d->cx, d->ctmp);
+                hdk::cg_residual(d->st, m, d->crhs, d->ctmp, d->cr);
+                hdk::cg_jacobi(d->st, m, d->cr, d->jac, d->cp, d->cz);
+            } else {
+                const bool look = left <= 1 || iter + 1 >= d->maxIter ||
+                                  ((iter + 1) % restart == 5 && iter + 2 >= d->maxIter);
+                hdk::cgj_iter(d->st, m, iter, d->jac, d->cMp, d->cx, d->cr, d->cz, d->cp, d->sc_d,
+                              look ? d->hsc : nullptr);
+            }
+            symv_M(d, d->cp, d->cMp);
+            ++iter;
+        }
+        if (sync(d) != HDSDP_RETCODE_OK) return -1;
+        stop = (int) d->hsc[hdk::CG_STOP];
+        if (stop != hdk::CG_RUNNING) {
+            iter = (int) d->hsc[hdk::CG_ITER];
+            break;
+        }
+    }
+    d->stats[2] += (stop == hdk::CG_RUNNING) ? iter : (stop == hdk::CG_TINY) ? 0 : iter + 1;
+    *pIter = iter;
+    return stop;
+}
+
 // conjGradSolve (linalg/hdsdp_linsolver.c:855-997) on crhs with the M on the device;
 // result in cx.  Returns 0 on success, 1 if the solution is left unwritten (tiny rhs),
 // -1 on failure.
 int cg_solve_inner(hdsdp_dev *d) {
     const int m = d->m;
-    const int restart = std::max(d->nRestart, 20);
-    hdk::cg_start(d->st, m, d->crhs, d->cr, d->cx, d->sc_d);
-    if (read_scalars(d) != HDSDP_RETCODE_OK) return -1;
-    double rnorm = d->hsc[hdk::CG_RNORM], bnorm = d->hsc[hdk::CG_BNORM];
-    double tol = std::min(d->absTol, bnorm * d->relTol);
-    tol = std::max(tol, 0.1 * d->absTol);
-    if (rnorm < tol) return 1;
-    apply_precond(d, d->cr, d->cz, d->cp);
-    symv_M(d, d->cp, d->cMp);
     int iter = 0, status = 0, refine = 0;
-    double prevTrue = 0.0, rtrue = -1.0;
-    for (iter = 0; iter < d->maxIter; ++iter) {
-        hdk::cg_step1(d->st, m, d->cz, d->cr, d->cp, d->cMp, d->cx, d->crn, d->sc_d);
-        d->stats[2] += 1;
-        if (iter % restart == 5 && d->useJacobi) {
-            symv_M(d, d->cx, d->ctmp);
-            hdk::cg_residual(d->st, m, d->crhs, d->ctmp, d->cr);
-            apply_precond(d, d->cr, d->cp, nullptr);
-            symv_M(d, d->cp, d->cMp);
-            apply_precond(d, d->cr, d->cz, nullptr);
-            continue;
-        }
-        apply_precond(d, d->crn, d->cz, nullptr);
-        hdk::cg_step2(d->st, m, d->crn, d->cz, d->cp, d->cr, d->sc_d);
-        symv_M(d, d->cp, d->cMp);
+    double rnorm = 0.0, bnorm = 0.0, tol = 0.0, rtrue = -1.0;
+    if (d->useJacobi && d->precKind == PREC_JACOBI) {
+        const int stop = cg_jacobi_solve(d, &iter);
+        if (stop < 0 || stop == hdk::CG_NAN) return -1;
+        if (stop == hdk::CG_TINY) return 1;
+        if (stop == hdk::CG_STALLED) status = 2;
+        rnorm = d->hsc[hdk::CG_RNORM];
+        bnorm = d->hsc[hdk::CG_BNORM];
+        tol = d->hsc[hdk::CG_TOL];
+    } else {
+        const int restart = std::max(d->nRestart, 20);
+        hdk::cg_start(d->st, m, d->crhs, d->cr, d->cx, d->sc_d);
         if (read_scalars(d) != HDSDP_RETCODE_OK) return -1;
         rnorm = d->hsc[hdk::CG_RNORM];
-        if (rnorm != rnorm) return -1;
-        if (iter > 20 && rnorm > 0.01 * bnorm) {
-            status = 2;
-            break;
-        }
-        if (rnorm < tol) {
-            // With the FP32 preconditioner the recursively updated residual drifts
-            // from b - M x: confirm convergence on the true FP64 residual and, if it
-            // is not met, restart from x (iterative refinement).  Refinement stops at
-            // tol or once the true residual stops halving (the rounding level of an
-            // FP64 product with M).  The FP64 factor needs no such check (as in the FP64 path).
-            if (d->precision != HDSDP_PRECISION_MIXED || d->useJacobi || d->precKind != PREC_CHOL32) break;
-            if (refine >= 8) break;
-            symv_M(d, d->cx, d->ctmp);
-            hdk::cg_true_residual(d->st, m, d->crhs, d->ctmp, d->cr, d->sc_d);
-            if (read_scalars(d) != HDSDP_RETCODE_OK) return -1;
-            rtrue = d->hsc[hdk::CG_TRUE];
-            if (rtrue != rtrue) return -1;
-            if (rtrue < tol) break;
-            if (refine > 0 && rtrue > 0.5 * prevTrue) break;
-            prevTrue = rtrue;
-            ++refine;
-            apply_precond(d, d->cr, d->cz, d->cp);
+        bnorm = d->hsc[hdk::CG_BNORM];
+        tol = std::min(d->absTol, bnorm * d->relTol);
+        tol = std::max(tol, 0.1 * d->absTol);
+        if (rnorm < tol) return 1;
+        apply_precond(d, d->cr, d->cz, d->cp);
+        symv_M(d, d->cp, d->cMp);
+        double prevTrue = 0.0;
+        for (iter = 0; iter < d->maxIter; ++iter) {
+            hdk::cg_step1(d->st, m, d->cz, d->cr, d->cp, d->cMp, d->cx, d->crn, d->sc_d);
+            d->stats[2] += 1;
+            if (iter % restart == 5 && d->useJacobi) {
+                symv_M(d, d->cx, d->ctmp);
+                hdk::cg_residual(d->st, m, d->crhs, d->ctmp, d->cr);
+                apply_precond(d, d->cr, d->cp, nullptr);
+                symv_M(d, d->cp, d->cMp);
+                apply_precond(d, d->cr, d->cz, nullptr);
+                continue;
+            }
+            apply_precond(d, d->crn, d->cz, nullptr);
+            hdk::cg_step2(d->st, m, d->crn, d->cz, d->cp, d->cr, d->sc_d);
             symv_M(d, d->cp, d->cMp);
+            if (read_scalars(d) != HDSDP_RETCODE_OK) return -1;
+            rnorm = d->hsc[hdk::CG_RNORM];
+            if (rnorm != rnorm) return -1;
+            if (iter > 20 && rnorm > 0.01 * bnorm) {
+                status = 2;
+                break;
+            }
+            if (rnorm < tol) {
+                // With the FP32 preconditioner the recursively updated residual drifts
+                // from b - M x: confirm convergence on the true FP64 residual and, if it
+                // is not met, restart from x (iterative refinement).  Refinement stops at
+                // tol or once the true residual stops halving (the rounding level of an
+                // FP64 product with M).  The FP64 factor needs no such check (as in the FP64 path).
+                if (d->precision != HDSDP_PRECISION_MIXED || d->useJacobi || d->precKind != PREC_CHOL32) break;
+                if (refine >= 8) break;
+                symv_M(d, d->cx, d->ctmp);
+                hdk::cg_true_residual(d->st, m, d->crhs, d->ctmp, d->cr, d->sc_d);
+                if (read_scalars(d) != HDSDP_RETCODE_OK) return -1;
+                rtrue = d->hsc[hdk::CG_TRUE];
+                if (rtrue != rtrue) return -1;
+                if (rtrue < tol) break;
+                if (refine > 0 && rtrue > 0.5 * prevTrue) break;
+                prevTrue = rtrue;
+                ++refine;
+                apply_precond(d, d->cr, d->cz, d->cp);
+                symv_M(d, d->cp, d->cMp);
+            }
         }
     }
     d->stats[5] = iter;

@@ -132,6 +132,101 @@ void cg_residual(hipStream_t s, int m, const double *rhs, const double *Mx, doub
     cg_residual_kernel<<<(m + 1023) / 1024, 1024, 0, s>>>(m, rhs, Mx, r);
 }
 
+// The Jacobi iteration on small systems is bound by launches and host round trips: four
+// launches, a copy and a synchronisation per iteration took 45 us at m = 368, of which
+// the arithmetic is under 5.  One launch per iteration beside the product with M, and
+// a host look every few iterations, take 12.  Same statements and reduction orders
+// as the separate kernels.
+__global__ __launch_bounds__(1024) void cgj_start_kernel(int m, const double *rhs, const double *jac, double relTol,
+                                                         double absTol, double *r, double *x, double *z, double *p,
+                                                         double *sc) {
+    __shared__ double red[17];
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < m; i += blockDim.x) {
+        const double v = rhs[i], t = v / jac[i];
+        r[i] = v;
+        x[i] = 0.0;
+        z[i] = t;
+        p[i] = t;
+        acc += v * v;
+    }
+    const double nrm = sqrt(block_sum(acc, red));
+    if (threadIdx.x == 0) {
+        const double tol = fmax(fmin(absTol, nrm * relTol), 0.1 * absTol);
+        sc[CG_RNORM] = nrm;
+        sc[CG_BNORM] = nrm;
+        sc[CG_TOL] = tol;
+        sc[CG_STOP] = (nrm < tol) ? CG_TINY : CG_RUNNING;
+        sc[CG_ITER] = 0.0;
+    }
+}
+
+template <bool HALF>
+__global__ __launch_bounds__(1024) void cgj_iter_kernel(int m, int iter, const double *jac, const double *Mp, double *x,
+                                                        double *r, double *z, double *p, double *sc, double *report) {
+    __shared__ double red[17];
+    if (sc[CG_STOP] == CG_RUNNING) {  // the same for every thread: only thread 0 writes it, below
+        double a = 0.0, b = 0.0;
+        for (int i = threadIdx.x; i < m; i += blockDim.x) {
+            a += z[i] * r[i];
+            b += p[i] * Mp[i];
+        }
+        const double rz = block_sum(a, red);
+        const double pMp = block_sum(b, red);
+        const double alpha = rz / pMp;
+        if (HALF) {
+            for (int i = threadIdx.x; i < m; i += blockDim.x) x[i] += alpha * p[i];
+            return;
+        }
+        a = 0.0;
+        for (int i = threadIdx.x; i < m; i += blockDim.x) {
+            x[i] += alpha * p[i];
+            const double v = r[i] - alpha * Mp[i], t = v / jac[i];
+            r[i] = v;
+            z[i] = t;
+            a += v * t;
+        }
+        const double beta = block_sum(a, red) / rz;
+        double c = 0.0;
+        for (int i = threadIdx.x; i < m; i += blockDim.x) {
+            p[i] = z[i] + beta * p[i];
+            c += r[i] * r[i];
+        }
+        const double nrm = sqrt(block_sum(c, red));
+        if (threadIdx.x == 0) {
+            const double stop = (nrm != nrm)                                   ? CG_NAN
+                                : (iter > 20 && nrm > 0.01 * sc[CG_BNORM]) ? CG_STALLED
+                                : (nrm < sc[CG_TOL])                           ? CG_CONVERGED
+                                                                               : CG_RUNNING;
+            sc[CG_RNORM] = nrm;
+            sc[CG_ITER] = iter;
+            sc[CG_STOP] = stop;
+        }
+        __threadfence_block();
+    }
+    if (report && threadIdx.x == 0) {
+        report[CG_RNORM] = sc[CG_RNORM];
+        report[CG_BNORM] = sc[CG_BNORM];
+        report[CG_TOL] = sc[CG_TOL];
+        report[CG_ITER] = sc[CG_ITER];
+        report[CG_STOP] = sc[CG_STOP];
+    }
+}
+
+void cgj_start(hipStream_t s, int m, const double *rhs, const double *jac, double relTol, double absTol, double *r,
+               double *x, double *z, double *p, double *sc) {
+    cgj_start_kernel<<<1, 1024, 0, s>>>(m, rhs, jac, relTol, absTol, r, x, z, p, sc);
+}
+void cgj_iter(hipStream_t s, int m, int iter, const double *jac, const double *Mp, double *x, double *r, double *z,
+              double *p, double *sc, double *report) {
+    cgj_iter_kernel<false><<<1, 1024, 0, s>>>(m, iter, jac, Mp, x, r, z, p, sc, report);
+}
+void cgj_half(hipStream_t s, int m, const double *z, const double *r, const double *p, const double *Mp, double *x,
+              double *sc) {
+    cgj_iter_kernel<true><<<1, 1024, 0, s>>>(m, 0, nullptr, Mp, x, const_cast<double *>(r), const_cast<double *>(z),
+                                             const_cast<double *>(p), sc, nullptr);
+}
+
 // ---- Lanczos (linalg/hdsdp_lanczos.c:196-286) ---------------------------------
 
 // One Lanczos orthogonalisation step on w = Op(v_k):
