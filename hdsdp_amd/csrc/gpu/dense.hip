@@ -702,7 +702,7 @@ __global__ __launch_bounds__(256) void coldot_kernel(int m, int ncols, int tri, 
         for (int k = i; k < hic[c]; k += 64) sum[c] += col[c][k] * x[k];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        for (int off = 32; off > 0; off >>= 1) sum[c] += __shfl_down(sum[c], off);
+        sum[c] = wave_tree_sum(sum[c]);
         if (lane == 0 && j0 + c < ncols) y[j0 + c] = alpha * sum[c] + ((beta != (T) 0) ? beta * y[j0 + c] : (T) 0);
     }
 }

@@ -77,22 +77,22 @@ struct hdsdp_dev {
     double *coef_d, *vecA_d, *vecB_d, *sc_d;
     int *info_d;
     // pinned staging
-    double *hcoef, *hvecA, *hvecB, *hsc, *hvec_n, *hY, *hHist;
+    double *hcoef, *hvecA, *hvecB, *hsc, *hHist;
     int *hinfo;
     bool stagingBusy;
+    bool rhsStaged, solStaged;  // hvecB holds the right-hand side / the solution of a small CG solve
 
     // Lanczos (linalg/hdsdp_lanczos.c): the dual cone's solver (lzComputed, lwarm) and the
     // primal method's own (lzComputedP, lwarmP; interface/hdsdp_psdp.c:113-116)
     int lzMax, lzComputed, lzComputedP;
-    double *V, *Hd, *lv, *lw, *lz1, *lz2, *lwarm, *lwarmP, *ly, *mv1, *mv2;
+    double *V, *Hd, *lv, *lw, *lz1, *lz2, *lwarm, *lwarmP, *mv1, *mv2;
     // primal method (interface/hdsdp_psdp.c): the primal iterate is X; Xs its value at the
     // start (the fixed scaling), dXp the direction, XSX the buffer X S X (+ Xs dS Xs), Sold
     // the dual matrix of the iteration, LX / LXi / LXiT the Cholesky factor of X and inverses
     double *Xs, *dXp, *XSX, *Sold, *LX, *LXi, *LXiT, *LXd;
-    double *lzHist;  // (alpha_k, ||w_k||) of every Lanczos step, read at the check steps
+    double *lzStart, *lzPert;  // Lanczos start vector and warm-start perturbation (fixed by n)
     double *symvW;   // tile partials of the lower-triangle product with M (large m), else null
-    std::vector<double> Hh;
-    std::vector<double> lzStart, lzPert;  // Lanczos start vector and warm-start perturbation (fixed by n)
+    std::vector<double> Hh;  // hHist: (alpha_k, ||w_k||) of every step, written by the device
 
     // Schur system; mVer counts changes of M, cholVer is the mVer its FP64 factor
     // (Mchol and the inverses of its diagonal blocks, MLi, MLiT) was computed from (-1: none)
@@ -246,67 +246,64 @@ void lz_mvec(hdsdp_dev *d, const LzOp &op, const double *in, double *out) {
 // glibc rand start vector and warm-start perturbation (linalg/hdsdp_lanczos.c:33-53).
 // Both restart the generator from srand(n) and reseed it per entry, so they are fixed
 // by n: they are generated once per device (n reseeds of glibc's generator cost ~1.5 us
-// each, ~3 ms per Lanczos call at n = 2000) and reused.  The perturbation entries are
+// each, ~3 ms per Lanczos call at n = 2000) and kept there.  The perturbation entries are
 // 1e-3 sqrt(sqrt(r)) times +-0.5 (an exact product), so adding the stored entry gives
 // the same sum as adding the expression.
-void lz_prepare(hdsdp_dev *d, int n, double *vVec) {
-    if ((int) d->lzStart.size() != n) {
-        d->lzStart.resize(n);
+hdsdp_retcode lz_vectors(hdsdp_dev *d) {
+    if (d->lzStart) return HDSDP_RETCODE_OK;
+    const int n = d->n;
+    double *st = nullptr, *pt = nullptr;
+    DCALL(dalloc(d, &st, n));
+    DCALL(dalloc(d, &pt, n));
+    std::vector<double> v(n);
+    for (int which = 0; which < 2; ++which) {
         srand(n);
         for (int i = 0; i < n; ++i) {
             srand(rand());
-            d->lzStart[i] = sqrt(sqrt((rand() % 1627))) * (rand() % 2 - 0.5);
+            const double r = sqrt(sqrt((rand() % 1627))), h = rand() % 2 - 0.5;
+            v[i] = which ? 1e-03 * r * h : r * h;
         }
+        HIP_OK(hipMemcpy(which ? pt : st, v.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     }
-    memcpy(vVec, d->lzStart.data(), sizeof(double) * n);
-}
-
-void lz_perturb(hdsdp_dev *d, int n, double *vVec) {
-    if ((int) d->lzPert.size() != n) {
-        d->lzPert.resize(n);
-        srand(n);
-        for (int i = 0; i < n; ++i) {
-            srand(rand());
-            d->lzPert[i] = 1e-03 * sqrt(sqrt((rand() % 1627))) * (rand() % 2 - 0.5);
-        }
-    }
-    for (int i = 0; i < n; ++i) vVec[i] += d->lzPert[i];
+    d->lzPert = pt;
+    d->lzStart = st;
+    return HDSDP_RETCODE_OK;
 }
 
 // HLanczosSolve (linalg/hdsdp_lanczos.c:161-292) with device mat-vecs.  The host
 // needs a step's (alpha, ||w||) only for the tridiagonal at the check steps (every
-// `check` steps and at a breakdown), so the steps run back to back and their scalars
-// are read once per check window and processed step by step in the reference's order.
-// A breakdown or a converged check inside a window has let the device run the rest
-// of the window's steps; those only write Krylov columns beyond the ones the
+// `check` steps and at a breakdown), so the steps run back to back, write their scalars to
+// host memory, and are looked at once per window and processed step by step in the
+// reference's order.  A breakdown or a converged check inside a window has let the device
+// run the rest of the window's steps; those only write Krylov columns beyond the ones the
 // estimate combines, so the result is that of the step-by-step loop.
 hdsdp_retcode lanczos(hdsdp_dev *d, const LzOp &op, double *maxStep) {
     const int n = d->n, maxDim = d->lzMax, nH = maxDim + 1;
+    const bool small = n <= hdk::LZS_MAX;
     std::vector<double> &H = d->Hh;
     std::fill(H.begin(), H.end(), 0.0);
-    if (*op.computed == 0) {
-        lz_prepare(d, n, d->hvec_n);
-    } else {
-        HIP_OK(hipMemcpyAsync(d->hvec_n, op.warm, n * sizeof(double), hipMemcpyDeviceToHost, d->st));
-        DCALL(sync(d));
-        lz_perturb(d, n, d->hvec_n);
-    }
-    hdk::fill(d->st, d->V, (long) n * nH, 0.0);
-    hdk::fill(d->st, d->Hd, (long) nH * nH, 0.0);
-    HIP_OK(hipMemcpyAsync(d->lw, d->hvec_n, n * sizeof(double), hipMemcpyHostToDevice, d->st));
-    hdk::lz_start(d->st, n, d->lw, d->lv, d->V);
+    DCALL(lz_vectors(d));
+    const double *x0 = (*op.computed == 0) ? d->lzStart : op.warm;
+    const double *pert = (*op.computed == 0) ? nullptr : d->lzPert;
+    if (!small) hdk::lz_start(d->st, n, x0, pert, d->lv, d->V);
     const int check = std::min(maxDim / 5, 3);
+    // steps per window: in one launch (small) two checks' steps cost less than a second look
+    const int window = small ? 2 * check : check;
     double Td[32], Te[32], evals[2], Y[2 * 32];
-    int kRead = 0;  // first step whose scalars the host has not processed
     bool done = false;
-    for (int k = 0; k < maxDim && !done; ++k) {
-        lz_mvec(d, op, d->lv, d->lw);
-        hdk::lz_step(d->st, n, k, d->lw, d->V, d->Hd, nH, d->lv, d->sc_d, d->lzHist);
-        if ((k + 1) % check != 0 && k < maxDim - 1) continue;
-        HIP_OK(hipMemcpyAsync(d->hHist + 2 * kRead, d->lzHist + 2 * kRead, sizeof(double) * 2 * (k + 1 - kRead),
-                              hipMemcpyDeviceToHost, d->st));
+    for (int k0 = 0, k1 = 0; k0 < maxDim && !done; k0 = k1) {
+        k1 = std::min(k0 + window, maxDim);
+        if (small) {
+            hdk::lz_small_steps(d->st, n, k0, k1, x0, pert, op.Li, op.LiT, op.D, d->V, d->Hd, nH, d->hHist);
+            d->stats[3] += k1 - k0;
+        } else {
+            for (int k = k0; k < k1; ++k) {
+                lz_mvec(d, op, d->lv, d->lw);
+                hdk::lz_step(d->st, n, k, d->lw, d->V, d->Hd, nH, d->lv, d->hHist);
+            }
+        }
         DCALL(sync(d));
-        for (int j = kRead; j <= k && !done; ++j) {
+        for (int j = k0; j < k1 && !done; ++j) {
             const double alpha = d->hHist[2 * j], normPres = d->hHist[2 * j + 1];
             H[j + j * nH] = alpha;
             if (normPres > 0.0) H[(j + 1) + j * nH] = H[j + (j + 1) * nH] = normPres;
@@ -320,16 +317,23 @@ hdsdp_retcode lanczos(hdsdp_dev *d, const LzOp &op, double *maxStep) {
             double resi = fabs(H[kp1 + j * nH] * Y[kp1 + j]);
             if (resi < 1e-04 || j >= maxDim - 1) {
                 double e1 = evals[1], e2 = evals[0];
-                memcpy(d->hY, Y, sizeof(double) * 2 * kp1);
-                HIP_OK(hipMemcpyAsync(d->ly, d->hY, sizeof(double) * 2 * kp1, hipMemcpyHostToDevice, d->st));
-                hdk::lz_comb(d->st, n, kp1, d->V, d->ly + kp1, d->lz1);
-                lz_mvec(d, op, d->lz1, d->lz2);
-                HIP_OK(hipMemcpyAsync(op.warm, d->lz2, n * sizeof(double), hipMemcpyDeviceToDevice, d->st));
-                hdk::axpy_norm(d->st, n, -e1, d->lz1, d->lz2, d->sc_d, hdk::LZ_R1);
-                hdk::lz_comb(d->st, n, kp1, d->V, d->ly, d->lz2);
-                lz_mvec(d, op, d->lz2, d->lz1);
-                hdk::axpy_norm(d->st, n, -e1, d->lz2, d->lz1, d->sc_d, hdk::LZ_R2);
-                DCALL(read_scalars(d));
+                hdk::LzCoef y1{}, y2{};
+                memcpy(y1.y, Y + kp1, sizeof(double) * kp1);
+                memcpy(y2.y, Y, sizeof(double) * kp1);
+                if (small) {
+                    hdk::lz_small_bound(d->st, n, kp1, e1, y1, y2, op.Li, op.LiT, op.D, d->V, op.warm, d->hsc);
+                    d->stats[3] += 2;
+                    DCALL(sync(d));
+                } else {
+                    hdk::lz_comb(d->st, n, kp1, d->V, y1, d->lz1);
+                    lz_mvec(d, op, d->lz1, d->lz2);
+                    HIP_OK(hipMemcpyAsync(op.warm, d->lz2, n * sizeof(double), hipMemcpyDeviceToDevice, d->st));
+                    hdk::axpy_norm(d->st, n, -e1, d->lz1, d->lz2, d->sc_d, hdk::LZ_R1);
+                    hdk::lz_comb(d->st, n, kp1, d->V, y2, d->lz2);
+                    lz_mvec(d, op, d->lz2, d->lz1);
+                    hdk::axpy_norm(d->st, n, -e1, d->lz2, d->lz1, d->sc_d, hdk::LZ_R2);
+                    DCALL(read_scalars(d));
+                }
                 double r1 = d->hsc[hdk::LZ_R1], r2 = d->hsc[hdk::LZ_R2];
                 double diff = e1 - e2 - r2;
                 double gamma = (diff > 0) ? diff : 1e-16;
@@ -344,7 +348,6 @@ hdsdp_retcode lanczos(hdsdp_dev *d, const LzOp &op, double *maxStep) {
                 }
             }
         }
-        kRead = k + 1;
     }
     *op.computed += 1;
     return check_launch();
@@ -483,6 +486,19 @@ int cg_solve(hdsdp_dev *d);
 // iterations, -1 on a failed call.
 int cg_jacobi_solve(hdsdp_dev *d, int *pIter) {
     const int m = d->m, restart = std::max(d->nRestart, 20);
+    if (m <= hdk::CGS_MAX) {
+        // the right-hand side and the solution pass through the staging buffer where
+        // hdsdp_dev_kkt_solve left it there
+        hdk::cg_small(d->st, m, d->M, m, d->rhsStaged ? d->hvecB : d->crhs, d->jac, d->relTol, d->absTol, d->maxIter,
+                      restart, d->crhs, d->cx, d->rhsStaged ? d->hvecB : nullptr, d->hsc);
+        if (sync(d) != HDSDP_RETCODE_OK) return -1;
+        const int stop = (int) d->hsc[hdk::CG_STOP];
+        *pIter = (int) d->hsc[hdk::CG_ITER];
+        d->stats[2] += (stop == hdk::CG_RUNNING) ? *pIter : (stop == hdk::CG_TINY) ? 0 : *pIter + 1;
+        d->solStaged = d->rhsStaged && stop == hdk::CG_CONVERGED;
+        d->rhsStaged = false;
+        return stop;
+    }
     // iterations queued between two looks: a look costs about two iterations of a small
     // system, and half a batch runs for nothing at the end
     const int batch = (m <= 2048) ? 5 : 3;
@@ -910,16 +926,14 @@ hdsdp_retcode hdsdp_dev_create(hdsdp_dev **pdev, int nRow, int nCol, int precisi
     DCALL(halloc(&d->hvecA, m + 1));
     DCALL(halloc(&d->hvecB, m + 1));
     DCALL(halloc(&d->hsc, hdk::SC_SLOTS));
-    DCALL(halloc(&d->hvec_n, n));
-    DCALL(halloc(&d->hY, 64));
     DCALL(halloc(&d->hinfo, 1));
-    d->lzMax = 30;
+    d->lzMax = hdk::LZ_MAX;
     d->lzComputed = d->lzComputedP = 0;
     d->psdpReady = 0;
     d->lwarmP = d->Xs = d->dXp = d->XSX = d->Sold = d->LX = d->LXi = d->LXiT = nullptr;
     d->Hh.assign((size_t) (d->lzMax + 1) * (d->lzMax + 1), 0.0);
     DCALL(halloc(&d->hHist, 2 * (d->lzMax + 1)));
-    DCALL(dalloc(d, &d->lzHist, 2 * (d->lzMax + 1)));
+    d->lzStart = d->lzPert = nullptr;
     DCALL(dalloc(d, &d->V, n * (d->lzMax + 1)));
     DCALL(dalloc(d, &d->Hd, (size_t) (d->lzMax + 1) * (d->lzMax + 1)));
     DCALL(dalloc(d, &d->lv, n));
@@ -927,7 +941,6 @@ hdsdp_retcode hdsdp_dev_create(hdsdp_dev **pdev, int nRow, int nCol, int precisi
     DCALL(dalloc(d, &d->lz1, n));
     DCALL(dalloc(d, &d->lz2, n));
     DCALL(dalloc(d, &d->lwarm, n));
-    DCALL(dalloc(d, &d->ly, 64));
     DCALL(dalloc(d, &d->mv1, n));
     DCALL(dalloc(d, &d->mv2, n));
     DCALL(dalloc(d, &d->M, m * m));
@@ -1349,7 +1362,7 @@ void hdsdp_dev_destroy(hdsdp_dev **pdev) {
     hdsdp_dev *d = *pdev;
     if (d->st) hipStreamSynchronize(d->st);
     for (void *p : d->allocs) hipFree(p);
-    double *hp[] = {d->hcoef, d->hvecA, d->hvecB, d->hsc, d->hvec_n, d->hY, d->hHist};
+    double *hp[] = {d->hcoef, d->hvecA, d->hvecB, d->hsc, d->hHist};
     for (double *p : hp)
         if (p) hipHostFree(p);
     if (d->hinfo) hipHostFree(d->hinfo);
@@ -1660,7 +1673,15 @@ int hdsdp_dev_kkt_uses_ldl(hdsdp_dev *d) {
 // HFpLinsysSolve (linalg/hdsdp_linsolver.c:1410-1425): a CG solve that fails switches the
 // system to the direct indefinite solver, which then solves this right-hand side
 hdsdp_retcode hdsdp_dev_kkt_solve(hdsdp_dev *d, const double *rhs, double *sol) {
-    DCALL(upload(d, d->crhs, rhs, d->m, d->hvecB));
+    d->solStaged = false;
+    d->rhsStaged = !d->useLU && d->m <= hdk::CGS_MAX && d->paramUseJacobi && d->precKind == PREC_JACOBI;
+    if (d->rhsStaged) {
+        // the kernel reads the staging buffer itself (and writes crhs and the solution)
+        if (d->stagingBusy) DCALL(sync(d));
+        memcpy(d->hvecB, rhs, sizeof(double) * d->m);
+    } else {
+        DCALL(upload(d, d->crhs, rhs, d->m, d->hvecB));
+    }
     prof_begin(d, HDSDP_PROF_CG);
     int rc = 0;
     if (d->useLU) {
@@ -1684,6 +1705,10 @@ hdsdp_retcode hdsdp_dev_kkt_solve(hdsdp_dev *d, const double *rhs, double *sol) 
     DCALL(prof_end(d, HDSDP_PROF_CG));
     if (rc < 0) return HDSDP_RETCODE_FAILED;
     if (rc == 1) return HDSDP_RETCODE_OK;  // tiny right-hand side: solution left as it was
+    if (d->solStaged) {
+        memcpy(sol, d->hvecB, sizeof(double) * d->m);
+        return HDSDP_RETCODE_OK;
+    }
     return download(d, sol, d->cx, d->m, d->hvecB);
 }
 

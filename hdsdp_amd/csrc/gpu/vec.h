@@ -11,8 +11,6 @@ enum {
     CG_BNORM = 1,
     CG_RZ = 2,
     CG_ALPHA = 3,
-    LZ_ALPHA = 4,
-    LZ_NORM = 5,
     LZ_R1 = 6,
     LZ_R2 = 7,
     SC_LOGDET = 8,
@@ -45,14 +43,38 @@ void cgj_iter(hipStream_t s, int m, int iter, const double *jac, const double *M
               double *p, double *sc, double *report);
 void cgj_half(hipStream_t s, int m, const double *z, const double *r, const double *p, const double *Mp, double *x,
               double *sc);
+// The whole Jacobi CG of a system of m <= CGS_MAX rows in one launch: M m x m (ldm, both
+// triangles), rhs in device or device-readable host memory (copied to crhs), at most
+// maxIter iterations with a restart from the true residual at iter % restart == 5.  The
+// scalars of cgj_iter go to report (CG_ITER: maxIter when it ran out), the solution to x
+// and xHost (both written on every exit but CG_TINY).
+constexpr int CGS_MAX = 256;
+void cg_small(hipStream_t s, int m, const double *M, long ldm, const double *rhs, const double *jac, double relTol,
+              double absTol, int maxIter, int restart, double *crhs, double *x, double *xHost, double *report);
 void cg_residual(hipStream_t s, int m, const double *rhs, const double *Mx, double *r);
 // r = rhs - Mx and sc[CG_TRUE] = ||r||
 void cg_true_residual(hipStream_t s, int m, const double *rhs, const double *Mx, double *r, double *sc);
 
-void lz_step(hipStream_t s, int n, int k, double *w, double *V, double *H, int ldh, double *v, double *sc,
-             double *hist);
-void lz_start(hipStream_t s, int n, const double *x, double *v, double *V);
-void lz_comb(hipStream_t s, int n, int kp1, const double *V, const double *y, double *z);
+// combination coefficients of a Krylov basis, passed by value
+constexpr int LZ_MAX = 30;
+struct LzCoef {
+    double y[LZ_MAX + 1];
+};
+// Step k of Lanczos on w: V_{k + 1}, v and the norm in H (zeros when the norm is 0), and
+// (alpha_k, norm_k) in hist (host memory the device can write).
+void lz_step(hipStream_t s, int n, int k, double *w, double *V, double *H, int ldh, double *v, double *hist);
+// v = V_0 = x / ||x|| with x = x0, or x0 + pert where pert is not null
+void lz_start(hipStream_t s, int n, const double *x0, const double *pert, double *v, double *V);
+void lz_comb(hipStream_t s, int n, int kp1, const double *V, const LzCoef &y, double *z);
+// n <= LZS_MAX: one workgroup runs the start (k0 = 0), the products L^-1 (-D) L^-T v and the
+// steps k0 .. k1 - 1 in one launch, ...
+constexpr int LZS_MAX = 160;
+void lz_small_steps(hipStream_t s, int n, int k0, int k1, const double *x0, const double *pert, const double *Li,
+                    const double *LiT, const double *D, double *V, double *H, int ldh, double *hist);
+// ... and the two residuals of the step bound in another: with z = V y1, warm = Op z,
+// report[LZ_R1] = ||Op z - e1 z|| and the same of V y2 in report[LZ_R2].
+void lz_small_bound(hipStream_t s, int n, int kp1, double e1, const LzCoef &y1, const LzCoef &y2, const double *Li,
+                    const double *LiT, const double *D, const double *V, double *warm, double *report);
 void axpy_norm(hipStream_t s, int n, double a, const double *x, double *y, double *sc, int slot);
 
 void axpy(hipStream_t s, long n, double a, const double *x, double *y);

@@ -9,19 +9,19 @@
 
 namespace hdk {
 
+// Sum over a workgroup of 1024 threads, in every thread: each wave's tree sum, then the
+// sixteen of them in order (every thread adds them up itself: one barrier per sum).  Two
+// sums in a row use different halves B of red (32 doubles).
+template <int B>
 __device__ inline double block_sum(double v, double *red) {
-    const int tid = threadIdx.x;
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    if ((tid & 63) == 0) red[tid >> 6] = v;
+    v = wave_tree_sum(v);
+    if ((threadIdx.x & 63) == 0) red[16 * B + (threadIdx.x >> 6)] = v;
     __syncthreads();
-    double total = 0.0;
-    if (tid == 0) {
-        for (int w = 0; w < (int) (blockDim.x >> 6); ++w) total += red[w];
-        red[16] = total;
-    }
-    __syncthreads();
-    total = red[16];
-    __syncthreads();
+    double t[16], total = 0.0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) t[w] = red[16 * B + w];
+#pragma unroll
+    for (int w = 0; w < 16; ++w) total += t[w];
     return total;
 }
 
@@ -29,7 +29,7 @@ __device__ inline double block_sum(double v, double *red) {
 
 // r = rhs, x = 0, sc[CG_RNORM] = sc[CG_BNORM] = ||rhs||
 __global__ __launch_bounds__(1024) void cg_start_kernel(int m, const double *rhs, double *r, double *x, double *sc) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     double acc = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         double v = rhs[i];
@@ -37,7 +37,7 @@ __global__ __launch_bounds__(1024) void cg_start_kernel(int m, const double *rhs
         x[i] = 0.0;
         acc += v * v;
     }
-    double nrm = sqrt(block_sum(acc, red));
+    double nrm = sqrt(block_sum<0>(acc, red));
     if (threadIdx.x == 0) {
         sc[CG_RNORM] = nrm;
         sc[CG_BNORM] = nrm;
@@ -56,14 +56,14 @@ __global__ __launch_bounds__(1024) void cg_jacobi_kernel(int m, const double *r,
 // rz = z.r; pMp = p.Mp; alpha = rz / pMp; x += alpha p; rn = r - alpha Mp
 __global__ __launch_bounds__(1024) void cg_step1_kernel(int m, const double *z, const double *r, const double *p,
                                                         const double *Mp, double *x, double *rn, double *sc) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     double a = 0.0, b = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         a += z[i] * r[i];
         b += p[i] * Mp[i];
     }
-    double rz = block_sum(a, red);
-    double pMp = block_sum(b, red);
+    double rz = block_sum<0>(a, red);
+    double pMp = block_sum<1>(b, red);
     double alpha = rz / pMp;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         x[i] += alpha * p[i];
@@ -78,10 +78,10 @@ __global__ __launch_bounds__(1024) void cg_step1_kernel(int m, const double *z, 
 // beta = rn.z / rz; p = z + beta p; r = rn; sc[CG_RNORM] = ||r||
 __global__ __launch_bounds__(1024) void cg_step2_kernel(int m, const double *rn, const double *z, double *p, double *r,
                                                         double *sc) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     double a = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) a += rn[i] * z[i];
-    double beta = block_sum(a, red) / sc[CG_RZ];
+    double beta = block_sum<0>(a, red) / sc[CG_RZ];
     double c = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         p[i] = z[i] + beta * p[i];
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(1024) void cg_step2_kernel(int m, const double *rn,
         r[i] = v;
         c += v * v;
     }
-    double nrm = sqrt(block_sum(c, red));
+    double nrm = sqrt(block_sum<1>(c, red));
     if (threadIdx.x == 0) sc[CG_RNORM] = nrm;
 }
 
@@ -100,14 +100,14 @@ __global__ void cg_residual_kernel(int m, const double *rhs, const double *Mx, d
 
 __global__ __launch_bounds__(1024) void cg_true_residual_kernel(int m, const double *rhs, const double *Mx, double *r,
                                                                 double *sc) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     double acc = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         const double v = rhs[i] - Mx[i];
         r[i] = v;
         acc += v * v;
     }
-    const double nrm = sqrt(block_sum(acc, red));
+    const double nrm = sqrt(block_sum<0>(acc, red));
     if (threadIdx.x == 0) sc[CG_TRUE] = nrm;
 }
 
@@ -140,7 +140,7 @@ void cg_residual(hipStream_t s, int m, const double *rhs, const double *Mx, doub
 __global__ __launch_bounds__(1024) void cgj_start_kernel(int m, const double *rhs, const double *jac, double relTol,
                                                          double absTol, double *r, double *x, double *z, double *p,
                                                          double *sc) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     double acc = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         const double v = rhs[i], t = v / jac[i];
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(1024) void cgj_start_kernel(int m, const double *rh
         p[i] = t;
         acc += v * v;
     }
-    const double nrm = sqrt(block_sum(acc, red));
+    const double nrm = sqrt(block_sum<0>(acc, red));
     if (threadIdx.x == 0) {
         const double tol = fmax(fmin(absTol, nrm * relTol), 0.1 * absTol);
         sc[CG_RNORM] = nrm;
@@ -164,15 +164,15 @@ __global__ __launch_bounds__(1024) void cgj_start_kernel(int m, const double *rh
 template <bool HALF>
 __global__ __launch_bounds__(1024) void cgj_iter_kernel(int m, int iter, const double *jac, const double *Mp, double *x,
                                                         double *r, double *z, double *p, double *sc, double *report) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     if (sc[CG_STOP] == CG_RUNNING) {  // the same for every thread: only thread 0 writes it, below
         double a = 0.0, b = 0.0;
         for (int i = threadIdx.x; i < m; i += blockDim.x) {
             a += z[i] * r[i];
             b += p[i] * Mp[i];
         }
-        const double rz = block_sum(a, red);
-        const double pMp = block_sum(b, red);
+        const double rz = block_sum<0>(a, red);
+        const double pMp = block_sum<1>(b, red);
         const double alpha = rz / pMp;
         if (HALF) {
             for (int i = threadIdx.x; i < m; i += blockDim.x) x[i] += alpha * p[i];
@@ -186,13 +186,13 @@ __global__ __launch_bounds__(1024) void cgj_iter_kernel(int m, int iter, const d
             z[i] = t;
             a += v * t;
         }
-        const double beta = block_sum(a, red) / rz;
+        const double beta = block_sum<0>(a, red) / rz;
         double c = 0.0;
         for (int i = threadIdx.x; i < m; i += blockDim.x) {
             p[i] = z[i] + beta * p[i];
             c += r[i] * r[i];
         }
-        const double nrm = sqrt(block_sum(c, red));
+        const double nrm = sqrt(block_sum<1>(c, red));
         if (threadIdx.x == 0) {
             const double stop = (nrm != nrm)                                   ? CG_NAN
                                 : (iter > 20 && nrm > 0.01 * sc[CG_BNORM]) ? CG_STALLED
@@ -227,15 +227,143 @@ void cgj_half(hipStream_t s, int m, const double *z, const double *r, const doub
                                              const_cast<double *>(p), sc, nullptr);
 }
 
+// y = M p (coldot's columns, tri 0) by the 16 waves of one workgroup: a wave takes four
+// columns at a time, each summed in coldot's order; NU = rows per lane
+template <int NU>
+__device__ inline void small_symv(int m, const double *__restrict__ M, long ldm, const double *p, double *y) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double v[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) v[u] = (u < NU - 1 || lane + 64 * u < m) ? p[lane + 64 * u] : 0.0;
+    for (int j0 = 4 * w; j0 < m; j0 += 64) {
+        double a[4][NU], s[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const double *col = M + (long) min(j0 + c, m - 1) * ldm + lane;
+#pragma unroll
+            for (int u = 0; u < NU; ++u) a[c][u] = (u < NU - 1 || lane + 64 * u < m) ? col[64 * u] : 0.0;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            s[c] = 0.0;
+#pragma unroll
+            for (int u = 0; u < NU; ++u) s[c] += a[c][u] * v[u];
+            s[c] = wave_tree_sum(s[c]);
+            if (lane == 0 && j0 + c < m) y[j0 + c] = s[c];
+        }
+    }
+    __syncthreads();
+}
+
+// One workgroup, every vector in LDS, M from L2.  One CU reads it at about 70 GB/s: an
+// iteration takes 8 us at m = 200 (M 320 KB) and 15 at m = 368, where the two launches of
+// the queued form cost the host 10; hence CGS_MAX.  Statements and reduction orders of
+// cgj_iter.
+template <int NU>
+__global__ __launch_bounds__(1024) void cg_small_kernel(int m, const double *M, long ldm, const double *rhs,
+                                                        const double *jacG, double relTol, double absTol, int maxIter,
+                                                        int restart, double *crhs, double *xG, double *xHost,
+                                                        double *report) {
+    __shared__ double red[32];
+    __shared__ double b[CGS_MAX], jac[CGS_MAX], x[CGS_MAX], r[CGS_MAX], z[CGS_MAX], p[CGS_MAX], Mp[CGS_MAX];
+    const int tid = threadIdx.x;
+    double acc = 0.0;
+    if (tid < m) {
+        const double v = rhs[tid], q = jacG[tid];
+        b[tid] = v;
+        crhs[tid] = v;
+        jac[tid] = q;
+        r[tid] = v;
+        x[tid] = 0.0;
+        z[tid] = v / q;
+        p[tid] = v / q;
+        acc = 0.0 + v * v;
+    }
+    const double bnorm = sqrt(block_sum<0>(acc, red));
+    const double tol = fmax(fmin(absTol, bnorm * relTol), 0.1 * absTol);
+    double nrm = bnorm;
+    int stop = (nrm < tol) ? CG_TINY : CG_RUNNING, iter = 0;
+    if (stop == CG_RUNNING) {
+        small_symv<NU>(m, M, ldm, p, Mp);
+        for (; iter < maxIter; ++iter) {
+            double a = 0.0, c = 0.0;
+            if (tid < m) {
+                a = 0.0 + z[tid] * r[tid];
+                c = 0.0 + p[tid] * Mp[tid];
+            }
+            const double rz = block_sum<1>(a, red);
+            const double alpha = rz / block_sum<0>(c, red);
+            if (iter % restart == 5) {
+                if (tid < m) x[tid] += alpha * p[tid];
+                __syncthreads();
+                small_symv<NU>(m, M, ldm, x, Mp);
+                if (tid < m) {
+                    const double v = b[tid] - Mp[tid], t = v / jac[tid];
+                    r[tid] = v;
+                    z[tid] = t;
+                    p[tid] = t;
+                }
+                __syncthreads();
+                small_symv<NU>(m, M, ldm, p, Mp);
+                continue;
+            }
+            a = 0.0;
+            if (tid < m) {
+                x[tid] += alpha * p[tid];
+                const double v = r[tid] - alpha * Mp[tid], t = v / jac[tid];
+                r[tid] = v;
+                z[tid] = t;
+                a = 0.0 + v * t;
+            }
+            const double beta = block_sum<1>(a, red) / rz;
+            c = 0.0;
+            if (tid < m) {
+                p[tid] = z[tid] + beta * p[tid];
+                c = 0.0 + r[tid] * r[tid];
+            }
+            nrm = sqrt(block_sum<0>(c, red));
+            stop = (nrm != nrm)                          ? CG_NAN
+                   : (iter > 20 && nrm > 0.01 * bnorm) ? CG_STALLED
+                   : (nrm < tol)                         ? CG_CONVERGED
+                                                         : CG_RUNNING;
+            if (stop != CG_RUNNING) break;
+            small_symv<NU>(m, M, ldm, p, Mp);
+        }
+    }
+    if (stop != CG_TINY && tid < m) {
+        xG[tid] = x[tid];
+        if (xHost) xHost[tid] = x[tid];
+    }
+    if (tid == 0) {
+        report[CG_RNORM] = nrm;
+        report[CG_BNORM] = bnorm;
+        report[CG_TOL] = tol;
+        report[CG_ITER] = iter;
+        report[CG_STOP] = stop;
+    }
+}
+
+void cg_small(hipStream_t s, int m, const double *M, long ldm, const double *rhs, const double *jac, double relTol,
+              double absTol, int maxIter, int restart, double *crhs, double *x, double *xHost, double *report) {
+#define HDK_CGS(nu)                                                                                              \
+    case nu:                                                                                                     \
+        cg_small_kernel<nu><<<1, 1024, 0, s>>>(m, M, ldm, rhs, jac, relTol, absTol, maxIter, restart, crhs, x,   \
+                                               xHost, report);                                                   \
+        break;
+    switch ((m + 63) / 64) {
+        HDK_CGS(1) HDK_CGS(2) HDK_CGS(3) HDK_CGS(4)
+    }
+#undef HDK_CGS
+}
+
 // ---- Lanczos (linalg/hdsdp_lanczos.c:196-286) ---------------------------------
 
 // One Lanczos orthogonalisation step on w = Op(v_k):
 //   w -= H(k,k-1) V_{k-1};  alp = -w.V_k;  w += alp V_k;  H(k,k) = -alp
-//   norm = ||w||;  v = w / norm (or 0);  if norm > 0: V_{k+1} = v, H(k+1,k) = H(k,k+1) = norm
-// sc[LZ_ALPHA] = -alp, sc[LZ_NORM] = norm.
+//   norm = ||w||;  V_{k+1} = v = w / norm (or 0);  H(k+1,k) = norm
 __global__ __launch_bounds__(1024) void lz_step_kernel(int n, int k, double *w, double *V, double *H, int ldh, double *v,
-                                                       double *sc, double *hist) {
-    __shared__ double red[17];
+                                                       double *hist) {
+    __shared__ double red[32];
     const double *Vk = V + (long) k * n;
     if (k > 0) {
         const double *Vkm = V + (long) (k - 1) * n;
@@ -245,78 +373,237 @@ __global__ __launch_bounds__(1024) void lz_step_kernel(int n, int k, double *w, 
     }
     double a = 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) a += w[i] * Vk[i];
-    double alp = -block_sum(a, red);
+    double alp = -block_sum<0>(a, red);
     double c = 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         double t = w[i] + alp * Vk[i];
         w[i] = t;
         c += t * t;
     }
-    double nrm = sqrt(block_sum(c, red));
+    double nrm = sqrt(block_sum<1>(c, red));
     double inv = (nrm > 0.0) ? 1.0 / nrm : 0.0;
     double *Vn = V + (long) (k + 1) * n;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         double t = (nrm > 0.0) ? w[i] * inv : 0.0;
         v[i] = t;
-        if (nrm > 0.0) Vn[i] = t;
+        Vn[i] = t;
     }
     if (threadIdx.x == 0) {
-        H[k + k * ldh] = -alp;
-        if (nrm > 0.0) {
-            H[(k + 1) + k * ldh] = nrm;
-            H[k + (k + 1) * ldh] = nrm;
-        }
-        sc[LZ_ALPHA] = -alp;
-        sc[LZ_NORM] = nrm;
+        H[(k + 1) + k * ldh] = (nrm > 0.0) ? nrm : 0.0;
         hist[2 * k] = -alp;
         hist[2 * k + 1] = nrm;
     }
 }
 
-// v = x / ||x|| (or 0); V_0 = v (start vector normalisation)
-__global__ __launch_bounds__(1024) void lz_start_kernel(int n, const double *x, double *v, double *V) {
-    __shared__ double red[17];
+// x = x0 (+ pert); v = V_0 = x / ||x|| (or 0)
+__global__ __launch_bounds__(1024) void lz_start_kernel(int n, const double *x0, const double *pert, double *v,
+                                                        double *V) {
+    __shared__ double red[32];
     double c = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) c += x[i] * x[i];
-    double nrm = sqrt(block_sum(c, red));
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const double x = pert ? x0[i] + pert[i] : x0[i];
+        c += x * x;
+    }
+    double nrm = sqrt(block_sum<0>(c, red));
     double inv = (nrm > 0.0) ? 1.0 / nrm : 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        double t = (nrm > 0.0) ? x[i] * inv : 0.0;
+        const double x = pert ? x0[i] + pert[i] : x0[i];
+        double t = (nrm > 0.0) ? x * inv : 0.0;
         v[i] = t;
         V[i] = t;
     }
 }
 
 // z = V[:, 0:kp1] y
-__global__ void lz_comb_kernel(int n, int kp1, const double *V, const double *y, double *z) {
+__global__ void lz_comb_kernel(int n, int kp1, const double *V, LzCoef y, double *z) {
     for (int i = threadIdx.x + blockIdx.x * blockDim.x; i < n; i += blockDim.x * gridDim.x) {
         double s = 0.0;
-        for (int c = 0; c < kp1; ++c) s += V[i + (long) c * n] * y[c];
+        for (int c = 0; c < kp1; ++c) s += V[i + (long) c * n] * y.y[c];
         z[i] = s;
     }
 }
 
+// y_j = <A(lo:hi, j), x(lo:hi)> with coldot's rows and order of summation (tri 0, 1, 2) for
+// the n <= 64 NU columns, by the 16 waves of one workgroup, four columns at a time; x
+// and y in LDS
+template <int NU, int TRI>
+__device__ inline void small_coldot(int n, const double *__restrict__ A, const double *x, double *y) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int j0 = 4 * w; j0 < n; j0 += 64) {
+        double a[4][NU], s[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int j = min(j0 + c, n - 1), lo = (TRI == 1) ? j : 0, hi = (TRI == 2) ? j + 1 : n;
+            const double *col = A + (long) j * n + lo + lane;
+#pragma unroll
+            for (int u = 0; u < NU; ++u) a[c][u] = (lo + lane + 64 * u < hi) ? col[64 * u] : 0.0;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int j = min(j0 + c, n - 1), lo = (TRI == 1) ? j : 0, hi = (TRI == 2) ? j + 1 : n;
+            s[c] = 0.0;
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+                s[c] += a[c][u] * ((lo + lane + 64 * u < hi) ? x[lo + lane + 64 * u] : 0.0);
+            s[c] = wave_tree_sum(s[c]);
+            if (lane == 0 && j0 + c < n) y[j0 + c] = s[c];
+        }
+    }
+    __syncthreads();
+}
+
+// out = L^-1 (-D) L^-T in (in, out, t in LDS)
+template <int NU>
+__device__ inline void small_op(int n, const double *Li, const double *LiT, const double *D, const double *in, double *t,
+                                double *out) {
+    small_coldot<NU, 1>(n, Li, in, out);
+    small_coldot<NU, 0>(n, D, out, t);
+    if ((int) threadIdx.x < n) t[threadIdx.x] = -1.0 * t[threadIdx.x];
+    __syncthreads();
+    small_coldot<NU, 2>(n, LiT, t, out);
+}
+
+// A Lanczos step of a small block is bound by its four launches (three products, the
+// step): about 18 us of host time at any n.  In one workgroup it takes the two triangles
+// and D at one CU's rate from L2: 6 us at n = 50, 12 at n = 121, 22 at n = 200; hence LZS_MAX.
+template <int NU>
+__global__ __launch_bounds__(1024) void lz_small_steps_kernel(int n, int k0, int k1, const double *x0,
+                                                              const double *pert, const double *Li, const double *LiT,
+                                                              const double *D, double *V, double *H, int ldh,
+                                                              double *hist) {
+    __shared__ double red[32], v[LZS_MAX], w[LZS_MAX], t[LZS_MAX];
+    const int i = threadIdx.x;
+    double vm = 0.0;  // V_{k - 1} and its norm at the step before
+    double prev = 0.0;
+    if (k0 == 0) {
+        double x = 0.0, c = 0.0;
+        if (i < n) {
+            x = pert ? x0[i] + pert[i] : x0[i];
+            c = 0.0 + x * x;
+        }
+        const double nrm = sqrt(block_sum<0>(c, red));
+        const double inv = (nrm > 0.0) ? 1.0 / nrm : 0.0;
+        if (i < n) {
+            const double q = (nrm > 0.0) ? x * inv : 0.0;
+            v[i] = q;
+            V[i] = q;
+        }
+    } else {
+        prev = H[k0 + (k0 - 1) * ldh];
+        if (i < n) {
+            vm = V[i + (long) (k0 - 1) * n];
+            v[i] = V[i + (long) k0 * n];
+        }
+    }
+    __syncthreads();
+    for (int k = k0; k < k1; ++k) {
+        small_op<NU>(n, Li, LiT, D, v, t, w);
+        double q = 0.0, vk = 0.0, a = 0.0;
+        if (i < n) {
+            q = w[i];
+            vk = v[i];
+            if (k > 0) q += -prev * vm;
+            a = 0.0 + q * vk;
+        }
+        const double alp = -block_sum<1>(a, red);
+        double c = 0.0;
+        if (i < n) {
+            q = q + alp * vk;
+            c = 0.0 + q * q;
+        }
+        const double nrm = sqrt(block_sum<0>(c, red));
+        const double inv = (nrm > 0.0) ? 1.0 / nrm : 0.0;
+        vm = vk;
+        prev = (nrm > 0.0) ? nrm : 0.0;
+        if (i < n) {
+            const double u = (nrm > 0.0) ? q * inv : 0.0;
+            v[i] = u;
+            V[i + (long) (k + 1) * n] = u;
+        }
+        if (i == 0) {
+            H[(k + 1) + k * ldh] = prev;
+            hist[2 * k] = -alp;
+            hist[2 * k + 1] = nrm;
+        }
+        __syncthreads();
+    }
+}
+
+template <int NU>
+__global__ __launch_bounds__(1024) void lz_small_bound_kernel(int n, int kp1, double e1, LzCoef y1, LzCoef y2,
+                                                              const double *Li, const double *LiT, const double *D,
+                                                              const double *V, double *warm, double *report) {
+    __shared__ double red[32], z[LZS_MAX], w[LZS_MAX], t[LZS_MAX];
+    const int i = threadIdx.x;
+    double s1 = 0.0, s2 = 0.0;
+    if (i < n) {
+        for (int c = 0; c < kp1; ++c) {
+            const double q = V[i + (long) c * n];
+            s1 += q * y1.y[c];
+            s2 += q * y2.y[c];
+        }
+        z[i] = s1;
+    }
+    __syncthreads();
+    small_op<NU>(n, Li, LiT, D, z, t, w);
+    double c = 0.0;
+    if (i < n) {
+        const double q = w[i];
+        warm[i] = q;
+        const double u = q + -e1 * s1;
+        c = 0.0 + u * u;
+        z[i] = s2;
+    }
+    const double r1 = sqrt(block_sum<0>(c, red));
+    small_op<NU>(n, Li, LiT, D, z, t, w);
+    c = 0.0;
+    if (i < n) {
+        const double u = w[i] + -e1 * s2;
+        c = 0.0 + u * u;
+    }
+    const double r2 = sqrt(block_sum<1>(c, red));
+    if (i == 0) {
+        report[LZ_R1] = r1;
+        report[LZ_R2] = r2;
+    }
+}
+
+#define HDK_LZS(call)                      \
+    switch ((n + 63) / 64) {               \
+        case 1: { constexpr int NU = 1; call; break; } \
+        case 2: { constexpr int NU = 2; call; break; } \
+        default: { constexpr int NU = 3; call; break; } \
+    }
+void lz_small_steps(hipStream_t s, int n, int k0, int k1, const double *x0, const double *pert, const double *Li,
+                    const double *LiT, const double *D, double *V, double *H, int ldh, double *hist) {
+    HDK_LZS((lz_small_steps_kernel<NU><<<1, 1024, 0, s>>>(n, k0, k1, x0, pert, Li, LiT, D, V, H, ldh, hist)))
+}
+void lz_small_bound(hipStream_t s, int n, int kp1, double e1, const LzCoef &y1, const LzCoef &y2, const double *Li,
+                    const double *LiT, const double *D, const double *V, double *warm, double *report) {
+    HDK_LZS((lz_small_bound_kernel<NU><<<1, 1024, 0, s>>>(n, kp1, e1, y1, y2, Li, LiT, D, V, warm, report)))
+}
+#undef HDK_LZS
+
 // y += a x; sc[slot] = ||y||
 __global__ __launch_bounds__(1024) void axpy_norm_kernel(int n, double a, const double *x, double *y, double *sc, int slot) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     double c = 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         double t = y[i] + a * x[i];
         y[i] = t;
         c += t * t;
     }
-    double nrm = sqrt(block_sum(c, red));
+    double nrm = sqrt(block_sum<0>(c, red));
     if (threadIdx.x == 0) sc[slot] = nrm;
 }
 
-void lz_step(hipStream_t s, int n, int k, double *w, double *V, double *H, int ldh, double *v, double *sc,
-             double *hist) {
-    lz_step_kernel<<<1, 1024, 0, s>>>(n, k, w, V, H, ldh, v, sc, hist);
+void lz_step(hipStream_t s, int n, int k, double *w, double *V, double *H, int ldh, double *v, double *hist) {
+    lz_step_kernel<<<1, 1024, 0, s>>>(n, k, w, V, H, ldh, v, hist);
 }
-void lz_start(hipStream_t s, int n, const double *x, double *v, double *V) {
-    lz_start_kernel<<<1, 1024, 0, s>>>(n, x, v, V);
+void lz_start(hipStream_t s, int n, const double *x0, const double *pert, double *v, double *V) {
+    lz_start_kernel<<<1, 1024, 0, s>>>(n, x0, pert, v, V);
 }
-void lz_comb(hipStream_t s, int n, int kp1, const double *V, const double *y, double *z) {
+void lz_comb(hipStream_t s, int n, int kp1, const double *V, const LzCoef &y, double *z) {
     lz_comb_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, kp1, V, y, z);
 }
 void axpy_norm(hipStream_t s, int n, double a, const double *x, double *y, double *sc, int slot) {
@@ -338,7 +625,7 @@ void axpy(hipStream_t s, long n, double a, const double *x, double *y) {
 // M_ii += reg where reg = min(r * min_i M_ii, 1e-5), dropped below 1e-14
 // (interface/hdsdp_schur.c:348-373)
 __global__ __launch_bounds__(1024) void regularize_kernel(int m, double *M, long ldm, double r) {
-    __shared__ double red[17];
+    __shared__ double red[32];
     double mn = 1e+30;
     for (int i = threadIdx.x; i < m; i += blockDim.x) mn = fmin(mn, M[i + i * ldm]);
     for (int off = 32; off > 0; off >>= 1) mn = fmin(mn, __shfl_down(mn, off));

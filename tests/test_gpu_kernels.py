@@ -486,3 +486,42 @@ def test_dense_gram_build(gpu_lib, n, m):
     u = 1.1e-16
     assert np.max(np.abs(M - ref)) <= 25.0 * n * u * np.max(np.abs(ref))
     assert np.max(np.abs(a - np.einsum("kij,ij->k", A, W))) <= 25.0 * n * u * np.sqrt(n) * np.max(np.abs(W))
+
+
+# the one-workgroup forms of the Schur CG (m <= 256) and of Lanczos (n <= 160) and the first
+# sizes past them; rows per lane change at multiples of 64
+@pytest.mark.parametrize("n,m", [(2, 1), (63, 64), (64, 65), (128, 129), (129, 256), (160, 257), (161, 192)])
+def test_small_cg_and_lanczos_edges(gpu_lib, oracle, n, m):
+    """Jacobi CG solutions and two ratio tests (the second from the warm start) against the
+    oracle's loops.  CG stops at a residual below 1e-11 |rhs| on both sides, so solutions
+    agree to 2e-11 cond(M) < 1e-9 (the added diagonal keeps cond(M) below 10).  The two
+    Lanczos runs of at most 30 steps differ by their rounding, held to 1e-6 here: the diagonal
+    dS makes the spectrum's end well separated."""
+    rng = np.random.default_rng(1000 * n + m)
+    # single-entry constraints on distinct positions, the first ones on the diagonal
+    r, c = np.tril_indices(n)
+    pick = rng.permutation(len(r))[:m]
+    one = np.ones(1)
+    con = [dt.Coeff(dt.SPARSE, n, row=[r[k]], col=[c[k]], val=one) for k in pick]
+    S, (C, _, _) = _spd_coeffs(n, rng)
+    rhs = rng.standard_normal(len(con))
+    dy = rng.standard_normal(len(con)) / np.sqrt(n)
+    res = []
+    for lib in (gpu_lib, oracle):
+        d = dt.Dev(lib, [C] + con)
+        d.kkt_params(1e-11, 1e-11, 200, -1)
+        d.update(1.0, 0.0, np.zeros(len(con)), 0.0, 0)
+        assert d.factorize(0) == 1
+        d.schur(0, 0.0)
+        d.add_diag(np.ones(len(con)))
+        assert d.kkt_factorize() == 0
+        x = d.kkt_solve(rhs)
+        tiny = d.kkt_solve(1e-14 * rhs)  # below the tolerance: the solution stays as it was
+        d.update(0.0, 1.0, dy, 0.0, 2)
+        steps = [d.ratio(0), d.ratio(0)]
+        res.append((x, tiny, steps))
+        d.close()
+    (gx, gt, gs), (ox, ot, os_) = res
+    assert rel(gx, ox) < 1e-9
+    assert np.all(gt == 0.0) and np.all(ot == 0.0)
+    assert rel(gs, os_) < 1e-6
