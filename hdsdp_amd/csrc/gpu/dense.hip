@@ -38,12 +38,15 @@ struct Mfma<float> {
 
 // k range of one output tile when an operand is triangular: tri 1 = op(B) lower
 // (B(k, j) = 0 for k < j), tri 2 = op(A) lower (A(i, k) = 0 for k > i), tri 3 = op(B) upper
-// (B(k, j) = 0 for k > j).  Only exact zeros are skipped, so the result is the same as
+// (B(k, j) = 0 for k > j), tri 4 = op(A) upper and op(B) lower (zero for k < max(i, j)),
+// tri 5 = op(A) upper.  Only exact zeros are skipped, so the result is the same as
 // the full product.
 __device__ inline void tri_krange(int tri, int i0, int j0, int tile, int K, int &kLo, int &kHi) {
     kLo = 0;
     kHi = K;
     if (tri == 1) kLo = (j0 / KSTEP) * KSTEP;
+    if (tri == 4) kLo = (max(i0, j0) / KSTEP) * KSTEP;
+    if (tri == 5) kLo = (i0 / KSTEP) * KSTEP;
     if (tri == 2) kHi = (i0 + tile < K) ? i0 + tile : K;
     if (tri == 3) kHi = (j0 + tile < K) ? j0 + tile : K;
 }
@@ -54,7 +57,7 @@ __device__ inline void tri_krange(int tri, int i0, int j0, int tile, int K, int 
 // share of the triangle (a 2-D grid gives tile column x to XCD x mod 8, and the
 // columns near the diagonal end hold unequal work).
 //
-// With tri == 2 (op(A) lower: the work of a tile grows with its row) the tile row of
+// With tri == 2 (op(A) lower: the work of a tile grows with its row; 4 and 5 shrink with it) the tile row of
 // a 2-D grid is rotated by the other grid coordinates: workgroup x + gridDim.x (y + ...)
 // goes to XCD (x + ...) mod 8, so with 8k tile rows XCD x would receive every tile of
 // row x (the heaviest rows all on one XCD); the rotation gives each XCD every row.
@@ -62,11 +65,11 @@ __device__ inline void tile_xy(int lin, int &bx, int &by, int tri = 0) {
     if (!lin) {
         bx = blockIdx.x;
         by = blockIdx.y;
-        if (tri == 2) bx = (int) ((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
+        if (tri == 2 || tri >= 4) bx = (int) ((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
         return;
     }
-    // a triangular operand makes the later tiles the longer ones: those go first
-    const int t = tri ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    // a triangular operand makes the later tiles the longer ones (tri 4: the earlier): those go first
+    const int t = (tri && tri != 4) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
     int x = (int) ((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
     while ((x + 1) * (x + 2) / 2 <= t) ++x;
     while (x * (x + 1) / 2 > t) --x;
@@ -456,6 +459,131 @@ static void gemm_big(hipStream_t s, bool transA, bool transB, bool lower, int M,
 #undef HDK_GEMM_BIG
 }
 
+// 32 x 32 tiles for products that leave CUs idle on 64-wide tiles (the levels of a
+// triangular inverse, S^-1 of a small block, the k parts of a rank-m update with few
+// tiles).  On 64-wide tiles such a product is bound by the MFMA chain of its few tiles, one
+// wave per SIMD: 0.43 us per 16 k whatever the rest of the chip does; here a tile takes a
+// quarter of it on four times the workgroups, with slabs of 64 k so that a load latency is
+// paid once per 64 k.  MFMA rows are tile columns, so that a wave loads and stores 16
+// consecutive rows.  Each operand is staged in its own order: rows consecutive as [k][48], k
+// consecutive as [row][66], both free of bank conflicts in the fragment reads.  Every
+// output sums its k in ascending order like the other tile widths, so the choice does not change
+// a bit.  The last batch entry may have fewer rows (mLast > 0) and a shorter k (kLast > 0).
+constexpr int TT = 32, TK = 64, TLR = 48, TLK = 66;
+
+template <typename T, bool KC>
+__device__ inline void thin_fetch(const T *X, long ldx, int rows, int K, int r0, int k0, int tid, T (&v)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        // addresses clamped into the operand; the k beyond K are zeroed in thin_stash
+        const int r = min(r0 + (KC ? (tid >> 6) + 4 * u : (tid & 31)), rows - 1);
+        const int k = min(k0 + (KC ? (tid & 63) : (tid >> 5) + 8 * u), K - 1);
+        v[u] = KC ? X[k + r * ldx] : X[r + k * ldx];
+    }
+}
+
+template <typename T, bool KC>
+__device__ inline void thin_stash(T *S, int K, int k0, int tid, const T (&v)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int r = KC ? (tid >> 6) + 4 * u : (tid & 31), k = KC ? (tid & 63) : (tid >> 5) + 8 * u;
+        S[KC ? r * TLK + k : k * TLR + r] = (k0 + k < K) ? v[u] : (T) 0;
+    }
+}
+
+template <typename T, bool TA, bool TB, bool LOWER>
+__global__ __launch_bounds__(256) void gemm_thin_kernel(int M, int N, int K, T alpha, const T *A, int lda, long sA,
+                                                        const T *B, int ldb, long sB, T beta, T *C, int ldc, long sC,
+                                                        int tri, int lin, int mLast, int kLast) {
+    constexpr bool KCA = TA, KCB = !TB;  // operand consecutive along k
+    __shared__ T As[KCA ? TT * TLK : TK * TLR], Bs[KCB ? TT * TLK : TK * TLR];
+    if (blockIdx.z == gridDim.z - 1) {
+        if (mLast > 0) M = mLast;
+        if (kLast > 0) K = kLast;
+    }
+    int bx, by;
+    tile_xy(lin, bx, by, tri);
+    const int i0 = bx * TT, j0 = by * TT;
+    if (i0 >= M || j0 >= N || (LOWER && i0 + TT - 1 < j0)) return;
+    int kLo, kHi;
+    tri_krange(tri, i0, j0, TT, K, kLo, kHi);
+    A += (long) blockIdx.z * sA;
+    B += (long) blockIdx.z * sB;
+    C += (long) blockIdx.z * sC;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wi = (wave & 1) * 16, wj = (wave >> 1) * 16, lr = lane & 15, lk = lane >> 4;
+    const int i = i0 + wi + lr;
+    T cin[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int j = j0 + wj + Mfma<T>::row(lk, r);
+        cin[r] = (beta != (T) 0 && i < M && j < N && (!LOWER || i >= j)) ? C[i + (long) j * ldc] : (T) 0;
+    }
+    typename Mfma<T>::acc_t acc = {0, 0, 0, 0};
+    T ra[8], rb[8];
+    if (kLo < kHi) {
+        thin_fetch<T, KCA>(A, lda, M, K, i0, kLo, tid, ra);
+        thin_fetch<T, KCB>(B, ldb, N, K, j0, kLo, tid, rb);
+    }
+    for (int k0 = kLo; k0 < kHi; k0 += TK) {
+        thin_stash<T, KCA>(As, K, k0, tid, ra);
+        thin_stash<T, KCB>(Bs, K, k0, tid, rb);
+        __syncthreads();
+        if (k0 + TK < kHi) {
+            thin_fetch<T, KCA>(A, lda, M, K, i0, k0 + TK, tid, ra);
+            thin_fetch<T, KCB>(B, ldb, N, K, j0, k0 + TK, tid, rb);
+        }
+#pragma unroll
+        for (int kk = 0; kk < TK; kk += 4) {
+            const T a = KCA ? As[(wi + lr) * TLK + kk + lk] : As[(kk + lk) * TLR + wi + lr];
+            const T b = KCB ? Bs[(wj + lr) * TLK + kk + lk] : Bs[(kk + lk) * TLR + wj + lr];
+            acc = Mfma<T>::op(b, a, acc);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int j = j0 + wj + Mfma<T>::row(lk, r);
+        if (i < M && j < N && (!LOWER || i >= j)) C[i + (long) j * ldc] = alpha * acc[r] + beta * cin[r];
+    }
+}
+
+template <typename T>
+static void gemm_thin(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int K, T alpha, const T *A,
+                      int lda, long strideA, const T *B, int ldb, long strideB, T beta, T *C, int ldc, long strideC,
+                      int batch, int tri, int mLast = 0, int kLast = 0) {
+    const int mt = (M + TT - 1) / TT, nt = (N + TT - 1) / TT;
+    const int lin = (lower && mt == nt) ? 1 : 0;
+    const dim3 grid(lin ? mt * (mt + 1) / 2 : mt, lin ? 1 : nt, batch);
+#define HDK_GEMM_THIN(ta, tb, lo)                                                                               \
+    if (transA == ta && transB == tb && lower == lo) {                                                          \
+        gemm_thin_kernel<T, ta, tb, lo><<<grid, 256, 0, s>>>(M, N, K, alpha, A, lda, strideA, B, ldb, strideB,  \
+                                                             beta, C, ldc, strideC, tri, lin, mLast, kLast);    \
+        return;                                                                                                 \
+    }
+    HDK_GEMM_THIN(false, false, false)
+    HDK_GEMM_THIN(false, true, false)
+    HDK_GEMM_THIN(true, false, false)
+    HDK_GEMM_THIN(true, true, false)
+    HDK_GEMM_THIN(false, false, true)
+    HDK_GEMM_THIN(false, true, true)
+    HDK_GEMM_THIN(true, false, true)
+    HDK_GEMM_THIN(true, true, true)
+#undef HDK_GEMM_THIN
+}
+
+// Up to THIN_TILES tiles of 64 x 64 the 32-wide tiles are faster or equal; beyond, both fill
+// the chip and the wider tile moves half the operands.  Measured, us, 64-wide against
+// 32-wide: 200^3 17.6 and 8.3, 512^3 36.6 and 14.4, 1000^3 (256 tiles) 69.5 and 64.1,
+// 1300^3 (441) 125 and 132; 16 products of 256^3 (256 tiles) 21.9 and 18.6, 32 (512) 31.3
+// both; S^-1 of n = 500 34.5 and 13.2; a lower rank-3001 update at n = 301 in two k parts 394 on
+// 128-wide tiles and 37.
+constexpr long THIN_TILES = 400;
+static bool use_thin(int M, int N, int K, bool lower, int batch) {
+    const long tiles = (long) ((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE) * batch / (lower ? 2 : 1);
+    return K >= 1 && tiles <= THIN_TILES;
+}
+
 template <typename T>
 void gemm(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int K, T alpha, const T *A,
           int lda, long strideA, const T *B, int ldb, long strideB, T beta, T *C, int ldc, long strideC,
@@ -467,6 +595,11 @@ void gemm(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int
     if (bigTiles >= 192 && K >= 256) {
         gemm_big<T>(s, transA, transB, lower, M, N, K, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
                     strideC, batch, tri, 0);
+        return;
+    }
+    if (use_thin(M, N, K, lower, batch)) {
+        gemm_thin<T>(s, transA, transB, lower, M, N, K, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
+                     strideC, batch, tri);
         return;
     }
     const int mt = (M + TILE - 1) / TILE, nt = (N + TILE - 1) / TILE;
@@ -493,6 +626,15 @@ template void gemm<double>(hipStream_t, bool, bool, bool, int, int, int, double,
                            const double *, int, long, double, double *, int, long, int, int);
 template void gemm<float>(hipStream_t, bool, bool, bool, int, int, int, float, const float *, int, long,
                           const float *, int, long, float, float *, int, long, int, int);
+
+// W = Li^T Li for a lower-triangular Li (n x n, zeros above): entry (i, j) sums k >= max(i, j)
+// only, n^3 / 3 multiply-adds, and is symmetric to the bit, so from THIN_TILES tiles on the
+// lower half is formed and mirrored (n^3 / 6).  n = 2000: 83 us, the full product 366.
+void gram_lower(hipStream_t s, int n, const double *Li, double *W) {
+    const bool half = !use_thin(n, n, n, false, 1);
+    gemm<double>(s, true, false, half, n, n, n, 1.0, Li, n, 0, Li, n, 0, 0.0, W, n, 0, 1, 4);
+    if (half) mirror_lower<double>(s, n, W, n);
+}
 
 // P_z = alpha X_z^T X_z (lower, r x r, ld r, stride r^2) over the k slices z of kc (the
 // last one kLast wide) of the k panels X (PANEL above; slab doubles per 16 k)
@@ -599,8 +741,12 @@ void gemm_splitk(hipStream_t s, bool transA, bool transB, bool lower, int M, int
     const int parts = (K + kc - 1) / kc;
     const int kLast = K - (parts - 1) * kc;
     const long sA = transA ? kc : (long) kc * lda, sB = transB ? (long) kc * ldb : kc;
-    gemm_big<T>(s, transA, transB, lower, M, N, kc, (T) 1, A, lda, sA, B, ldb, sB, (T) 0, work, M, (long) mn, parts,
-                0, kLast);
+    if (use_thin(M, N, kc, lower, parts))
+        gemm_thin<T>(s, transA, transB, lower, M, N, kc, (T) 1, A, lda, sA, B, ldb, sB, (T) 0, work, M, (long) mn,
+                     parts, 0, 0, kLast);
+    else
+        gemm_big<T>(s, transA, transB, lower, M, N, kc, (T) 1, A, lda, sA, B, ldb, sB, (T) 0, work, M, (long) mn,
+                    parts, 0, kLast);
     splitk_reduce_kernel<T><<<4096, 256, 0, s>>>(M, N, parts, alpha, work, beta, C, ldc, lower ? 1 : 0);
 }
 
@@ -621,7 +767,9 @@ __global__ void place_diag_kernel(int n, int span, const double *Dinv, T *Linv, 
 }
 
 // inv([[A, 0], [B, C]]) = [[A^-1, 0], [-C^-1 B A^-1, C^-1]], applied level by level
-// with every pair of one level batched into two GEMMs.
+// with every pair of one level batched into two GEMMs.  On the 32-wide tiles a shorter last
+// pair is in the same two launches; n = 500 takes 40 us (129 on 64-wide tiles with launches
+// of its own for that pair), n = 2000 172 (442).
 template <typename T>
 void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work, int span) {
     if (span <= 0 || span > n) span = n;
@@ -629,16 +777,24 @@ void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Lin
     for (int sz = NB; sz < span; sz *= 2) {
         int npair = n / (2 * sz);
         long strideL = 2L * sz * (ldl + 1), strideI = 2L * sz * (ldi + 1), strideW = (long) sz * sz;
+        const int o = npair * 2 * sz, sc = std::max(0, n - o - sz);  // rows of a last, shorter pair
+        // W = L21 Linv11 (Linv11 lower), then Linv21 = -Linv22 W (Linv22 lower)
+        if (use_thin(sz, sz, sz, false, npair + 1)) {
+            const int cnt = npair + (sc > 0 ? 1 : 0);
+            if (cnt == 0) continue;
+            gemm_thin<T>(s, false, false, false, sz, sz, sz, (T) 1, L + sz, ldl, strideL, Linv, ldi, strideI, (T) 0,
+                         work, sz, strideW, cnt, 1, sc, 0);
+            gemm_thin<T>(s, false, false, false, sz, sz, sz, (T) -1, Linv + (long) sz * (ldi + 1), ldi, strideI, work,
+                         sz, strideW, (T) 0, Linv + sz, ldi, strideI, cnt, 2, sc, sc);
+            continue;
+        }
         if (npair > 0) {
-            // W = L21 Linv11 (Linv11 lower), then Linv21 = -Linv22 W (Linv22 lower)
             gemm<T>(s, false, false, false, sz, sz, sz, (T) 1, L + sz, ldl, strideL, Linv, ldi, strideI, (T) 0,
                     work, sz, strideW, npair, 1);
             gemm<T>(s, false, false, false, sz, sz, sz, (T) -1, Linv + (long) sz * (ldi + 1), ldi, strideI, work,
                     sz, strideW, (T) 0, Linv + sz, ldi, strideI, npair, 2);
         }
-        int o = npair * 2 * sz, rem = n - o;
-        if (rem > sz) {
-            int sc = rem - sz;
+        if (sc > 0) {
             gemm<T>(s, false, false, false, sc, sz, sz, (T) 1, L + (o + sz) + (long) o * ldl, ldl, 0,
                     Linv + o + (long) o * ldi, ldi, 0, (T) 0, work, sc, 0, 1, 1);
             gemm<T>(s, false, false, false, sc, sz, sc, (T) -1, Linv + (long) (o + sz) * (ldi + 1), ldi, 0, work,

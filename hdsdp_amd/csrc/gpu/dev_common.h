@@ -57,12 +57,15 @@ constexpr int NB = 64;     // Cholesky / triangular-inverse block
 // C = alpha * op(A) * op(B) + beta * C over `batch` problems (column-major).
 // lower != 0 restricts the output to i >= j (tiles above the diagonal skipped).
 // tri = 1 when op(B) is lower triangular, 2 when op(A) is, 3 when op(B) is upper
-// triangular: the k ranges that multiply the zero triangle are skipped (the stored zeros
-// must be present).
+// triangular, 5 when op(A) is, 4 when op(A) is upper and op(B) lower: the k ranges that
+// multiply the zero triangle are skipped (the stored zeros must be present).
 template <typename T>
 void gemm(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int K, T alpha,
           const T *A, int lda, long strideA, const T *B, int ldb, long strideB, T beta, T *C,
           int ldc, long strideC, int batch = 1, int tri = 0);
+
+// W = Li^T Li, both triangles, for a lower-triangular n x n Li with zeros above the diagonal
+void gram_lower(hipStream_t s, int n, const double *Li, double *W);
 
 // gemm with the k range split into parts whose partial products go to work (P x M x N)
 // and are summed in a fixed order, for products with few output tiles and long k

@@ -1489,8 +1489,7 @@ hdsdp_retcode hdsdp_dev_schur(hdsdp_dev *d, int typeKKT, double Rd, double *asin
         if (typeKKT != 1) prof_begin(d, HDSDP_PROF_SCHUR);
         DCALL(ensure_linv(d, 0));
         // W = S^-1 = L^-T L^-1
-        hdk::gemm<double>(d->st, true, false, false, n, n, n, 1.0, d->Li[0], n, 0, d->Li[0], n, 0, 0.0, d->W, n, 0,
-                          1);
+        hdk::gram_lower(d->st, n, d->Li[0], d->W);
     }
     if (Rd != 0.0)
         hdk::gemm<double>(d->st, false, false, false, n, n, n, 1.0, d->W, n, 0, d->W, n, 0, 0.0, d->W2, n, 0, 1);
@@ -1799,11 +1798,11 @@ hdsdp_retcode hdsdp_dev_primal(hdsdp_dev *d, double mu, const double *y, const d
     hdk::mirror_lower<double>(d->st, n, d->S[2], n);
     DCALL(ensure_linv(d, 1));
     // X = mu L^-T (I + L^-1 dS L^-T) L^-1 for the checker factor L
-    hdk::gemm<double>(d->st, false, false, false, n, n, n, 1.0, d->Li[1], n, 0, d->S[2], n, 0, 0.0, d->T1, n, 0, 1);
-    hdk::gemm<double>(d->st, false, true, false, n, n, n, 1.0, d->T1, n, 0, d->Li[1], n, 0, 0.0, d->T2, n, 0, 1);
+    hdk::gemm<double>(d->st, false, false, false, n, n, n, 1.0, d->Li[1], n, 0, d->S[2], n, 0, 0.0, d->T1, n, 0, 1, 2);
+    hdk::gemm<double>(d->st, false, true, false, n, n, n, 1.0, d->T1, n, 0, d->Li[1], n, 0, 0.0, d->T2, n, 0, 1, 3);
     hdk::sym_avg(d->st, n, d->T2, 1.0, 1.0, d->T1);
-    hdk::gemm<double>(d->st, true, false, false, n, n, n, 1.0, d->Li[1], n, 0, d->T1, n, 0, 0.0, d->T2, n, 0, 1);
-    hdk::gemm<double>(d->st, false, false, false, n, n, n, 1.0, d->T2, n, 0, d->Li[1], n, 0, 0.0, d->T1, n, 0, 1);
+    hdk::gemm<double>(d->st, true, false, false, n, n, n, 1.0, d->Li[1], n, 0, d->T1, n, 0, 0.0, d->T2, n, 0, 1, 5);
+    hdk::gemm<double>(d->st, false, false, false, n, n, n, 1.0, d->T2, n, 0, d->Li[1], n, 0, 0.0, d->T1, n, 0, 1, 1);
     hdk::sym_avg(d->st, n, d->T1, mu, 0.0, d->X);
     DCALL(check_launch());
     return prof_end(d, HDSDP_PROF_PRIMAL);
@@ -1952,7 +1951,7 @@ hdsdp_retcode hdsdp_dev_adjoint(hdsdp_dev *d, double mu, const double *dLdy, dou
     for (int i = 0; i < m; ++i) dLdb[i] = lam[i] / mu;
     // dLdC = W (sum_i lambda_i A_i) W with W = S^-1 of the dual factor
     DCALL(ensure_linv(d, 0));
-    hdk::gemm<double>(d->st, true, false, false, n, n, n, 1.0, d->Li[0], n, 0, d->Li[0], n, 0, 0.0, d->W, n, 0, 1);
+    hdk::gram_lower(d->st, n, d->Li[0], d->W);
     DCALL(hdsdp_dev_update_buffer(d, 0.0, 1.0, lam.data(), 0.0, 2));
     hdk::mirror_lower<double>(d->st, n, d->S[2], n);
     hdk::gemm<double>(d->st, false, false, false, n, n, n, 1.0, d->W, n, 0, d->S[2], n, 0, 0.0, d->T1, n, 0, 1);

@@ -525,3 +525,60 @@ def test_small_cg_and_lanczos_edges(gpu_lib, oracle, n, m):
     assert rel(gx, ox) < 1e-9
     assert np.all(gt == 0.0) and np.all(ot == 0.0)
     assert rel(gs, os_) < 1e-6
+
+
+# edges of the 32-wide tiles and their slabs of 64 k, full and shorter last pairs of the
+# triangular inverse's levels, and the first size whose S^-1 is formed in its lower half
+@pytest.mark.parametrize("n", [2, 31, 32, 33, 64, 65, 96, 97, 129, 193, 257, 321, 449, 1280, 1281])
+def test_products_on_small_tiles(gpu_lib, n):
+    """S^-1 (through the Schur matrix of off-diagonal entries, which reads both triangles) and the
+    primal recovery X = mu S^-1 (S + dS) S^-1 against numpy.  With condition kappa < 5 of S,
+    the inverse and four products of n terms round to 30 n u kappa (u = 1.1e-16) relative to
+    the largest entry at worst."""
+    rng = np.random.default_rng(n)
+    S, (C, _, _) = _spd_coeffs(n, rng)
+    r, c = np.tril_indices(n)
+    pick = rng.permutation(len(r))[:min(len(r), 40)]
+    r, c, m = r[pick], c[pick], len(pick)
+    one = np.ones(1)
+    d = dt.Dev(gpu_lib, [C] + [dt.Coeff(dt.SPARSE, n, row=[r[k]], col=[c[k]], val=one) for k in range(m)])
+    for which in (0, 1):
+        d.update(1.0, 0.0, np.zeros(m), 0.0, which)
+        assert d.factorize(which) == 1
+    d.schur(0, 0.0)
+    M = d.get_schur()
+    W = np.linalg.inv(S)
+    w = np.where(r == c, 1.0, 2.0)
+    ref = (W[np.ix_(r, r)] * W[np.ix_(c, c)] + W[np.ix_(r, c)] * W[np.ix_(c, r)]) * np.outer(w, w) / 2.0
+    tol = 150.0 * n * 1.1e-16
+    assert np.max(np.abs(M - ref)) <= tol * np.max(np.abs(ref))
+    dy = rng.standard_normal(m)
+    dS = np.zeros((n, n))
+    dS[r, c] = dy
+    dS[c, r] = dy
+    d.primal(0.5, np.zeros(m), dy)
+    X = d.get_primal()
+    d.close()
+    want = 0.5 * (W + W @ dS @ W)
+    assert np.max(np.abs(X - want)) <= tol * np.max(np.abs(want)) * max(1.0, np.linalg.norm(dS, 2))
+    assert np.array_equal(X, X.T)
+
+
+# rank-m updates of few tiles: one part, two, a shorter last part, whole and ragged tiles
+@pytest.mark.parametrize("n,m", [(32, 1000), (33, 2049), (64, 3001), (101, 2050), (130, 5000)])
+def test_rank_one_buffer_on_small_tiles(gpu_lib, n, m):
+    """S = C - sum y_i s_i f_i f_i^T over dense rank-one constraints against numpy: sums of m
+    terms, rounding to m u sum_i |y_i s_i f_i f_i^T| at worst (u = 1.1e-16)."""
+    rng = np.random.default_rng(n + m)
+    _, (C, _, _) = _spd_coeffs(n, rng)
+    cons = [dt.rand_dsr1(rng, n) for _ in range(m)]
+    y = rng.standard_normal(m)
+    d = dt.Dev(gpu_lib, [C] + cons)
+    d.update(1.0, -1.0, y, 0.0, 0)
+    S = d.get_dual()
+    d.close()
+    F = np.array([c.val for c in cons])
+    w = y * np.array([c.sign for c in cons])
+    want = C.dense() - F.T @ (F * w[:, None])
+    bound = np.abs(F).T @ (np.abs(F) * np.abs(w)[:, None])
+    assert np.all(np.abs(S - want) <= 2.0 * m * 1.1e-16 * (bound + np.abs(want)))
