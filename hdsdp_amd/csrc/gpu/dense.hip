@@ -1,9 +1,9 @@
 // dense.hip -- dense linear algebra for the dual slack S and the Schur matrix M
 // on gfx950: MFMA GEMM, blocked Cholesky, recursive triangular inverse, GEMV.
 //
-// GEMM tiles are 64 x 64 per workgroup of four 64-wide waves; each wave owns a
-// 32 x 32 quadrant as 2 x 2 MFMA 16x16 accumulators and the k-dimension is
-// staged through LDS in slabs of 16.  FP64 uses v_mfma_f64_16x16x4_f64, FP32
+// GEMM tiles are 32, 64 or 128 wide per workgroup of four 64-wide waves; each wave owns a
+// quadrant as MFMA 16x16 accumulators and the k-dimension is staged through LDS in
+// slabs.  FP64 uses v_mfma_f64_16x16x4_f64, FP32
 // v_mfma_f32_16x16x4_f32; both take one A and one B element per lane,
 //   A[i][k] at lane i + 16 k,  B[k][j] at lane j + 16 k,
 // and return four accumulator elements per lane in different row orders
@@ -75,117 +75,6 @@ __device__ inline void tile_xy(int lin, int &bx, int &by, int tri = 0) {
     while (x * (x + 1) / 2 > t) --x;
     bx = x;
     by = t - x * (x + 1) / 2;
-}
-
-// One k slab of a 64-wide tile into registers: thread t moves elements t + 256 u of
-// each operand's 64 x 16 slab (zero outside the matrix).
-template <typename T, bool TA, bool TB>
-__device__ inline void tile_fetch(const T *A, int lda, const T *B, int ldb, int M, int N, int K, int i0, int j0,
-                                  int k0, int tid, T (&ra)[4], T (&rb)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int e = tid + 256 * u;
-        int i, k;
-        if (!TA) { i = e & 63; k = e >> 6; } else { k = e & 15; i = e >> 4; }
-        const int gi = i0 + i, gk = k0 + k;
-        T v = 0;
-        if (gi < M && gk < K) v = TA ? A[gk + (long) gi * lda] : A[gi + (long) gk * lda];
-        ra[u] = v;
-        int j, kb;
-        if (!TB) { kb = e & 15; j = e >> 4; } else { j = e & 63; kb = e >> 6; }
-        const int gj = j0 + j, gkb = k0 + kb;
-        T w = 0;
-        if (gj < N && gkb < K) w = TB ? B[gj + (long) gkb * ldb] : B[gkb + (long) gj * ldb];
-        rb[u] = w;
-    }
-}
-
-template <typename T, bool TA, bool TB>
-__device__ inline void tile_stash(T (*As)[TILE + 1], T (*Bs)[TILE + 1], int tid, const T (&ra)[4],
-                                  const T (&rb)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int e = tid + 256 * u;
-        int i, k;
-        if (!TA) { i = e & 63; k = e >> 6; } else { k = e & 15; i = e >> 4; }
-        As[k][i] = ra[u];
-        int j, kb;
-        if (!TB) { kb = e & 15; j = e >> 4; } else { j = e & 63; kb = e >> 6; }
-        Bs[kb][j] = rb[u];
-    }
-}
-
-// 64 x 64 tiles: the C tile (beta != 0) is fetched before the k loop and the k slabs
-// are double-buffered (slab s + 1 loads in flight while slab s is multiplied), so a
-// short-k product such as a rank-64 update does not wait on memory once per slab and
-// again for C.
-template <typename T, bool TA, bool TB, bool LOWER>
-__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, T alpha, const T *A, int lda,
-                                                   long sA, const T *B, int ldb, long sB, T beta,
-                                                   T *C, int ldc, long sC, int tri, int lin) {
-    typedef typename Mfma<T>::acc_t acc_t;
-    int bx, by;
-    tile_xy(lin, bx, by, tri);
-    const int i0 = bx * TILE, j0 = by * TILE;
-    if (LOWER && i0 + TILE - 1 < j0) return;
-    int kLo, kHi;
-    tri_krange(tri, i0, j0, TILE, K, kLo, kHi);
-    A += (long) blockIdx.z * sA;
-    B += (long) blockIdx.z * sB;
-    C += (long) blockIdx.z * sC;
-    __shared__ T As[2][KSTEP][TILE + 1];
-    __shared__ T Bs[2][KSTEP][TILE + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
-    const int lr = lane & 15, lk = lane >> 4;
-    T cin[2][2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = i0 + wi + a * 16 + Mfma<T>::row(lk, r);
-                const int j = j0 + wj + b * 16 + lr;
-                const bool ok = i < M && j < N && (!LOWER || i >= j);
-                cin[a][b][r] = (ok && beta != (T) 0) ? C[i + (long) j * ldc] : (T) 0;
-            }
-    acc_t acc[2][2];
-    for (int a = 0; a < 2; ++a)
-        for (int b = 0; b < 2; ++b) acc[a][b] = (acc_t){0, 0, 0, 0};
-    const int nslab = kHi > kLo ? (kHi - kLo + KSTEP - 1) / KSTEP : 0;
-    if (nslab > 0) {
-        T ra[4], rb[4];
-        tile_fetch<T, TA, TB>(A, lda, B, ldb, M, N, K, i0, j0, kLo, tid, ra, rb);
-        tile_stash<T, TA, TB>(As[0], Bs[0], tid, ra, rb);
-        __syncthreads();
-        for (int sl = 0; sl < nslab; ++sl) {
-            const int cur = sl & 1;
-            const bool more = sl + 1 < nslab;
-            if (more) tile_fetch<T, TA, TB>(A, lda, B, ldb, M, N, K, i0, j0, kLo + (sl + 1) * KSTEP, tid, ra, rb);
-#pragma unroll
-            for (int kk = 0; kk < KSTEP; kk += 4) {
-                T a0 = As[cur][kk + lk][wi + lr], a1 = As[cur][kk + lk][wi + 16 + lr];
-                T b0 = Bs[cur][kk + lk][wj + lr], b1 = Bs[cur][kk + lk][wj + 16 + lr];
-                acc[0][0] = Mfma<T>::op(a0, b0, acc[0][0]);
-                acc[0][1] = Mfma<T>::op(a0, b1, acc[0][1]);
-                acc[1][0] = Mfma<T>::op(a1, b0, acc[1][0]);
-                acc[1][1] = Mfma<T>::op(a1, b1, acc[1][1]);
-            }
-            if (more) tile_stash<T, TA, TB>(As[cur ^ 1], Bs[cur ^ 1], tid, ra, rb);
-            __syncthreads();
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = i0 + wi + a * 16 + Mfma<T>::row(lk, r);
-                const int j = j0 + wj + b * 16 + lr;
-                if (i < M && j < N && (!LOWER || i >= j)) C[i + (long) j * ldc] = alpha * acc[a][b][r] + beta * cin[a][b][r];
-            }
 }
 
 // 128 x 128 tiles for large products: four waves, each a 64 x 64 quadrant as 4 x 4
@@ -425,6 +314,13 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(int M, int N, int K, T al
     }
 }
 
+// 16-byte loads need even leading dimensions, strides and addresses
+template <typename T>
+static bool vec_ok(const T *A, long lda, long sA, const T *B, long ldb, long sB) {
+    return sizeof(T) == 8 && lda % 2 == 0 && ldb % 2 == 0 && sA % 2 == 0 && sB % 2 == 0 &&
+           ((uintptr_t) A % 16) == 0 && ((uintptr_t) B % 16) == 0;
+}
+
 // 128-wide tile launch; batch z multiplies K-wide slices at strides sA, sB (the last
 // one kLast wide when kLast > 0)
 template <typename T>
@@ -434,9 +330,7 @@ static void gemm_big(hipStream_t s, bool transA, bool transB, bool lower, int M,
     const int mt = (M + BT - 1) / BT, nt = (N + BT - 1) / BT;
     const int lin = (lower && mt == nt) ? 1 : 0;
     dim3 bgrid(lin ? mt * (mt + 1) / 2 : mt, lin ? 1 : nt, batch);
-    // 16-byte loads need even leading dimensions, strides and addresses
-    const bool vec = sizeof(T) == 8 && lda % 2 == 0 && ldb % 2 == 0 && strideA % 2 == 0 && strideB % 2 == 0 &&
-                     ((uintptr_t) A % 16) == 0 && ((uintptr_t) B % 16) == 0;
+    const bool vec = vec_ok<T>(A, lda, strideA, B, ldb, strideB);
 #define HDK_GEMM_BIG(ta, tb, lo)                                                                                 \
     if (transA == ta && transB == tb && lower == lo) {                                                           \
         if (vec)                                                                                                 \
@@ -459,129 +353,193 @@ static void gemm_big(hipStream_t s, bool transA, bool transB, bool lower, int M,
 #undef HDK_GEMM_BIG
 }
 
-// 32 x 32 tiles for products that leave CUs idle on 64-wide tiles (the levels of a
+// 64- and 32-wide tiles (TI) of four waves, each a quadrant of F x F MFMA blocks, F = TI / 32,
+// with slabs of 32 or 64 k.
+//
+// 32-wide tiles serve products that leave CUs idle on 64-wide ones (the levels of a
 // triangular inverse, S^-1 of a small block, the k parts of a rank-m update with few
-// tiles).  On 64-wide tiles such a product is bound by the MFMA chain of its few tiles, one
-// wave per SIMD: 0.43 us per 16 k whatever the rest of the chip does; here a tile takes a
-// quarter of it on four times the workgroups, with slabs of 64 k so that a load latency is
-// paid once per 64 k.  MFMA rows are tile columns, so that a wave loads and stores 16
-// consecutive rows.  Each operand is staged in its own order: rows consecutive as [k][48], k
-// consecutive as [row][66], both free of bank conflicts in the fragment reads.  Every
-// output sums its k in ascending order like the other tile widths, so the choice does not change
-// a bit.  The last batch entry may have fewer rows (mLast > 0) and a shorter k (kLast > 0).
-constexpr int TT = 32, TK = 64, TLR = 48, TLK = 66;
+// tiles): on 64-wide tiles such a product is bound by the MFMA chain of its few tiles, 0.43 us
+// per 16 k whatever the rest of the chip does; a 32-wide tile takes a quarter of it on four
+// times the workgroups, and pays a load latency once per 64 k.
+//
+// MFMA rows are tile columns, so that a wave loads and stores 16 consecutive rows.  Each
+// operand is staged in its own order: rows consecutive as [k][TI + 16], k consecutive as
+// [row][slab + 2], both free of bank conflicts in the fragment reads.  The slab sits in LDS
+// once (40 to 50 KB, three workgroups per CU); the next one is in flight in registers
+// while it is multiplied.  Every output sums its k in ascending order whatever the tile, so
+// the choice of one does not change a bit.  The last batch entry may have fewer rows
+// (mLast > 0) and a shorter k (kLast > 0).  PACK: the strictly lower part of a square result
+// goes to C packed by columns and its diagonal to dg (beta = 0).
+template <int TI>
+struct MidTile {
+    static constexpr int TK = (TI == 32) ? 64 : 32, LR = TI + 16, LK = TK + 2, F = TI / 32;
+    static constexpr int PER = TI * TK / 256;  // elements of a slab per thread
+};
 
-template <typename T, bool KC>
-__device__ inline void thin_fetch(const T *X, long ldx, int rows, int K, int r0, int k0, int tid, T (&v)[8]) {
+template <typename T, bool KC, int TI>
+__device__ inline void mid_fetch(const T *X, long ldx, int rows, int K, int r0, int k0, int tid,
+                                 T (&v)[MidTile<TI>::PER]) {
+    constexpr int TK = MidTile<TI>::TK;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        // addresses clamped into the operand; the k beyond K are zeroed in thin_stash
-        const int r = min(r0 + (KC ? (tid >> 6) + 4 * u : (tid & 31)), rows - 1);
-        const int k = min(k0 + (KC ? (tid & 63) : (tid >> 5) + 8 * u), K - 1);
+    for (int u = 0; u < MidTile<TI>::PER; ++u) {
+        // addresses clamped into the operand; the k beyond K are zeroed in mid_stash
+        const int r = min(r0 + (KC ? tid / TK + 256 / TK * u : tid % TI), rows - 1);
+        const int k = min(k0 + (KC ? tid % TK : tid / TI + 256 / TI * u), K - 1);
         v[u] = KC ? X[k + r * ldx] : X[r + k * ldx];
     }
 }
 
-template <typename T, bool KC>
-__device__ inline void thin_stash(T *S, int K, int k0, int tid, const T (&v)[8]) {
+template <typename T, bool KC, int TI>
+__device__ inline void mid_stash(T *S, int K, int k0, int tid, const T (&v)[MidTile<TI>::PER]) {
+    constexpr int TK = MidTile<TI>::TK;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const int r = KC ? (tid >> 6) + 4 * u : (tid & 31), k = KC ? (tid & 63) : (tid >> 5) + 8 * u;
-        S[KC ? r * TLK + k : k * TLR + r] = (k0 + k < K) ? v[u] : (T) 0;
+    for (int u = 0; u < MidTile<TI>::PER; ++u) {
+        const int r = KC ? tid / TK + 256 / TK * u : tid % TI, k = KC ? tid % TK : tid / TI + 256 / TI * u;
+        S[KC ? r * MidTile<TI>::LK + k : k * MidTile<TI>::LR + r] = (k0 + k < K) ? v[u] : (T) 0;
     }
 }
 
-template <typename T, bool TA, bool TB, bool LOWER>
-__global__ __launch_bounds__(256) void gemm_thin_kernel(int M, int N, int K, T alpha, const T *A, int lda, long sA,
-                                                        const T *B, int ldb, long sB, T beta, T *C, int ldc, long sC,
-                                                        int tri, int lin, int mLast, int kLast) {
+template <typename T, bool TA, bool TB, bool LOWER, int TI, int PACK = 0>
+__global__ __launch_bounds__(256) void gemm_mid_kernel(int M, int N, int K, T alpha, const T *A, int lda, long sA,
+                                                       const T *B, int ldb, long sB, T beta, T *C, int ldc, long sC,
+                                                       int tri, int lin, int mLast, int kLast, T *dg = nullptr,
+                                                       long sDg = 0) {
+    typedef MidTile<TI> G;
+    constexpr int F = G::F, TK = G::TK, LR = G::LR, LK = G::LK;
     constexpr bool KCA = TA, KCB = !TB;  // operand consecutive along k
-    __shared__ T As[KCA ? TT * TLK : TK * TLR], Bs[KCB ? TT * TLK : TK * TLR];
+    __shared__ T As[KCA ? TI * LK : TK * LR], Bs[KCB ? TI * LK : TK * LR];
     if (blockIdx.z == gridDim.z - 1) {
         if (mLast > 0) M = mLast;
         if (kLast > 0) K = kLast;
     }
     int bx, by;
     tile_xy(lin, bx, by, tri);
-    const int i0 = bx * TT, j0 = by * TT;
-    if (i0 >= M || j0 >= N || (LOWER && i0 + TT - 1 < j0)) return;
+    const int i0 = bx * TI, j0 = by * TI;
+    if (i0 >= M || j0 >= N || (LOWER && i0 + TI - 1 < j0)) return;
     int kLo, kHi;
-    tri_krange(tri, i0, j0, TT, K, kLo, kHi);
+    tri_krange(tri, i0, j0, TI, K, kLo, kHi);
     A += (long) blockIdx.z * sA;
     B += (long) blockIdx.z * sB;
     C += (long) blockIdx.z * sC;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = (wave & 1) * 16, wj = (wave >> 1) * 16, lr = lane & 15, lk = lane >> 4;
-    const int i = i0 + wi + lr;
-    T cin[4];
+    const int wi = (wave & 1) * (TI / 2), wj = (wave >> 1) * (TI / 2), lr = lane & 15, lk = lane >> 4;
+    typename Mfma<T>::acc_t acc[F][F];
+    T cin[F][F][4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int j = j0 + wj + Mfma<T>::row(lk, r);
-        cin[r] = (beta != (T) 0 && i < M && j < N && (!LOWER || i >= j)) ? C[i + (long) j * ldc] : (T) 0;
-    }
-    typename Mfma<T>::acc_t acc = {0, 0, 0, 0};
-    T ra[8], rb[8];
+    for (int a = 0; a < F; ++a)
+#pragma unroll
+        for (int b = 0; b < F; ++b) {
+            acc[a][b] = (typename Mfma<T>::acc_t){0, 0, 0, 0};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = i0 + wi + 16 * a + lr, j = j0 + wj + 16 * b + Mfma<T>::row(lk, r);
+                cin[a][b][r] = (beta != (T) 0 && i < M && j < N && (!LOWER || i >= j)) ? C[i + (long) j * ldc] : (T) 0;
+            }
+        }
+    T ra[G::PER], rb[G::PER];
     if (kLo < kHi) {
-        thin_fetch<T, KCA>(A, lda, M, K, i0, kLo, tid, ra);
-        thin_fetch<T, KCB>(B, ldb, N, K, j0, kLo, tid, rb);
+        mid_fetch<T, KCA, TI>(A, lda, M, K, i0, kLo, tid, ra);
+        mid_fetch<T, KCB, TI>(B, ldb, N, K, j0, kLo, tid, rb);
     }
     for (int k0 = kLo; k0 < kHi; k0 += TK) {
-        thin_stash<T, KCA>(As, K, k0, tid, ra);
-        thin_stash<T, KCB>(Bs, K, k0, tid, rb);
+        mid_stash<T, KCA, TI>(As, K, k0, tid, ra);
+        mid_stash<T, KCB, TI>(Bs, K, k0, tid, rb);
         __syncthreads();
         if (k0 + TK < kHi) {
-            thin_fetch<T, KCA>(A, lda, M, K, i0, k0 + TK, tid, ra);
-            thin_fetch<T, KCB>(B, ldb, N, K, j0, k0 + TK, tid, rb);
+            mid_fetch<T, KCA, TI>(A, lda, M, K, i0, k0 + TK, tid, ra);
+            mid_fetch<T, KCB, TI>(B, ldb, N, K, j0, k0 + TK, tid, rb);
         }
 #pragma unroll
         for (int kk = 0; kk < TK; kk += 4) {
-            const T a = KCA ? As[(wi + lr) * TLK + kk + lk] : As[(kk + lk) * TLR + wi + lr];
-            const T b = KCB ? Bs[(wj + lr) * TLK + kk + lk] : Bs[(kk + lk) * TLR + wj + lr];
-            acc = Mfma<T>::op(b, a, acc);
+            T af[F], bf[F];
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const int i = wi + 16 * f + lr, j = wj + 16 * f + lr, k = kk + lk;
+                af[f] = As[KCA ? i * LK + k : k * LR + i];
+                bf[f] = Bs[KCB ? j * LK + k : k * LR + j];
+            }
+#pragma unroll
+            for (int a = 0; a < F; ++a)
+#pragma unroll
+                for (int b = 0; b < F; ++b) acc[a][b] = Mfma<T>::op(bf[b], af[a], acc[a][b]);
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int j = j0 + wj + Mfma<T>::row(lk, r);
-        if (i < M && j < N && (!LOWER || i >= j)) C[i + (long) j * ldc] = alpha * acc[r] + beta * cin[r];
-    }
+    for (int a = 0; a < F; ++a)
+#pragma unroll
+        for (int b = 0; b < F; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = i0 + wi + 16 * a + lr, j = j0 + wj + 16 * b + Mfma<T>::row(lk, r);
+                if (i >= M || j >= N || (LOWER && i < j)) continue;
+                if (PACK) {
+                    if (i == j) dg[blockIdx.z * sDg + i] = alpha * acc[a][b][r];
+                    else C[(long) j * N - (long) j * (j + 1) / 2 + (i - j - 1)] = alpha * acc[a][b][r];
+                } else {
+                    C[i + (long) j * ldc] = alpha * acc[a][b][r] + beta * cin[a][b][r];
+                }
+            }
 }
 
-template <typename T>
-static void gemm_thin(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int K, T alpha, const T *A,
-                      int lda, long strideA, const T *B, int ldb, long strideB, T beta, T *C, int ldc, long strideC,
-                      int batch, int tri, int mLast = 0, int kLast = 0) {
-    const int mt = (M + TT - 1) / TT, nt = (N + TT - 1) / TT;
+template <int TI, typename T>
+static void gemm_mid(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int K, T alpha, const T *A,
+                     int lda, long strideA, const T *B, int ldb, long strideB, T beta, T *C, int ldc, long strideC,
+                     int batch, int tri, int mLast = 0, int kLast = 0) {
+    const int mt = (M + TI - 1) / TI, nt = (N + TI - 1) / TI;
     const int lin = (lower && mt == nt) ? 1 : 0;
     const dim3 grid(lin ? mt * (mt + 1) / 2 : mt, lin ? 1 : nt, batch);
-#define HDK_GEMM_THIN(ta, tb, lo)                                                                               \
-    if (transA == ta && transB == tb && lower == lo) {                                                          \
-        gemm_thin_kernel<T, ta, tb, lo><<<grid, 256, 0, s>>>(M, N, K, alpha, A, lda, strideA, B, ldb, strideB,  \
-                                                             beta, C, ldc, strideC, tri, lin, mLast, kLast);    \
-        return;                                                                                                 \
+#define HDK_GEMM_MID(ta, tb, lo)                                                                               \
+    if (transA == ta && transB == tb && lower == lo) {                                                         \
+        gemm_mid_kernel<T, ta, tb, lo, TI><<<grid, 256, 0, s>>>(M, N, K, alpha, A, lda, strideA, B, ldb,       \
+                                                                strideB, beta, C, ldc, strideC, tri, lin,      \
+                                                                mLast, kLast);                                 \
+        return;                                                                                                \
     }
-    HDK_GEMM_THIN(false, false, false)
-    HDK_GEMM_THIN(false, true, false)
-    HDK_GEMM_THIN(true, false, false)
-    HDK_GEMM_THIN(true, true, false)
-    HDK_GEMM_THIN(false, false, true)
-    HDK_GEMM_THIN(false, true, true)
-    HDK_GEMM_THIN(true, false, true)
-    HDK_GEMM_THIN(true, true, true)
-#undef HDK_GEMM_THIN
+    HDK_GEMM_MID(false, false, false)
+    HDK_GEMM_MID(false, true, false)
+    HDK_GEMM_MID(true, false, false)
+    HDK_GEMM_MID(true, true, false)
+    HDK_GEMM_MID(false, false, true)
+    HDK_GEMM_MID(false, true, true)
+    HDK_GEMM_MID(true, false, true)
+    HDK_GEMM_MID(true, true, true)
+#undef HDK_GEMM_MID
 }
 
-// Up to THIN_TILES tiles of 64 x 64 the 32-wide tiles are faster or equal; beyond, both fill
-// the chip and the wider tile moves half the operands.  Measured, us, 64-wide against
-// 32-wide: 200^3 17.6 and 8.3, 512^3 36.6 and 14.4, 1000^3 (256 tiles) 69.5 and 64.1,
-// 1300^3 (441) 125 and 132; 16 products of 256^3 (256 tiles) 21.9 and 18.6, 32 (512) 31.3
-// both; S^-1 of n = 500 34.5 and 13.2; a lower rank-3001 update at n = 301 in two k parts 394 on
-// 128-wide tiles and 37.
-constexpr long THIN_TILES = 400;
-static bool use_thin(int M, int N, int K, bool lower, int batch) {
-    const long tiles = (long) ((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE) * batch / (lower ? 2 : 1);
-    return K >= 1 && tiles <= THIN_TILES;
+// Tile width of a product: the least modelled time
+//   k per tile x time per k and tile x tiles per CU (rounded up)
+// over the three widths.  A CU's workgroups share its matrix cores, so the time of a width
+// grows with the tiles per CU and not below what its latencies take alone (1.3, 1.7, 2.2
+// tiles' worth); a tile of a triangular product walks half its k and half a tile on average;
+// prologue and epilogue cost as much as 96 and 32 k; the bounds-checked loads of ragged
+// 128-wide tiles cost 0.8 of a tile more, unaligned operands a fifth.  Measured on MI355X,
+// us at 32, 64 and 128: 500^3 14.6, 34.5, 109; 1000^3 67, 67, 218; 1300^3 137, 127, 262;
+// 4000^3 2967, 2473, 2231; lower 4000^3 1480, 1218, 1670; lower 8000^2 x 768 1177, 951, 863;
+// 8000 x 768 x 768 lower 241, 208, 237; 450 triangular products of n = 300 540, 433, 709, of
+// n = 200 211, 238, 334; 16 lower k parts 450^2 x 2800 268, 338, 484.
+static int pick_tile(int M, int N, int K, bool lower, int batch, int tri, bool vec) {
+    const int width[3] = {32, 64, 128};
+    const double perK[3] = {0.0137, 0.041, 0.125}, alone[3] = {2.2, 1.7, 1.3}, extra[3] = {32, 32, 96};
+    int best = 64;
+    double tBest = 1e300;
+    for (int v = 0; v < 3; ++v) {
+        const int t = width[v];
+        const long mt = (M + t - 1) / t, nt = (N + t - 1) / t, c = std::min(mt, nt);
+        const long tiles = (lower ? mt * nt - c * (c - 1) / 2 : mt * nt) * batch;
+        const double depth = std::max(alone[v], (double) ((tiles + 255) / 256));
+        const double k = (tri == 0) ? K : (tri == 4) ? (K + t) / 3.0 : std::min<double>(K, (K + t) / 2.0);
+        double time = perK[v] * depth * (k + extra[v]);
+        if (t == 128) {
+            const double ragged = 1.0 - (double) (M / t) * (N / t) / (double) (mt * nt);
+            time *= (1.0 + 0.8 * ragged) * (vec ? 1.0 : 1.2);
+        }
+        if (time < tBest) {
+            tBest = time;
+            best = t;
+        }
+    }
+    return best;
 }
 
 template <typename T>
@@ -589,37 +547,16 @@ void gemm(hipStream_t s, bool transA, bool transB, bool lower, int M, int N, int
           int lda, long strideA, const T *B, int ldb, long strideB, T beta, T *C, int ldc, long strideC,
           int batch, int tri) {
     if (M <= 0 || N <= 0 || batch <= 0) return;
-    const long bigTiles = (long) ((M + BT - 1) / BT) * ((N + BT - 1) / BT) * batch / (lower ? 2 : 1);
-    // the 128-wide tiles pay off only when the k loop is long enough to hide their
-    // prologue and epilogue (measured: rank-64 updates run faster on 64-wide tiles)
-    if (bigTiles >= 192 && K >= 256) {
+    const int t = pick_tile(M, N, K, lower, batch, tri, vec_ok<T>(A, lda, strideA, B, ldb, strideB));
+    if (t == 128)
         gemm_big<T>(s, transA, transB, lower, M, N, K, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
                     strideC, batch, tri, 0);
-        return;
-    }
-    if (use_thin(M, N, K, lower, batch)) {
-        gemm_thin<T>(s, transA, transB, lower, M, N, K, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
-                     strideC, batch, tri);
-        return;
-    }
-    const int mt = (M + TILE - 1) / TILE, nt = (N + TILE - 1) / TILE;
-    const int lin = (lower && mt == nt) ? 1 : 0;
-    dim3 grid(lin ? mt * (mt + 1) / 2 : mt, lin ? 1 : nt, batch);
-#define HDK_GEMM_CASE(ta, tb, lo)                                                                    \
-    if (transA == ta && transB == tb && lower == lo) {                                               \
-        gemm_kernel<T, ta, tb, lo><<<grid, 256, 0, s>>>(M, N, K, alpha, A, lda, strideA, B, ldb, strideB, \
-                                                        beta, C, ldc, strideC, tri, lin);           \
-        return;                                                                                      \
-    }
-    HDK_GEMM_CASE(false, false, false)
-    HDK_GEMM_CASE(false, true, false)
-    HDK_GEMM_CASE(true, false, false)
-    HDK_GEMM_CASE(true, true, false)
-    HDK_GEMM_CASE(false, false, true)
-    HDK_GEMM_CASE(false, true, true)
-    HDK_GEMM_CASE(true, false, true)
-    HDK_GEMM_CASE(true, true, true)
-#undef HDK_GEMM_CASE
+    else if (t == 64)
+        gemm_mid<64, T>(s, transA, transB, lower, M, N, K, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
+                        strideC, batch, tri);
+    else
+        gemm_mid<32, T>(s, transA, transB, lower, M, N, K, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
+                        strideC, batch, tri);
 }
 
 template void gemm<double>(hipStream_t, bool, bool, bool, int, int, int, double, const double *, int, long,
@@ -628,10 +565,10 @@ template void gemm<float>(hipStream_t, bool, bool, bool, int, int, int, float, c
                           const float *, int, long, float, float *, int, long, int, int);
 
 // W = Li^T Li for a lower-triangular Li (n x n, zeros above): entry (i, j) sums k >= max(i, j)
-// only, n^3 / 3 multiply-adds, and is symmetric to the bit, so from THIN_TILES tiles on the
+// only, n^3 / 3 multiply-adds, and is symmetric to the bit, so beyond the 32-wide tiles the
 // lower half is formed and mirrored (n^3 / 6).  n = 2000: 83 us, the full product 366.
 void gram_lower(hipStream_t s, int n, const double *Li, double *W) {
-    const bool half = !use_thin(n, n, n, false, 1);
+    const bool half = pick_tile(n, n, n, false, 1, 4, n % 2 == 0) > 32;
     gemm<double>(s, true, false, half, n, n, n, 1.0, Li, n, 0, Li, n, 0, 0.0, W, n, 0, 1, 4);
     if (half) mirror_lower<double>(s, n, W, n);
 }
@@ -649,26 +586,26 @@ void gram_panels(hipStream_t s, int r, int kc, int kLast, int parts, double alph
 // C_z = A_z B_z^T for z < batch, lower triangle, packed (PACK above); tri as in gemm
 void gemm_nt_packed(hipStream_t s, int rows, int n, const double *A, int lda, long sA, const double *B, int ldb,
                     long sB, double *off, long K1, long slab, double *dg, long sDg, int batch, int tri) {
-    const int nt = (rows + BT - 1) / BT;
+    const bool vec = vec_ok<double>(A, lda, sA, B, ldb, sB);
+    const int t = (slab > 0) ? 128 : pick_tile(n, n, n, true, batch, tri, vec);
+    if (t < 128) rows = n;
+    const int nt = (rows + t - 1) / t, K = std::min(rows, (n + KSTEP - 1) / KSTEP * KSTEP);
     const dim3 grid(nt * (nt + 1) / 2, 1, batch);
-    const bool vec = lda % 2 == 0 && ldb % 2 == 0 && sA % 2 == 0 && sB % 2 == 0 && ((uintptr_t) A % 16) == 0 &&
-                     ((uintptr_t) B % 16) == 0;
-    const int K = std::min(rows, (n + KSTEP - 1) / KSTEP * KSTEP);
     if (slab > 0)
         gemm_big_kernel<double, false, true, true, true, 2><<<grid, 256, 0, s>>>(
             rows, rows, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, 0, tri, 1, 0, dg, sDg, slab);
+    else if (t == 32)
+        gemm_mid_kernel<double, false, true, true, 32, 1><<<grid, 256, 0, s>>>(
+            n, n, n, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, K1, tri, 1, 0, 0, dg, sDg);
+    else if (t == 64)
+        gemm_mid_kernel<double, false, true, true, 64, 1><<<grid, 256, 0, s>>>(
+            n, n, n, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, K1, tri, 1, 0, 0, dg, sDg);
     else if (vec)
         gemm_big_kernel<double, false, true, true, true, 1><<<grid, 256, 0, s>>>(
             rows, rows, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, K1, tri, 1, 0, dg, sDg);
     else
         gemm_big_kernel<double, false, true, true, false, 1><<<grid, 256, 0, s>>>(
             rows, rows, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, K1, tri, 1, 0, dg, sDg);
-}
-
-// whether a lower n x n product of this batch and depth runs on 128-wide tiles
-bool gemm_lower_is_big(int n, int K, int batch) {
-    const long t = (n + BT - 1) / BT;
-    return t * t * batch / 2 >= 192 && K >= 256;
 }
 
 // ---- split-K ---------------------------------------------------------------------
@@ -741,12 +678,16 @@ void gemm_splitk(hipStream_t s, bool transA, bool transB, bool lower, int M, int
     const int parts = (K + kc - 1) / kc;
     const int kLast = K - (parts - 1) * kc;
     const long sA = transA ? kc : (long) kc * lda, sB = transB ? (long) kc * ldb : kc;
-    if (use_thin(M, N, kc, lower, parts))
-        gemm_thin<T>(s, transA, transB, lower, M, N, kc, (T) 1, A, lda, sA, B, ldb, sB, (T) 0, work, M, (long) mn,
-                     parts, 0, 0, kLast);
-    else
+    const int t = pick_tile(M, N, kc, lower, parts, 0, vec_ok<T>(A, lda, sA, B, ldb, sB));
+    if (t == 128)
         gemm_big<T>(s, transA, transB, lower, M, N, kc, (T) 1, A, lda, sA, B, ldb, sB, (T) 0, work, M, (long) mn,
                     parts, 0, kLast);
+    else if (t == 64)
+        gemm_mid<64, T>(s, transA, transB, lower, M, N, kc, (T) 1, A, lda, sA, B, ldb, sB, (T) 0, work, M, (long) mn,
+                        parts, 0, 0, kLast);
+    else
+        gemm_mid<32, T>(s, transA, transB, lower, M, N, kc, (T) 1, A, lda, sA, B, ldb, sB, (T) 0, work, M, (long) mn,
+                        parts, 0, 0, kLast);
     splitk_reduce_kernel<T><<<4096, 256, 0, s>>>(M, N, parts, alpha, work, beta, C, ldc, lower ? 1 : 0);
 }
 
@@ -767,9 +708,9 @@ __global__ void place_diag_kernel(int n, int span, const double *Dinv, T *Linv, 
 }
 
 // inv([[A, 0], [B, C]]) = [[A^-1, 0], [-C^-1 B A^-1, C^-1]], applied level by level
-// with every pair of one level batched into two GEMMs.  On the 32-wide tiles a shorter last
-// pair is in the same two launches; n = 500 takes 40 us (129 on 64-wide tiles with launches
-// of its own for that pair), n = 2000 172 (442).
+// with every pair of one level batched into two GEMMs.  Below the 128-wide tiles a
+// shorter last pair is in the same two launches; n = 500 takes 40 us (129 on 64-wide tiles
+// with launches of its own for that pair), n = 2000 172 (442).
 template <typename T>
 void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work, int span) {
     if (span <= 0 || span > n) span = n;
@@ -779,13 +720,15 @@ void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Lin
         long strideL = 2L * sz * (ldl + 1), strideI = 2L * sz * (ldi + 1), strideW = (long) sz * sz;
         const int o = npair * 2 * sz, sc = std::max(0, n - o - sz);  // rows of a last, shorter pair
         // W = L21 Linv11 (Linv11 lower), then Linv21 = -Linv22 W (Linv22 lower)
-        if (use_thin(sz, sz, sz, false, npair + 1)) {
-            const int cnt = npair + (sc > 0 ? 1 : 0);
-            if (cnt == 0) continue;
-            gemm_thin<T>(s, false, false, false, sz, sz, sz, (T) 1, L + sz, ldl, strideL, Linv, ldi, strideI, (T) 0,
-                         work, sz, strideW, cnt, 1, sc, 0);
-            gemm_thin<T>(s, false, false, false, sz, sz, sz, (T) -1, Linv + (long) sz * (ldi + 1), ldi, strideI, work,
-                         sz, strideW, (T) 0, Linv + sz, ldi, strideI, cnt, 2, sc, sc);
+        const int cnt = npair + (sc > 0 ? 1 : 0);
+        if (cnt == 0) continue;
+        const int t = pick_tile(sz, sz, sz, false, cnt, 1, false);
+        if (t < 128) {
+            const auto mid = (t == 32) ? gemm_mid<32, T> : gemm_mid<64, T>;
+            mid(s, false, false, false, sz, sz, sz, (T) 1, L + sz, ldl, strideL, Linv, ldi, strideI, (T) 0, work, sz,
+                strideW, cnt, 1, sc, 0);
+            mid(s, false, false, false, sz, sz, sz, (T) -1, Linv + (long) sz * (ldi + 1), ldi, strideI, work, sz,
+                strideW, (T) 0, Linv + sz, ldi, strideI, cnt, 2, sc, sc);
             continue;
         }
         if (npair > 0) {

@@ -50,8 +50,7 @@ __device__ inline float wave_tree_sum(float v) {
     return v;
 }
 
-constexpr int TILE = 64;   // GEMM output tile (rows and columns)
-constexpr int KSTEP = 16;  // GEMM k-slab staged through LDS
+constexpr int KSTEP = 16;  // k slab of the 128-wide GEMM tiles, granularity of skipped k ranges
 constexpr int NB = 64;     // Cholesky / triangular-inverse block
 
 // C = alpha * op(A) * op(B) + beta * C over `batch` problems (column-major).
@@ -82,15 +81,12 @@ void gemm_splitk(hipStream_t s, bool transA, bool transB, bool lower, int M, int
 // 16 p + k % 16, p up to whole tiles of 128.
 void gram_panels(hipStream_t s, int r, int kc, int kLast, int parts, double alpha, const double *X, long slab,
                  double *P);
-// A_z B_z^T (z < batch) on 128-wide tiles, operands of `rows` >= n rows: of the first n rows
+// A_z B_z^T (z < batch), operands of `rows` >= n rows: of the first n rows
 // and columns the strictly lower part, packed by columns, and the diagonal, into dg + z sDg.
 // slab = 0: packed entries into off + z K1; slab > 0: entry e into off[(e / 16) slab + 16 z +
 // e % 16] (operands 16-byte aligned, even ld, whole tiles of rows).  tri as in gemm.
 void gemm_nt_packed(hipStream_t s, int rows, int n, const double *A, int lda, long sA, const double *B, int ldb,
                     long sB, double *off, long K1, long slab, double *dg, long sDg, int batch, int tri);
-// whether gemm runs a lower n x n product of this depth and batch on 128-wide tiles
-bool gemm_lower_is_big(int n, int K, int batch);
-
 // C = alpha * X^T Y + beta * C from bf16 split products on the matrix cores: each FP32
 // operand split into `terms` bf16 terms (2: three products, ~16 bits; 3: six products,
 // ~24 bits, FP32-equivalent), FP32 accumulation flushed into FP64 every 256 k.

@@ -716,13 +716,7 @@ void dense_gram(hdsdp_dev *d, const double *Li) {
         const double *A = half ? d->Ubuf : Li, *B = half ? Li : d->Ubuf;
         const long sA = half ? nl : 0, sB = half ? 0 : nl;
         const int tri = half ? 3 : 2;
-        if (slab > 0 || hdk::gemm_lower_is_big(n, n, cnt)) {
-            hdk::gemm_nt_packed(d->st, rows, n, A, ld, sA, B, ld, sB, off, K1, slab, dg, ld, cnt, tri);
-        } else {
-            hdk::gemm<double>(d->st, false, true, true, n, n, n, 1.0, A, ld, sA, B, ld, sB, 0.0, d->Dbuf, ld, nl, cnt,
-                              tri);
-            hdk::pack_lower<double>(d->st, n, cnt, d->Dbuf, ld, nl, off, K1, dg, ld);
-        }
+        hdk::gemm_nt_packed(d->st, rows, n, A, ld, sA, B, ld, sB, off, K1, slab, dg, ld, cnt, tri);
     }
     const long kc = d->gramChunk, rr = (long) r * r;
     const int parts = (int) ((K1 + kc - 1) / kc);

@@ -446,7 +446,6 @@ void pack_lower(hipStream_t s, int n, int cnt, const T *Tin, long ldt, long stri
     pack_lower_kernel<T><<<dim3((unsigned) blocks, cnt), 256, 0, s>>>(n, Tin, ldt, strideIn, off, K1, dg, ldg);
 }
 
-template void pack_lower<double>(hipStream_t, int, int, const double *, long, long, double *, long, double *, long);
 template void pack_lower<float>(hipStream_t, int, int, const float *, long, long, float *, long, float *, long);
 
 __global__ void add_diag_delta_kernel(int r, const int *con, const double *cur, const double *ref, double *M,

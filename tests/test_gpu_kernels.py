@@ -582,3 +582,10 @@ def test_rank_one_buffer_on_small_tiles(gpu_lib, n, m):
     want = C.dense() - F.T @ (F * w[:, None])
     bound = np.abs(F).T @ (np.abs(F) * np.abs(w)[:, None])
     assert np.all(np.abs(S - want) <= 2.0 * m * 1.1e-16 * (bound + np.abs(want)))
+
+
+# the T_p of small blocks, stored packed by 32- and 64-wide tiles: one tile, ragged tiles, many
+@pytest.mark.parametrize("n,m", [(2, 3), (31, 2), (33, 40), (65, 70), (130, 200), (257, 90), (300, 450)])
+def test_dense_gram_packed_tiles(gpu_lib, n, m):
+    """The dense Gram build as above (same bounds) at the edges of the narrower tiles."""
+    test_dense_gram_build(gpu_lib, n, m)
