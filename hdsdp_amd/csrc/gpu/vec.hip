@@ -7,6 +7,8 @@
 // the host reads back once per step.
 #include "vec.h"
 
+#include <type_traits>
+
 namespace hdk {
 
 // Sum over a workgroup of 1024 threads, in every thread: each wave's tree sum, then the
@@ -227,45 +229,73 @@ void cgj_half(hipStream_t s, int m, const double *z, const double *r, const doub
                                              const_cast<double *>(p), sc, nullptr);
 }
 
-// y = M p (coldot's columns, tri 0) by the 16 waves of one workgroup: a wave takes four
-// columns at a time, each summed in coldot's order; NU = rows per lane
-template <int NU>
-__device__ inline void small_symv(int m, const double *__restrict__ M, long ldm, const double *p, double *y) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    double v[NU];
-#pragma unroll
-    for (int u = 0; u < NU; ++u) v[u] = (u < NU - 1 || lane + 64 * u < m) ? p[lane + 64 * u] : 0.0;
-    for (int j0 = 4 * w; j0 < m; j0 += 64) {
-        double a[4][NU], s[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const double *col = M + (long) min(j0 + c, m - 1) * ldm + lane;
-#pragma unroll
-            for (int u = 0; u < NU; ++u) a[c][u] = (u < NU - 1 || lane + 64 * u < m) ? col[64 * u] : 0.0;
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            s[c] = 0.0;
-#pragma unroll
-            for (int u = 0; u < NU; ++u) s[c] += a[c][u] * v[u];
-            s[c] = wave_tree_sum(s[c]);
-            if (lane == 0 && j0 + c < m) y[j0 + c] = s[c];
-        }
+// Workgroups of eight waves that keep small matrices on the CU: wave w holds the columns
+// 4 (w + 8 q) + c, c < 4, q < 2 NU, of a matrix of at most 64 NU rows, lane l the rows l,
+// l + 64, ... of each.
+
+// Sum over a workgroup whose first four waves hold the values, in every thread: each wave's
+// tree sum, then the four in order, block_sum's result (its other waves add zeros).
+template <int B>
+__device__ inline double block_sum4(double v, double *red) {
+    if (threadIdx.x < 256) {
+        v = wave_tree_sum(v);
+        if ((threadIdx.x & 63) == 0) red[4 * B + (threadIdx.x >> 6)] = v;
     }
     __syncthreads();
+    double total = 0.0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) total += red[4 * B + w];
+    return total;
 }
 
-// One workgroup, every vector in LDS, M from L2.  One CU reads it at about 70 GB/s: an
-// iteration takes 8 us at m = 200 (M 320 KB) and 15 at m = 368, where the two launches of
-// the queued form cost the host 10; hence CGS_MAX.  Statements and reduction orders of
-// cgj_iter.
+// One workgroup: M in registers (and, of a matrix of more than 192 rows, the last quarter of
+// its columns in LDS), every vector in LDS.  An iteration reads nothing from memory and takes
+// 2.9 us at m = 243; with M from L2 in every iteration, at 60 GB/s to the one CU, it took 8.
+// CGS_MAX is what a CU holds.  Statements and reduction orders of cgj_iter.
 template <int NU>
-__global__ __launch_bounds__(1024) void cg_small_kernel(int m, const double *M, long ldm, const double *rhs,
-                                                        const double *jacG, double relTol, double absTol, int maxIter,
-                                                        int restart, double *crhs, double *xG, double *xHost,
-                                                        double *report) {
-    __shared__ double red[32];
+__global__ __launch_bounds__(512, 2) void cg_small_kernel(int m, const double *M, long ldm, const double *rhs,
+                                                          const double *jacG, double relTol, double absTol, int maxIter,
+                                                          int restart, double *crhs, double *xG, double *xHost,
+                                                          double *report) {
+    constexpr int Q = 2 * NU, QR = (NU == 4) ? 6 : Q;  // column groups of a wave, those in registers
+    __shared__ double red[8];
     __shared__ double b[CGS_MAX], jac[CGS_MAX], x[CGS_MAX], r[CGS_MAX], z[CGS_MAX], p[CGS_MAX], Mp[CGS_MAX];
+    __shared__ double Ml[(Q > QR) ? 8 * (Q - QR) * 4 * 64 * NU : 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double Mr[QR][4][NU];
+    double *mine = Ml + (Q > QR ? wave * (Q - QR) * 4 * 64 * NU + lane : 0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int u = 0; u < NU; ++u) {
+                const int j = 4 * (wave + 8 * q) + c, i = lane + 64 * u;
+                const double v = (j < m && i < m) ? M[i + j * ldm] : 0.0;
+                if (q < QR) Mr[q < QR ? q : 0][c][u] = v;
+                else mine[((q - QR) * 4 + c) * 64 * NU + 64 * u] = v;
+            }
+    // y = M p, each column summed in coldot's order
+    auto symv = [&](const double *in, double *out) {
+        double v[NU];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) v[u] = (lane + 64 * u < m) ? in[lane + 64 * u] : 0.0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            double s[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                s[c] = 0.0;
+#pragma unroll
+                for (int u = 0; u < NU; ++u)
+                    s[c] += ((q < QR) ? Mr[q < QR ? q : 0][c][u] : mine[((q - QR) * 4 + c) * 64 * NU + 64 * u]) * v[u];
+            }
+            const double t = wave_tree_sum4(s[0], s[1], s[2], s[3]);
+            const int j = 4 * (wave + 8 * q) + tree_sum4_slot(lane);
+            if ((lane & 15) == 0 && j < m) out[j] = t;
+        }
+        __syncthreads();
+    };
     const int tid = threadIdx.x;
     double acc = 0.0;
     if (tid < m) {
@@ -279,24 +309,24 @@ __global__ __launch_bounds__(1024) void cg_small_kernel(int m, const double *M, 
         p[tid] = v / q;
         acc = 0.0 + v * v;
     }
-    const double bnorm = sqrt(block_sum<0>(acc, red));
+    const double bnorm = sqrt(block_sum4<0>(acc, red));
     const double tol = fmax(fmin(absTol, bnorm * relTol), 0.1 * absTol);
     double nrm = bnorm;
     int stop = (nrm < tol) ? CG_TINY : CG_RUNNING, iter = 0;
     if (stop == CG_RUNNING) {
-        small_symv<NU>(m, M, ldm, p, Mp);
+        symv(p, Mp);
         for (; iter < maxIter; ++iter) {
             double a = 0.0, c = 0.0;
             if (tid < m) {
                 a = 0.0 + z[tid] * r[tid];
                 c = 0.0 + p[tid] * Mp[tid];
             }
-            const double rz = block_sum<1>(a, red);
-            const double alpha = rz / block_sum<0>(c, red);
+            const double rz = block_sum4<1>(a, red);
+            const double alpha = rz / block_sum4<0>(c, red);
             if (iter % restart == 5) {
                 if (tid < m) x[tid] += alpha * p[tid];
                 __syncthreads();
-                small_symv<NU>(m, M, ldm, x, Mp);
+                symv(x, Mp);
                 if (tid < m) {
                     const double v = b[tid] - Mp[tid], t = v / jac[tid];
                     r[tid] = v;
@@ -304,7 +334,7 @@ __global__ __launch_bounds__(1024) void cg_small_kernel(int m, const double *M, 
                     p[tid] = t;
                 }
                 __syncthreads();
-                small_symv<NU>(m, M, ldm, p, Mp);
+                symv(p, Mp);
                 continue;
             }
             a = 0.0;
@@ -315,19 +345,19 @@ __global__ __launch_bounds__(1024) void cg_small_kernel(int m, const double *M, 
                 z[tid] = t;
                 a = 0.0 + v * t;
             }
-            const double beta = block_sum<1>(a, red) / rz;
+            const double beta = block_sum4<1>(a, red) / rz;
             c = 0.0;
             if (tid < m) {
                 p[tid] = z[tid] + beta * p[tid];
                 c = 0.0 + r[tid] * r[tid];
             }
-            nrm = sqrt(block_sum<0>(c, red));
+            nrm = sqrt(block_sum4<0>(c, red));
             stop = (nrm != nrm)                          ? CG_NAN
                    : (iter > 20 && nrm > 0.01 * bnorm) ? CG_STALLED
                    : (nrm < tol)                         ? CG_CONVERGED
                                                          : CG_RUNNING;
             if (stop != CG_RUNNING) break;
-            small_symv<NU>(m, M, ldm, p, Mp);
+            symv(p, Mp);
         }
     }
     if (stop != CG_TINY && tid < m) {
@@ -347,7 +377,7 @@ void cg_small(hipStream_t s, int m, const double *M, long ldm, const double *rhs
               double absTol, int maxIter, int restart, double *crhs, double *x, double *xHost, double *report) {
 #define HDK_CGS(nu)                                                                                              \
     case nu:                                                                                                     \
-        cg_small_kernel<nu><<<1, 1024, 0, s>>>(m, M, ldm, rhs, jac, relTol, absTol, maxIter, restart, crhs, x,   \
+        cg_small_kernel<nu><<<1, 512, 0, s>>>(m, M, ldm, rhs, jac, relTol, absTol, maxIter, restart, crhs, x,   \
                                                xHost, report);                                                   \
         break;
     switch ((m + 63) / 64) {
@@ -445,9 +475,10 @@ __device__ inline void small_coldot(int n, const double *__restrict__ A, const d
 #pragma unroll
             for (int u = 0; u < NU; ++u)
                 s[c] += a[c][u] * ((lo + lane + 64 * u < hi) ? x[lo + lane + 64 * u] : 0.0);
-            s[c] = wave_tree_sum(s[c]);
-            if (lane == 0 && j0 + c < n) y[j0 + c] = s[c];
         }
+        const double q = wave_tree_sum4(s[0], s[1], s[2], s[3]);
+        const int j = j0 + tree_sum4_slot(lane);
+        if ((lane & 15) == 0 && j < n) y[j] = q;
     }
     __syncthreads();
 }
@@ -464,8 +495,9 @@ __device__ inline void small_op(int n, const double *Li, const double *LiT, cons
 }
 
 // A Lanczos step of a small block is bound by its four launches (three products, the
-// step): about 18 us of host time at any n.  In one workgroup it takes the two triangles
-// and D at one CU's rate from L2: 6 us at n = 50, 12 at n = 121, 22 at n = 200; hence LZS_MAX.
+// step): about 18 us of host time at any n.  In one workgroup, with the two triangles and D
+// from L2 at one CU's rate, it takes 12 us at n = 128, 15 at 160 and 22 at 200, where the
+// launches cost less; hence LZS_MAX.
 template <int NU>
 __global__ __launch_bounds__(1024) void lz_small_steps_kernel(int n, int k0, int k1, const double *x0,
                                                               const double *pert, const double *Li, const double *LiT,
@@ -512,6 +544,116 @@ __global__ __launch_bounds__(1024) void lz_small_steps_kernel(int n, int k0, int
             c = 0.0 + q * q;
         }
         const double nrm = sqrt(block_sum<0>(c, red));
+        const double inv = (nrm > 0.0) ? 1.0 / nrm : 0.0;
+        vm = vk;
+        prev = (nrm > 0.0) ? nrm : 0.0;
+        if (i < n) {
+            const double u = (nrm > 0.0) ? q * inv : 0.0;
+            v[i] = u;
+            V[i + (long) (k + 1) * n] = u;
+        }
+        if (i == 0) {
+            H[(k + 1) + k * ldh] = prev;
+            hist[2 * k] = -alp;
+            hist[2 * k + 1] = nrm;
+        }
+        __syncthreads();
+    }
+}
+
+// The same with L^-1, D and L^-T in the registers of eight waves (n <= 64 NU <= 128): a step
+// reads nothing from memory.  n = 121: 4 us per step, 12 with the matrices from L2; n = 50: 2.5
+// and 6.
+template <int NU>
+__global__ __launch_bounds__(512, 2) void lz_resident_steps_kernel(int n, int k0, int k1, const double *x0,
+                                                                   const double *pert, const double *Li,
+                                                                   const double *LiT, const double *D, double *V,
+                                                                   double *H, int ldh, double *hist) {
+    constexpr int Q = 2 * NU;
+    // vectors padded with zeros: a column of L^-1 starts at its diagonal and runs past n
+    __shared__ double red[8], v[128 * NU], w[128 * NU], t[128 * NU];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double R[3][Q][4][NU];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int u = 0; u < NU; ++u) {
+                const int j = 4 * (wave + 8 * q) + c, row = lane + 64 * u;
+                R[0][q][c][u] = (j < n && j + row < n) ? Li[j + row + (long) j * n] : 0.0;
+                R[1][q][c][u] = (j < n && row < n) ? D[row + (long) j * n] : 0.0;
+                R[2][q][c][u] = (j < n && row < j + 1) ? LiT[row + (long) j * n] : 0.0;
+            }
+    for (int e = threadIdx.x; e < 128 * NU; e += 512) v[e] = w[e] = t[e] = 0.0;
+    __syncthreads();
+    // products with matrix f and coldot's rows and order of summation: 0 from the diagonal
+    // down, 1 all rows, 2 down to the diagonal
+    auto product = [&](auto f, const double *in, double *out) {
+        constexpr int F = decltype(f)::value;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int j0 = 4 * (wave + 8 * q);
+            double s[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                s[c] = 0.0;
+#pragma unroll
+                for (int u = 0; u < NU; ++u) {
+                    const double x = in[(F == 0 ? min(j0 + c, n - 1) : 0) + lane + 64 * u];
+                    s[c] += R[F][q][c][u] * ((F == 2 && lane + 64 * u > j0 + c) ? 0.0 : x);
+                }
+            }
+            const double sum = wave_tree_sum4(s[0], s[1], s[2], s[3]);
+            const int j = j0 + tree_sum4_slot(lane);
+            if ((lane & 15) == 0 && j < n) out[j] = sum;
+        }
+        __syncthreads();
+    };
+    const int i = threadIdx.x;
+    double vm = 0.0;  // V_{k - 1} and its norm at the step before
+    double prev = 0.0;
+    if (k0 == 0) {
+        double x = 0.0, c = 0.0;
+        if (i < n) {
+            x = pert ? x0[i] + pert[i] : x0[i];
+            c = 0.0 + x * x;
+        }
+        const double nrm = sqrt(block_sum4<0>(c, red));
+        const double inv = (nrm > 0.0) ? 1.0 / nrm : 0.0;
+        if (i < n) {
+            const double q = (nrm > 0.0) ? x * inv : 0.0;
+            v[i] = q;
+            V[i] = q;
+        }
+    } else {
+        prev = H[k0 + (k0 - 1) * ldh];
+        if (i < n) {
+            vm = V[i + (long) (k0 - 1) * n];
+            v[i] = V[i + (long) k0 * n];
+        }
+    }
+    __syncthreads();
+    for (int k = k0; k < k1; ++k) {
+        product(std::integral_constant<int, 0>(), v, w);
+        product(std::integral_constant<int, 1>(), w, t);
+        if (i < n) t[i] = -1.0 * t[i];
+        __syncthreads();
+        product(std::integral_constant<int, 2>(), t, w);
+        double q = 0.0, vk = 0.0, a = 0.0;
+        if (i < n) {
+            q = w[i];
+            vk = v[i];
+            if (k > 0) q += -prev * vm;
+            a = 0.0 + q * vk;
+        }
+        const double alp = -block_sum4<1>(a, red);
+        double c = 0.0;
+        if (i < n) {
+            q = q + alp * vk;
+            c = 0.0 + q * q;
+        }
+        const double nrm = sqrt(block_sum4<0>(c, red));
         const double inv = (nrm > 0.0) ? 1.0 / nrm : 0.0;
         vm = vk;
         prev = (nrm > 0.0) ? nrm : 0.0;
@@ -576,7 +718,12 @@ __global__ __launch_bounds__(1024) void lz_small_bound_kernel(int n, int kp1, do
     }
 void lz_small_steps(hipStream_t s, int n, int k0, int k1, const double *x0, const double *pert, const double *Li,
                     const double *LiT, const double *D, double *V, double *H, int ldh, double *hist) {
-    HDK_LZS((lz_small_steps_kernel<NU><<<1, 1024, 0, s>>>(n, k0, k1, x0, pert, Li, LiT, D, V, H, ldh, hist)))
+    if (n <= 64)
+        lz_resident_steps_kernel<1><<<1, 512, 0, s>>>(n, k0, k1, x0, pert, Li, LiT, D, V, H, ldh, hist);
+    else if (n <= 128)
+        lz_resident_steps_kernel<2><<<1, 512, 0, s>>>(n, k0, k1, x0, pert, Li, LiT, D, V, H, ldh, hist);
+    else
+        lz_small_steps_kernel<3><<<1, 1024, 0, s>>>(n, k0, k1, x0, pert, Li, LiT, D, V, H, ldh, hist);
 }
 void lz_small_bound(hipStream_t s, int n, int kp1, double e1, const LzCoef &y1, const LzCoef &y2, const double *Li,
                     const double *LiT, const double *D, const double *V, double *warm, double *report) {
