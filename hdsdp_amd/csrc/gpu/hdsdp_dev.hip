@@ -85,7 +85,7 @@ struct hdsdp_dev {
     // Lanczos (linalg/hdsdp_lanczos.c): the dual cone's solver (lzComputed, lwarm) and the
     // primal method's own (lzComputedP, lwarmP; interface/hdsdp_psdp.c:113-116)
     int lzMax, lzComputed, lzComputedP;
-    double *V, *Hd, *lv, *lw, *lz1, *lz2, *lwarm, *lwarmP, *mv1, *mv2;
+    double *V, *Hd, *lv, *lw, *lz1, *lz2, *lwarm, *lwarmP, *mv1, *mv2, *lzq;
     // primal method (interface/hdsdp_psdp.c): the primal iterate is X; Xs its value at the
     // start (the fixed scaling), dXp the direction, XSX the buffer X S X (+ Xs dS Xs), Sold
     // the dual matrix of the iteration, LX / LXi / LXiT the Cholesky factor of X and inverses
@@ -279,7 +279,8 @@ hdsdp_retcode lz_vectors(hdsdp_dev *d) {
 // estimate combines, so the result is that of the step-by-step loop.
 hdsdp_retcode lanczos(hdsdp_dev *d, const LzOp &op, double *maxStep) {
     const int n = d->n, maxDim = d->lzMax, nH = maxDim + 1;
-    const bool small = n <= hdk::LZS_MAX;
+    // small: the steps of a window in one launch; fused: a step with the next one's first product
+    const bool small = n <= hdk::LZS_MAX, fused = !small && n <= hdk::LZF_MAX;
     std::vector<double> &H = d->Hh;
     std::fill(H.begin(), H.end(), 0.0);
     DCALL(lz_vectors(d));
@@ -298,8 +299,17 @@ hdsdp_retcode lanczos(hdsdp_dev *d, const LzOp &op, double *maxStep) {
             d->stats[3] += k1 - k0;
         } else {
             for (int k = k0; k < k1; ++k) {
-                lz_mvec(d, op, d->lv, d->lw);
-                hdk::lz_step(d->st, n, k, d->lw, d->V, d->Hd, nH, d->lv, d->hHist);
+                if (fused) {
+                    // lzq = L^-T v_k: from the step before, past the look between two windows
+                    if (k == 0) hdk::coldot<double>(d->st, n, n, 1, 1.0, op.Li, n, d->lv, 0.0, d->lzq);
+                    hdk::coldot<double>(d->st, n, n, 0, -1.0, op.D, n, d->lzq, 0.0, d->mv2);
+                    hdk::coldot<double>(d->st, n, n, 2, 1.0, op.LiT, n, d->mv2, 0.0, d->lw);
+                    hdk::lz_step_product(d->st, n, k, d->lw, d->V, d->Hd, nH, d->hHist, op.Li, d->lzq);
+                    d->stats[3] += 1;
+                } else {
+                    lz_mvec(d, op, d->lv, d->lw);
+                    hdk::lz_step(d->st, n, k, d->lw, d->V, d->Hd, nH, d->lv, d->hHist);
+                }
             }
         }
         DCALL(sync(d));
@@ -937,6 +947,7 @@ hdsdp_retcode hdsdp_dev_create(hdsdp_dev **pdev, int nRow, int nCol, int precisi
     DCALL(dalloc(d, &d->lwarm, n));
     DCALL(dalloc(d, &d->mv1, n));
     DCALL(dalloc(d, &d->mv2, n));
+    DCALL(dalloc(d, &d->lzq, n));
     DCALL(dalloc(d, &d->M, m * m));
     {
         long lowerMin = 16384;

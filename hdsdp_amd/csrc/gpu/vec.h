@@ -63,6 +63,11 @@ struct LzCoef {
 // Step k of Lanczos on w: V_{k + 1}, v and the norm in H (zeros when the norm is 0), and
 // (alpha_k, norm_k) in hist (host memory the device can write).
 void lz_step(hipStream_t s, int n, int k, double *w, double *V, double *H, int ldh, double *v, double *hist);
+// lz_step for n <= LZF_MAX without its v, and y = Li^T V_{k + 1} for the lower-triangular Li
+// (n x n) in the same launch; w is left as it is
+constexpr int LZF_MAX = 2048;
+void lz_step_product(hipStream_t s, int n, int k, const double *w, double *V, double *H, int ldh, double *hist,
+                     const double *Li, double *y);
 // v = V_0 = x / ||x|| with x = x0, or x0 + pert where pert is not null
 void lz_start(hipStream_t s, int n, const double *x0, const double *pert, double *v, double *V);
 void lz_comb(hipStream_t s, int n, int kp1, const double *V, const LzCoef &y, double *z);

@@ -589,3 +589,26 @@ def test_rank_one_buffer_on_small_tiles(gpu_lib, n, m):
 def test_dense_gram_packed_tiles(gpu_lib, n, m):
     """The dense Gram build as above (same bounds) at the edges of the narrower tiles."""
     test_dense_gram_build(gpu_lib, n, m)
+
+
+# the step with the next product in one launch (n <= 2048) and the separate launches past it
+@pytest.mark.parametrize("n", [161, 255, 1023, 1025, 2048, 2049])
+def test_lanczos_step_with_product(gpu_lib, n):
+    """Two ratio tests (the second from the warm start) for dS = -e_0 e_0^T, where the largest
+    step is 1 / (S^-1)_00.  The iteration stops once its bound on the eigenvalue is within
+    1e-3 of the estimate and takes the larger one, so the step is at most the true one (up to
+    rounding, n u kappa) and short of it by 1e-3 (1 / lambda) of it."""
+    rng = np.random.default_rng(n)
+    S, coeffs = _spd_coeffs(n, rng)
+    d = dt.Dev(gpu_lib, coeffs)
+    d.update(1.0, 0.0, np.zeros(2), 0.0, 0)
+    assert d.factorize(0) == 1
+    e0 = np.zeros(n)
+    e0[0] = 1.0
+    lam = np.linalg.solve(S, e0)[0]
+    for _ in range(2):
+        d.update(0.0, 1.0, np.array([-1.0, 0.0]), 0.0, 2)
+        step = d.ratio(0)
+        assert step <= (1.0 / lam) * (1.0 + 10.0 * n * 1.1e-16)
+        assert step >= 1.0 / (lam + 1e-3) * (1.0 - 1e-9)
+    d.close()
