@@ -215,12 +215,103 @@ __global__ __launch_bounds__(1024) void cgj_iter_kernel(int m, int iter, const d
     }
 }
 
+// The same iteration of a vector of at most 1024 E entries, every vector read once into
+// registers (E entries per thread) and written once.  The loops above wait for memory in
+// each of their three passes: m = 3001 9.5 us against 6.9.  Six entries of six vectors are
+// what 128 registers hold; longer vectors keep the loops.
+template <int E>
+__global__ __launch_bounds__(1024) void cgj_iter_reg_kernel(int m, int iter, const double *jac, const double *Mp,
+                                                            double *x, double *r, double *z, double *p, double *sc,
+                                                            double *report) {
+    __shared__ double red[32];
+    const bool running = sc[CG_STOP] == CG_RUNNING;  // the same for every thread, as above
+    if (running) {
+        const double bnorm = sc[CG_BNORM], tol = sc[CG_TOL];
+        double vz[E], vr[E], vp[E], vM[E], vx[E], vj[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = threadIdx.x + 1024 * e;
+            const bool in = i < m;
+            vz[e] = in ? z[i] : 0.0;
+            vr[e] = in ? r[i] : 0.0;
+            vp[e] = in ? p[i] : 0.0;
+            vM[e] = in ? Mp[i] : 0.0;
+            vx[e] = in ? x[i] : 0.0;
+            vj[e] = in ? jac[i] : 1.0;
+        }
+        double a = 0.0, b = 0.0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            a += vz[e] * vr[e];
+            b += vp[e] * vM[e];
+        }
+        const double rz = block_sum<0>(a, red);
+        const double pMp = block_sum<1>(b, red);
+        const double alpha = rz / pMp;
+        a = 0.0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            vx[e] += alpha * vp[e];
+            const double v = vr[e] - alpha * vM[e], t = v / vj[e];
+            vr[e] = v;
+            vz[e] = t;
+            if ((int) threadIdx.x + 1024 * e < m) a += v * t;
+        }
+        const double beta = block_sum<0>(a, red) / rz;
+        double c = 0.0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = threadIdx.x + 1024 * e;
+            if (i >= m) continue;
+            x[i] = vx[e];
+            r[i] = vr[e];
+            z[i] = vz[e];
+            p[i] = vz[e] + beta * vp[e];
+            c += vr[e] * vr[e];
+        }
+        const double nrm = sqrt(block_sum<1>(c, red));
+        if (threadIdx.x == 0) {
+            const double stop = (nrm != nrm)                          ? CG_NAN
+                                : (iter > 20 && nrm > 0.01 * bnorm) ? CG_STALLED
+                                : (nrm < tol)                         ? CG_CONVERGED
+                                                                      : CG_RUNNING;
+            sc[CG_RNORM] = nrm;
+            sc[CG_ITER] = iter;
+            sc[CG_STOP] = stop;
+            if (report) {
+                report[CG_RNORM] = nrm;
+                report[CG_BNORM] = bnorm;
+                report[CG_TOL] = tol;
+                report[CG_ITER] = iter;
+                report[CG_STOP] = stop;
+            }
+        }
+    } else if (report && threadIdx.x == 0) {
+        report[CG_RNORM] = sc[CG_RNORM];
+        report[CG_BNORM] = sc[CG_BNORM];
+        report[CG_TOL] = sc[CG_TOL];
+        report[CG_ITER] = sc[CG_ITER];
+        report[CG_STOP] = sc[CG_STOP];
+    }
+}
+
 void cgj_start(hipStream_t s, int m, const double *rhs, const double *jac, double relTol, double absTol, double *r,
                double *x, double *z, double *p, double *sc) {
     cgj_start_kernel<<<1, 1024, 0, s>>>(m, rhs, jac, relTol, absTol, r, x, z, p, sc);
 }
 void cgj_iter(hipStream_t s, int m, int iter, const double *jac, const double *Mp, double *x, double *r, double *z,
               double *p, double *sc, double *report) {
+#define HDK_CGJ(e)                                                                                           \
+    if (m <= 1024 * e) {                                                                                     \
+        cgj_iter_reg_kernel<e><<<1, 1024, 0, s>>>(m, iter, jac, Mp, x, r, z, p, sc, report);                 \
+        return;                                                                                              \
+    }
+    HDK_CGJ(1)
+    HDK_CGJ(2)
+    HDK_CGJ(3)
+    HDK_CGJ(4)
+    HDK_CGJ(6)
+#undef HDK_CGJ
     cgj_iter_kernel<false><<<1, 1024, 0, s>>>(m, iter, jac, Mp, x, r, z, p, sc, report);
 }
 void cgj_half(hipStream_t s, int m, const double *z, const double *r, const double *p, const double *Mp, double *x,

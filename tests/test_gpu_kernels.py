@@ -612,3 +612,47 @@ def test_lanczos_step_with_product(gpu_lib, n):
         assert step <= (1.0 / lam) * (1.0 + 10.0 * n * 1.1e-16)
         assert step >= 1.0 / (lam + 1e-3) * (1.0 - 1e-9)
     d.close()
+
+
+# entries per thread of the Jacobi CG's vector step, and the first size past them
+@pytest.mark.parametrize("m", [1024, 1025, 2049, 3072, 4096, 4097, 6144, 6145])
+def test_jacobi_cg_vector_step_edges(gpu_lib, m):
+    """Jacobi CG to |r| < 1e-11 |b| on M + I of single-entry constraints against numpy's M x: cond
+    < 3 and the recursive residual's drift of a few m u leave 1e-10 of |b|."""
+    rng = np.random.default_rng(m)
+    n = 120
+    S, (C, _, _) = _spd_coeffs(n, rng)
+    r, c = np.tril_indices(n)
+    pick = np.sort(rng.choice(len(r), size=m, replace=False))
+    one = np.ones(1)
+    d = dt.Dev(gpu_lib, [C] + [dt.Coeff(dt.SPARSE, n, row=[r[k]], col=[c[k]], val=one) for k in pick])
+    d.kkt_params(1e-11, 1e-11, 200, -1)
+    d.update(1.0, 0.0, np.zeros(m), 0.0, 0)
+    assert d.factorize(0) == 1
+    d.schur(0, 0.0)
+    d.add_diag(np.ones(m))
+    assert d.kkt_factorize() == 0
+    b = rng.standard_normal(m)
+    x = d.kkt_solve(b)
+    M = d.get_schur()
+    d.close()
+    assert np.linalg.norm(M @ x - b) <= 1e-10 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 600])
+def test_primal_dot_products(gpu_lib, n):
+    """<X, S> and tr(X) of the recovered X against sums of its entries in numpy: n^2 terms in
+    at most n + 300 additions each, relative to the sum of absolute values."""
+    rng = np.random.default_rng(n)
+    S, coeffs = _spd_coeffs(n, rng)
+    d = dt.Dev(gpu_lib, coeffs)
+    for which in (0, 1):
+        d.update(1.0, 0.0, np.zeros(2), 0.0, which)
+        assert d.factorize(which) == 1
+    d.primal(0.5, np.zeros(2), np.zeros(2))
+    X = d.get_primal()
+    _, _, xs, tx = d.primal_stats()
+    d.close()
+    u = 1.1e-16
+    assert abs(xs - np.sum(X * S)) <= (2.0 * n + 600.0) * u * np.sum(np.abs(X * S))
+    assert abs(tx - np.trace(X)) <= (n + 300.0) * u * np.sum(np.abs(np.diag(X)))
