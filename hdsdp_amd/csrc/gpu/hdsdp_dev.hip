@@ -86,6 +86,7 @@ struct hdsdp_dev {
     // primal method's own (lzComputedP, lwarmP; interface/hdsdp_psdp.c:113-116)
     int lzMax, lzComputed, lzComputedP;
     double *V, *Hd, *lv, *lw, *lz1, *lz2, *lwarm, *lwarmP, *mv1, *mv2, *lzq;
+    double *dotPart;  // 512 partial sums of xdots
     // primal method (interface/hdsdp_psdp.c): the primal iterate is X; Xs its value at the
     // start (the fixed scaling), dXp the direction, XSX the buffer X S X (+ Xs dS Xs), Sold
     // the dual matrix of the iteration, LX / LXi / LXiT the Cholesky factor of X and inverses
@@ -948,6 +949,7 @@ hdsdp_retcode hdsdp_dev_create(hdsdp_dev **pdev, int nRow, int nCol, int precisi
     DCALL(dalloc(d, &d->mv1, n));
     DCALL(dalloc(d, &d->mv2, n));
     DCALL(dalloc(d, &d->lzq, n));
+    DCALL(dalloc(d, &d->dotPart, 512));
     DCALL(dalloc(d, &d->M, m * m));
     {
         long lowerMin = 16384;
@@ -1660,7 +1662,9 @@ hdsdp_retcode lu_factor(hdsdp_dev *d) {
 // fails switches the system to the direct indefinite solver
 hdsdp_retcode hdsdp_dev_kkt_factorize(hdsdp_dev *d) {
     if (d->useLU) return lu_factor(d);
-    hdk::mirror_lower<double>(d->st, d->m, d->M, d->m);
+    // the products with a large M read its lower triangle only (symv_M), as the factorisations
+    // do; the one-workgroup CG of a small one reads both
+    if (!d->symvW || d->m <= hdk::CGS_MAX) hdk::mirror_lower<double>(d->st, d->m, d->M, d->m);
     hdsdp_retcode rc = build_precond(d);
     if (rc != HDSDP_RETCODE_OK && d->mGramPending) {
         DCALL(rebuild_gram_fp64(d));
@@ -1817,7 +1821,7 @@ hdsdp_retcode hdsdp_dev_primal_stats(hdsdp_dev *d, double *AX, double *traceCX, 
     const int m = d->m;
     hdk::traces(d->st, d->c, 0, m + 1, d->X, nullptr, 0.0, d->vecA_d, nullptr, false);
     hdk::r1_quadforms(d->st, d->c, d->X, true, 0, m + 1, 0.0, d->vecA_d, nullptr, d->H1);
-    hdk::xdots(d->st, d->n, d->X, d->S[0], d->sc_d + hdk::SC_AUX);
+    hdk::xdots(d->st, d->n, d->X, d->S[0], d->dotPart, d->sc_d + hdk::SC_AUX);
     DCALL(check_launch());
     DCALL(download(d, d->hvecB, d->vecA_d, m + 1, d->hvecA));
     *traceCX = d->hvecB[0];
@@ -1938,7 +1942,7 @@ hdsdp_retcode hdsdp_dev_psdp_step(hdsdp_dev *d, double alpha, int *isPsd, double
     // <C, X> and <X, S> with the dual matrix of this iteration (hdsdp_psdp.c:268-271)
     hdk::traces(d->st, d->c, 0, 1, d->X, nullptr, 0.0, d->vecA_d, nullptr, false);
     hdk::r1_quadforms(d->st, d->c, d->X, true, 0, 1, 0.0, d->vecA_d, nullptr, d->H1);
-    hdk::xdots(d->st, n, d->X, d->Sold, d->sc_d + hdk::SC_AUX);
+    hdk::xdots(d->st, n, d->X, d->Sold, d->dotPart, d->sc_d + hdk::SC_AUX);
     DCALL(check_launch());
     DCALL(download(d, d->hvecB, d->vecA_d, 1, d->hvecA));
     *traceCX = d->hvecB[0];

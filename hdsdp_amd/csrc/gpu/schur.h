@@ -85,7 +85,8 @@ void schur_pairs(hipStream_t s, const DevCoeffs &c, const double *W, double *M, 
 void scatter_row(hipStream_t s, int m, int h, const double *t, double *M, long ldm);
 void densify(hipStream_t s, const DevCoeffs &c, int k, double *out);
 void sym_avg(hipStream_t s, int n, const double *A, double scale, double diag, double *out);
-void xdots(hipStream_t s, int n, const double *X, const double *S, double *out);
+// out[0] = <X, S> over the lower triangles, out[1] = tr(X); part: 512 doubles
+void xdots(hipStream_t s, int n, const double *X, const double *S, double *part, double *out);
 void trace_diag(hipStream_t s, int n, const double *A, double *out);
 
 }  // namespace hdk

@@ -688,42 +688,51 @@ void sym_avg(hipStream_t s, int n, const double *A, double scale, double diag, d
     sym_avg_kernel<<<4096, 256, 0, s>>>(n, A, scale, diag, out);
 }
 
-// out[0] = sum_{i >= j} (2 - [i == j]) X_ij S_ij ; out[1] = tr(X) ; out[2] = tr(W)-like trace of A (diag)
-__global__ __launch_bounds__(1024) void xdots_kernel(int n, const double *X, const double *S, double *out) {
-    __shared__ double red[17];
+// part[0][g] = the share of workgroup g in sum_{i >= j} (2 - [i == j]) X_ij S_ij, part[1][g] in
+// tr(X): columns g, g + gridDim.x, ..., each thread its rows
+__global__ __launch_bounds__(256) void xdots_kernel(int n, const double *X, const double *S, double *part) {
+    __shared__ double red[2][4];
     double a = 0.0, t = 0.0;
-    long total = (long) n * n;
-    for (long e = threadIdx.x; e < total; e += blockDim.x) {
-        long i = e % n, j = e / n;
-        if (i > j) a += 2.0 * X[e] * S[e];
-        else if (i == j) {
-            a += X[e] * S[e];
-            t += X[e];
+    for (int j = blockIdx.x; j < n; j += gridDim.x) {
+        const double *x = X + (long) j * n, *s = S + (long) j * n;
+        for (int i = j + threadIdx.x; i < n; i += 256) {
+            if (i > j) a += 2.0 * x[i] * s[i];
+            else {
+                a += x[i] * s[i];
+                t += x[i];
+            }
         }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_down(a, off);
-        t += __shfl_down(t, off);
-    }
-    __shared__ double red2[17];
+    a = wave_sum(a);
+    t = wave_sum(t);
     if ((threadIdx.x & 63) == 0) {
-        red[threadIdx.x >> 6] = a;
-        red2[threadIdx.x >> 6] = t;
+        red[0][threadIdx.x >> 6] = a;
+        red[1][threadIdx.x >> 6] = t;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double sa = 0.0, st = 0.0;
-        for (int w = 0; w < (int) (blockDim.x >> 6); ++w) {
-            sa += red[w];
-            st += red2[w];
-        }
-        out[0] = sa;
-        out[1] = st;
-    }
+    if (threadIdx.x < 2)
+        part[threadIdx.x * gridDim.x + blockIdx.x] =
+            red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
 }
 
-void xdots(hipStream_t s, int n, const double *X, const double *S, double *out) {
-    xdots_kernel<<<1, 1024, 0, s>>>(n, X, S, out);
+// out[w] = the sum of the cnt <= 256 parts w, w < 2
+__global__ __launch_bounds__(256) void xdots_sum_kernel(int cnt, const double *part, double *out) {
+    __shared__ double red[2][4];
+    for (int w = 0; w < 2; ++w) {
+        const double v = wave_sum(((int) threadIdx.x < cnt) ? part[w * cnt + threadIdx.x] : 0.0);
+        if ((threadIdx.x & 63) == 0) red[w][threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        out[threadIdx.x] = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
+}
+
+// One pass over both lower triangles on up to 256 workgroups; the one workgroup it replaces
+// walked all n^2 entries: n = 250 34 us against 3, n = 2000 1.7 ms.
+void xdots(hipStream_t s, int n, const double *X, const double *S, double *part, double *out) {
+    const int g = std::min(n, 256);
+    xdots_kernel<<<g, 256, 0, s>>>(n, X, S, part);
+    xdots_sum_kernel<<<1, 256, 0, s>>>(g, part, out);
 }
 
 __global__ __launch_bounds__(1024) void trace_diag_kernel(int n, const double *A, double *out) {
