@@ -55,7 +55,8 @@ __global__ __launch_bounds__(1024) void cg_jacobi_kernel(int m, const double *r,
     }
 }
 
-// rz = z.r; pMp = p.Mp; alpha = rz / pMp; x += alpha p; rn = r - alpha Mp
+// rz = z.r; pMp = p.Mp; alpha = rz / pMp; x += alpha p; rn = r - alpha Mp; sc[CG_RNORM] = ||rn||:
+// the host decides on it before the preconditioner and the product of a next step
 __global__ __launch_bounds__(1024) void cg_step1_kernel(int m, const double *z, const double *r, const double *p,
                                                         const double *Mp, double *x, double *rn, double *sc) {
     __shared__ double red[32];
@@ -67,32 +68,32 @@ __global__ __launch_bounds__(1024) void cg_step1_kernel(int m, const double *z, 
     double rz = block_sum<0>(a, red);
     double pMp = block_sum<1>(b, red);
     double alpha = rz / pMp;
+    double c = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         x[i] += alpha * p[i];
-        rn[i] = r[i] - alpha * Mp[i];
+        const double v = r[i] - alpha * Mp[i];
+        rn[i] = v;
+        c += v * v;
     }
+    const double nrm = sqrt(block_sum<0>(c, red));
     if (threadIdx.x == 0) {
         sc[CG_RZ] = rz;
         sc[CG_ALPHA] = alpha;
+        sc[CG_RNORM] = nrm;
     }
 }
 
-// beta = rn.z / rz; p = z + beta p; r = rn; sc[CG_RNORM] = ||r||
+// beta = rn.z / rz; p = z + beta p; r = rn
 __global__ __launch_bounds__(1024) void cg_step2_kernel(int m, const double *rn, const double *z, double *p, double *r,
                                                         double *sc) {
     __shared__ double red[32];
     double a = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) a += rn[i] * z[i];
     double beta = block_sum<0>(a, red) / sc[CG_RZ];
-    double c = 0.0;
     for (int i = threadIdx.x; i < m; i += blockDim.x) {
         p[i] = z[i] + beta * p[i];
-        double v = rn[i];
-        r[i] = v;
-        c += v * v;
+        r[i] = rn[i];
     }
-    double nrm = sqrt(block_sum<1>(c, red));
-    if (threadIdx.x == 0) sc[CG_RNORM] = nrm;
 }
 
 // r = rhs - Mx (Mx precomputed)
