@@ -434,9 +434,10 @@ hdsdp_retcode build_precond(hdsdp_dev *d) {
     d->stats[4] += 1;
     prof_begin(d, HDSDP_PROF_MFACTOR);
     // Mixed precision factors M in FP32 when its Gram blocks are bf16 products (an FP32-
-    // accurate matrix) or when M is large enough for the FP32 factorisation to save more
-    // than the extra CG steps of the coarser preconditioner cost (measured: m = 20000
-    // saves 15 ms per iteration for 9 ms of CG; m = 8084 saves 1.7 ms for 7 ms of CG)
+    // accurate matrix), or when M is so large that three FP64 matrices beside it are a
+    // question of memory (m = 65536: 137 GB in all).  Below, the FP64 factor is the faster one:
+    // at m = 20000 the FP32 factorisation saves 1.5 ms per iteration and its coarser
+    // preconditioner costs 22 ms of CG (0.219 s per iteration against 0.197); m = 8084 1.7 and 7.
     if (d->precision == HDSDP_PRECISION_MIXED && (d->mGramPending || d->m >= d->chol32Min)) {
         int ok = 0;
         DCALL(build_chol32(d, &ok));
@@ -978,7 +979,7 @@ hdsdp_retcode hdsdp_dev_create(hdsdp_dev **pdev, int nRow, int nCol, int precisi
     d->absTol = 1e-06;
     d->relTol = 1e-06;
     d->useJacobi = d->paramUseJacobi = 1;
-    d->chol32Min = 16384;
+    d->chol32Min = 65536;
     if (const char *c32 = getenv("HDSDP_MIXED_CHOL32_MIN")) d->chol32Min = atoi(c32);
     d->mixedFloor = 1e-13;
     if (const char *mf = getenv("HDSDP_MIXED_FLOOR")) d->mixedFloor = atof(mf);
