@@ -193,8 +193,7 @@ __device__ inline void big_store(T (*As)[BT + BPAD], T (*Bs)[BT + BPAD], int tid
 
 // PACK 1 (square lower products with beta = 0): the strictly lower part of the result's
 // first ldc rows and columns goes to C packed by columns and the diagonal to dg (stride
-// sDg), as pack_lower stores them.  PACK 2: the same entries in k panels, packed entry e of
-// matrix z at C[(e / 16) slab + 16 z + e % 16].
+// sDg), as pack_lower stores them.
 // PANEL: both operands are read from k panels of 16, entry (k, i) at (k / 16) slab + 16 i +
 // k % 16, so that a slab of a tile is 16 KB of consecutive memory; K a multiple of 16,
 // rows of whole tiles present.
@@ -292,8 +291,7 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(int M, int N, int K, T al
                 const T v = alpha * stage[cc][lane];
                 const long e = j * n - j * (j + 1) / 2 + (i - j - 1);
                 if (i == j) dg[(long) blockIdx.z * sDg + i] = v;
-                else if (PACK == 1) C[e] = v;
-                else C[(e >> 4) * slab + 16 * blockIdx.z + (e & 15)] = v;
+                else C[e] = v;
             }
             continue;
         }
@@ -369,7 +367,8 @@ static void gemm_big(hipStream_t s, bool transA, bool transB, bool lower, int M,
 // while it is multiplied.  Every output sums its k in ascending order whatever the tile, so
 // the choice of one does not change a bit.  The last batch entry may have fewer rows
 // (mLast > 0) and a shorter k (kLast > 0).  PACK: the strictly lower part of a square result
-// goes to C packed by columns and its diagonal to dg (beta = 0).
+// goes to C packed by columns (1) or in k panels (2: packed entry e of matrix z at
+// C[(e / 16) slab + 16 z + e % 16]) and its diagonal to dg (beta = 0).
 template <int TI>
 struct MidTile {
     static constexpr int TK = (TI == 32) ? 64 : 32, LR = TI + 16, LK = TK + 2, F = TI / 32;
@@ -403,7 +402,7 @@ template <typename T, bool TA, bool TB, bool LOWER, int TI, int PACK = 0>
 __global__ __launch_bounds__(256) void gemm_mid_kernel(int M, int N, int K, T alpha, const T *A, int lda, long sA,
                                                        const T *B, int ldb, long sB, T beta, T *C, int ldc, long sC,
                                                        int tri, int lin, int mLast, int kLast, T *dg = nullptr,
-                                                       long sDg = 0) {
+                                                       long sDg = 0, long slab = 0) {
     typedef MidTile<TI> G;
     constexpr int F = G::F, TK = G::TK, LR = G::LR, LK = G::LK;
     constexpr bool KCA = TA, KCB = !TB;  // operand consecutive along k
@@ -475,7 +474,10 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(int M, int N, int K, T al
                 if (i >= M || j >= N || (LOWER && i < j)) continue;
                 if (PACK) {
                     if (i == j) dg[blockIdx.z * sDg + i] = alpha * acc[a][b][r];
-                    else C[(long) j * N - (long) j * (j + 1) / 2 + (i - j - 1)] = alpha * acc[a][b][r];
+                    else {
+                        const long q = (long) j * N - (long) j * (j + 1) / 2 + (i - j - 1);
+                        C[PACK == 1 ? q : (q >> 4) * slab + 16 * blockIdx.z + (q & 15)] = alpha * acc[a][b][r];
+                    }
                 } else {
                     C[i + (long) j * ldc] = alpha * acc[a][b][r] + beta * cin[a][b][r];
                 }
@@ -583,17 +585,20 @@ void gram_panels(hipStream_t s, int r, int kc, int kLast, int parts, double alph
         nullptr, 0, slab);
 }
 
-// C_z = A_z B_z^T for z < batch, lower triangle, packed (PACK above); tri as in gemm
+// C_z = A_z B_z^T for z < batch, lower triangle, packed (PACK above); tri as in gemm.  k panels
+// (operands of whole 128-wide tiles, n >= 512) are stored by the 64-wide tiles, whose triangle
+// of tiles and k ranges wastes less: T_p = U_p L^-T, us at 64 and 128: 60 of n = 512 119 and 151,
+// of 1024 599 and 691, 28 of 1536 804 and 887, 16 of 2048 1038 and 1134.
 void gemm_nt_packed(hipStream_t s, int rows, int n, const double *A, int lda, long sA, const double *B, int ldb,
                     long sB, double *off, long K1, long slab, double *dg, long sDg, int batch, int tri) {
     const bool vec = vec_ok<double>(A, lda, sA, B, ldb, sB);
-    const int t = (slab > 0) ? 128 : pick_tile(n, n, n, true, batch, tri, vec);
+    const int t = (slab > 0) ? 64 : pick_tile(n, n, n, true, batch, tri, vec);
     if (t < 128) rows = n;
     const int nt = (rows + t - 1) / t, K = std::min(rows, (n + KSTEP - 1) / KSTEP * KSTEP);
     const dim3 grid(nt * (nt + 1) / 2, 1, batch);
     if (slab > 0)
-        gemm_big_kernel<double, false, true, true, true, 2><<<grid, 256, 0, s>>>(
-            rows, rows, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, 0, tri, 1, 0, dg, sDg, slab);
+        gemm_mid_kernel<double, false, true, true, 64, 2><<<grid, 256, 0, s>>>(
+            n, n, n, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, 0, tri, 1, 0, 0, dg, sDg, slab);
     else if (t == 32)
         gemm_mid_kernel<double, false, true, true, 32, 1><<<grid, 256, 0, s>>>(
             n, n, n, 1.0, A, lda, sA, B, ldb, sB, 0.0, off, n, K1, tri, 1, 0, 0, dg, sDg);

@@ -707,7 +707,7 @@ int cg_solve(hdsdp_dev *d) {
 //
 // From n = GRAM_HALF_MIN: T(i, j) sums U(i, k) L^-1(j, k) over k <= j <= i, so of
 // U = L^-1 A_p the lower triangle is formed only: n^3 / 3 + n^3 / 6 multiply-adds per
-// constraint (n = 1000, 1000 constraints: 15 and 10 ms; <T_p, T_q> 9 ms, 64 TF).  Below,
+// constraint (n = 1000, 1000 constraints: 16 and 9 ms; <T_p, T_q> 9 ms, 64 TF).  Below,
 // the full U and T_p = L^-1 U^T, n^3 / 2 + n^3 / 3 (26 and 18 ms at that size): there the products are a small share of the build, and the
 // Lanczos step bound that the Schur solutions feed, run without reorthogonalisation to a
 // good part of n steps, turns a last-bit change of M into one of up to 4e-3 (n = 121;
