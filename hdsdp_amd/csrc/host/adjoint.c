@@ -95,8 +95,9 @@ exit_cleanup:
  * distance (17 systems there) one start in two hundred, of random SDPs with mu down to 1e-7,
  * ran out of steps where the guaranteed step converged; with 0.6 one of 9500 did.  A path
  * with longer steps that fails is taken again from its start with the guaranteed ones.
- * One more full step is taken below tol unless the residual is at rounding level, so that
- * the result does not depend on how far below tol the last step happened to land. */
+ * Where longer steps were taken, one more full step follows the first residual below tol
+ * unless that is at rounding level, so that the result does not depend on how far below tol
+ * the last step happened to land; a path of guaranteed and full steps ends at tol. */
 #define CENTRE_GROW (1.5)
 #define CENTRE_BACK (0.6)
 #define CENTRE_FLOOR (1e-05)
@@ -135,9 +136,11 @@ static hdsdp_retcode centre_newton( hdsdp *s, double mu, double *y, int maxIter,
             best = res;
             memcpy(ybest, y, sizeof(double) * m);
         }
-        if ( it >= maxIter ) break;
-        if ( res <= tol && (polished || res <= HMAX(1e-03 * tol, 1e-14)) ) break;
-        if ( res <= tol ) polished = 1;
+        if ( it >= maxIter || polished ) break;
+        if ( res <= tol ) {
+            if ( !*longer || res <= HMAX(1e-03 * tol, 1e-14) ) break;
+            polished = 1;
+        }
         /* after the quadratic phase: three full steps without halving the residual */
         stall = (res > 0.5 * prev) ? stall + 1 : 0;
         if ( stall >= 3 ) break;
