@@ -702,10 +702,11 @@ template void gemm_splitk<double>(hipStream_t, bool, bool, bool, int, int, int, 
 // ---- triangular inverse ------------------------------------------------------
 
 // Linv = the inverses of the 64 x 64 diagonal blocks, zero elsewhere in the diagonal blocks
-// of `span` rows (the rest of Linv is left alone)
+// of `span` rows (the rest of Linv is left alone).  The columns run over grid x: there may be
+// more of them than the 65535 workgroups of grid y.
 template <typename T>
 __global__ void place_diag_kernel(int n, int span, const double *Dinv, T *Linv, long ldi) {
-    const int j = blockIdx.y, t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = blockIdx.x, t = blockIdx.y * blockDim.x + threadIdx.x;
     const int i = j / span * span + t;
     if (t >= span || i >= n) return;
     const bool in = (i >> 6) == (j >> 6);
@@ -719,7 +720,7 @@ __global__ void place_diag_kernel(int n, int span, const double *Dinv, T *Linv, 
 template <typename T>
 void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work, int span) {
     if (span <= 0 || span > n) span = n;
-    place_diag_kernel<T><<<dim3((span + 255) / 256, n), 256, 0, s>>>(n, span, Dinv, Linv, ldi);
+    place_diag_kernel<T><<<dim3(n, (span + 255) / 256), 256, 0, s>>>(n, span, Dinv, Linv, ldi);
     for (int sz = NB; sz < span; sz *= 2) {
         int npair = n / (2 * sz);
         long strideL = 2L * sz * (ldl + 1), strideI = 2L * sz * (ldi + 1), strideW = (long) sz * sz;
