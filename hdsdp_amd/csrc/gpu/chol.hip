@@ -350,6 +350,7 @@ __global__ __launch_bounds__(CH_THREADS, 2) void chol_step_kernel(int n, T *A, l
                                                                   int k, int kp, int jEnd, int *info) {
     __shared__ __attribute__((aligned(16))) double P0[64][CH_LD], P1[64][CH_LD];
     __shared__ LeafScratch ls;
+    __shared__ int bad;
     if (blockIdx.x == 0) {
         if (k == 0 && threadIdx.x == 0) *info = 0;
         leaf_role(n, A, lda, L, ldl, Dinv, k, kp, info, P0, P1, &ls);
@@ -380,14 +381,16 @@ __global__ __launch_bounds__(CH_THREADS, 2) void chol_step_kernel(int n, T *A, l
             const int col = 64 * j + 16 * (cb0 + h) + 4 * r + g;
             cin[h][r] = (crow < n && col < n && crow >= col) ? (double) A[crow + (long) col * lda] : 0.0;
         }
-    const int bad = *info;
+    // workgroup 0 may write info while this one runs: one read for all threads, so that they
+    // leave together
+    if (tid == 0) bad = *info;
     stash64(P1, xp, tid);
     __syncthreads();
-    if (bad) return;
     {
         v4d p[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) p[c] = panel_block(P1, av, c, l, g);
+        if (bad) return;
         __syncthreads();
         double(*P)[CH_LD] = (w < 4) ? P0 : P1;
 #pragma unroll

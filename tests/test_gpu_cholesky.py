@@ -1,0 +1,53 @@
+"""The blocked Cholesky (hdk::potrf) called by itself, on the GPU, against numpy."""
+import ctypes as C
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+from hdsdp_amd.solver import LIB_PATH
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def potrf(gpu_lib):
+    """potrf(A) -> (L, info) of the lower triangle of a float64 or float32 array."""
+    syms = [x.split()[-1] for x in subprocess.run(["nm", "-D", LIB_PATH], capture_output=True, text=True,
+                                                  check=True).stdout.splitlines()]
+    syms = [x for x in syms if "3hdk" in x]
+    plain = subprocess.run(["c++filt"], input="\n".join(syms), capture_output=True, text=True, check=True).stdout
+    table = {p.split("(")[0].split()[-1]: s for s, p in zip(syms, plain.splitlines()) if "lambda" not in p}
+
+    def call(A):
+        n = len(A)
+        a = torch.as_tensor(np.ascontiguousarray(A.T), device="cuda")  # column-major
+        L, info = torch.zeros_like(a), torch.full((1,), 7, dtype=torch.int32, device="cuda")
+        dinv = torch.zeros((n + 63) // 64 * 4096, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        fn = getattr(gpu_lib, table["hdk::potrf<%s>" % ("double" if A.dtype == np.float64 else "float")])
+        p = lambda t: C.c_void_p(t.data_ptr())
+        fn(C.c_void_p(0), C.c_int(n), p(a), C.c_int(n), p(L), C.c_int(n), p(dinv), p(info), C.c_void_p(0))
+        torch.cuda.synchronize()
+        return L.cpu().numpy().T, int(info.cpu()[0])
+
+    return call
+
+
+def _spd(n, rng, flips=()):
+    G = rng.standard_normal((n, n)) / np.sqrt(n)
+    S = 4.0 * np.eye(n) + 0.6 * (G + G.T) / np.sqrt(2.0)
+    for i in flips:
+        S[i, i] = -1.0
+    return S
+
+
+# a single tile, launches of several tiles, more tiles than CUs, outer blocks (from 3073 rows on)
+@pytest.mark.parametrize("n,flips", [(40, ()), (64, (17,)), (65, (64,)), (200, (137, 150)), (1500, (700, 1400)),
+                                     (3000, (64,)), (3200, ()), (3200, (2309,)), (3200, (3199,))])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_info_is_the_first_failing_column(potrf, dtype, n, flips):
+    """info: the first column whose pivot is not positive, from 1, or 0."""
+    _, info = potrf(_spd(n, np.random.default_rng(n), flips).astype(dtype))
+    assert info == (min(flips) + 1 if flips else 0)
