@@ -179,6 +179,9 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = lane & 15,
               g = lane >> 4;
     const int k0 = 64 * k, kb = min(64, n - k0);
+    // the first step of an outer block (the others read info below); this workgroup is the
+    // only one that writes it, so every thread reads the same
+    const int failed = (kp < 0 && k > 0) ? *info : 0;
     // entry (r, c) of the diagonal tile, identity beyond kb; only the lower triangle of A
     // is valid
     auto diag = [&](int r, int c) -> double {
@@ -195,6 +198,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
         if (w != 4) cA[r] = diag(16 * rbA + l, 16 * cbA + 4 * r + g);
         if (w > 4) cB[r] = diag(16 * rbB + l, 16 * cbB + 4 * r + g);
     }
+    if (failed) return;  // an earlier pivot was not positive
     if (kp >= 0) {
         const int rb = w & 3, ca = (w < 4) ? 0 : 1, cb = 3 - ca;
         const Pair4 xp = fetch64(Dinv + (long) kp * 4096, tid);
@@ -209,7 +213,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
             P[16 * ca + 4 * r + g][16 * rb + l] = pa[r];
             P[16 * cb + 4 * r + g][16 * rb + l] = pb[r];
         }
-        if (bad) return;  // an earlier pivot was not positive
+        if (bad) return;
         store_panel(L, ldl, n, k0 + 16 * rb + l, kp, ca, g, pa);
         store_panel(L, ldl, n, k0 + 16 * rb + l, kp, cb, g, pb);
         __syncthreads();

@@ -43,9 +43,11 @@ def _spd(n, rng, flips=()):
     return S
 
 
-# a single tile, launches of several tiles, more tiles than CUs, outer blocks (from 3073 rows on)
+# a single tile, launches of several tiles, more tiles than CUs, outer blocks of 768 (from 3073
+# rows on): a failure in an earlier one, alone and with another in the first tile of a later one
 @pytest.mark.parametrize("n,flips", [(40, ()), (64, (17,)), (65, (64,)), (200, (137, 150)), (1500, (700, 1400)),
-                                     (3000, (64,)), (3200, ()), (3200, (2309,)), (3200, (3199,))])
+                                     (3000, (64,)), (3200, ()), (3200, (2309,)), (3200, (3199,)), (3200, (100,)),
+                                     (3200, (100, 2309)), (3200, (800, 1536))])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_info_is_the_first_failing_column(potrf, dtype, n, flips):
     """info: the first column whose pivot is not positive, from 1, or 0."""
