@@ -47,19 +47,28 @@ __device__ inline double row_bcast(double v) {
     return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + K, 0xf, 0xf, true);
 }
 
-// 1 / p to about half an ulp: the hardware's approximation (relative error e below 2^-22)
-// with the third-order step x (1 + e + e^2); 0 for an infinite p, as a division gives
+// a / p of the elimination.  Fast form: r = recip(p) from the hardware's approximation
+// (relative error e below 2^-22) with the third-order step x (1 + e + e^2), half an ulp and
+// 2^-13 of one off at most, and the quotient from a r with one residual step: correctly
+// rounded unless a / p lies within some 2^-53 ulp of the middle of two numbers (or |a| below
+// 2^-969 makes the residual underflow: an ulp then).  p and r have to be normal numbers: a tile
+// with a pivot outside FAST_MIN .. FAST_MAX is factored again with divisions (DIV), which
+// takes the step from 20 us to 38.
+constexpr double FAST_MIN = 0x1p-960, FAST_MAX = 0x1p960;
+
+template <bool DIV>
 __device__ inline double recip(double p) {
+    if (DIV) return 0.0;
     const double x = __builtin_amdgcn_rcp(p);
     const double e = __builtin_fma(-p, x, 1.0);
-    const double y = __builtin_fma(x, __builtin_fma(e, e, e), x);
-    return __builtin_isinf(p) ? 0.0 : y;
+    return __builtin_fma(x, __builtin_fma(e, e, e), x);
 }
 
-// a / p correctly rounded, from r = recip(p) and one residual step
+template <bool DIV>
 __device__ inline double quot(double a, double p, double r) {
+    if (DIV) return a / p;
     const double u = a * r;
-    return __builtin_fma(__builtin_fma(-u, __builtin_isinf(p) ? 0.0 : p, a), r, u);
+    return __builtin_fma(__builtin_fma(-u, p, a), r, u);
 }
 
 template <int... C>
@@ -74,17 +83,17 @@ __device__ inline void row_bcast_all(double v, double (&out)[16], std::integer_s
 // column K of the factor).  The next pivot is formed from its own two entries ahead of
 // the row updates, by the operations of those updates: the chain from pivot to pivot
 // has no cross-lane operation.  Entries above the diagonal are scratch.
-template <int K>
+template <int K, bool DIV>
 __device__ inline void elim_step(double (&a)[16], double (&z)[16], double &p, double &piv, int j) {
     piv = (j == K) ? p : piv;
-    const double r = recip(p), pk = p;
+    const double r = recip<DIV>(p), pk = p;
     if (K < 15) {
         const double q = row_bcast<(K + 1) & 15>(a[K]), d = row_bcast<(K + 1) & 15>(a[(K + 1) & 15]);
-        p = __builtin_fma(-quot(q, pk, r), q, d);
+        p = __builtin_fma(-quot<DIV>(q, pk, r), q, d);
     }
     double col[16];
     row_bcast_all(a[K], col, std::make_integer_sequence<int, 16>());
-    const double ta = -quot(a[K], pk, r), tz = -quot(z[K], pk, r);
+    const double ta = -quot<DIV>(a[K], pk, r), tz = -quot<DIV>(z[K], pk, r);
 #pragma unroll
     for (int c = K + 1; c < 16; ++c) {
         a[c] = __builtin_fma(ta, col[c], a[c]);
@@ -93,11 +102,11 @@ __device__ inline void elim_step(double (&a)[16], double (&z)[16], double &p, do
 }
 
 // the 16 columns of a block; returns pivot j on the lanes (j, .)
-template <int... K>
+template <bool DIV, int... K>
 __device__ inline double elim(double (&a)[16], double (&z)[16], int j, std::integer_sequence<int, K...>) {
     asm volatile("" : "+v"(j));  // keeps the step masks out of the caller's registers
     double p = row_bcast<0>(a[0]), piv = 1.0;
-    (elim_step<K>(a, z, p, piv, j), ...);
+    (elim_step<K, DIV>(a, z, p, piv, j), ...);
     return piv;
 }
 
@@ -168,11 +177,12 @@ __device__ inline v4d rank64(const double (*P1)[CH_LD], const double (*P0)[CH_LD
 // the blocking does not change a bit of them.
 struct LeafScratch {
     double p[64], r[64];  // pivots and their reciprocals
-    int fail;
+    int fail, again;
 };
 
-template <typename T>
-__device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *Dinv, int k, int kp, int *info,
+// Returns whether the tile has to be factored again with divisions (L and X not stored).
+template <typename T, bool DIV>
+__device__ bool leaf_role(int n, const T *A, long lda, T *L, long ldl, double *Dinv, int k, int kp, int *info,
                           double (*B0)[CH_LD], double (*B1)[CH_LD], LeafScratch *ls) {
     // B0: the panel rows P, then X; B1: the inverse of the last diagonal factor, then the tile
     double (*P)[CH_LD] = B0, (*Xs)[CH_LD] = B0, (*As)[CH_LD] = B1;
@@ -198,7 +208,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
         if (w != 4) cA[r] = diag(16 * rbA + l, 16 * cbA + 4 * r + g);
         if (w > 4) cB[r] = diag(16 * rbB + l, 16 * cbB + 4 * r + g);
     }
-    if (failed) return;  // an earlier pivot was not positive
+    if (failed) return false;  // an earlier pivot was not positive
     if (kp >= 0) {
         const int rb = w & 3, ca = (w < 4) ? 0 : 1, cb = 3 - ca;
         const Pair4 xp = fetch64(Dinv + (long) kp * 4096, tid);
@@ -213,7 +223,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
             P[16 * ca + 4 * r + g][16 * rb + l] = pa[r];
             P[16 * cb + 4 * r + g][16 * rb + l] = pb[r];
         }
-        if (bad) return;
+        if (bad) return false;
         store_panel(L, ldl, n, k0 + 16 * rb + l, kp, ca, g, pa);
         store_panel(L, ldl, n, k0 + 16 * rb + l, kp, cb, g, pb);
         __syncthreads();
@@ -222,7 +232,10 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
     if (w < 4)
 #pragma unroll
         for (int r = 0; r < 4; ++r) As[16 * cbA + 4 * r + g][16 * rbA + l] = cA[r];
-    if (tid == 0) ls->fail = 64;
+    if (tid == 0) {
+        ls->fail = 64;
+        ls->again = 0;
+    }
     __syncthreads();
     if (w > 4) {
         if (kp >= 0) {
@@ -243,7 +256,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int K = 16 * b + 4 * q + g;
-            c = mma(-As[K][16 * j + l], quot(As[K][16 * i + l], ls->p[K], ls->r[K]), c);
+            c = mma(-As[K][16 * j + l], quot<DIV>(As[K][16 * i + l], ls->p[K], ls->r[K]), c);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) As[16 * j + 4 * r + g][16 * i + l] = c[r];
@@ -267,7 +280,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
             const double d = As[16 * b + k][16 * b + k];
-            x[k] = quot(x[k], d, recip(d));
+            x[k] = quot<DIV>(x[k], d, recip<DIV>(d));
 #pragma unroll
             for (int i = k + 1; i < 16; ++i) x[i] = __builtin_fma(-As[16 * b + k][16 * b + i], x[k], x[i]);
         }
@@ -282,7 +295,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int c = 16 * b + 4 * q + g;
-            const double s = sqrt(ls->p[c]), v = quot(As[c][16 * i + l], s, recip(s));
+            const double s = sqrt(ls->p[c]), v = quot<DIV>(As[c][16 * i + l], s, recip<DIV>(s));
             if (i > b) As[16 * i + l][c] = v;
             else As[c][16 * i + l] = (4 * q + g == l) ? s : v;
         }
@@ -297,7 +310,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
                 a[c] = As[16 * b + c][16 * b + l];
                 z[c] = As[16 * b + c][16 * zb + l];
             }
-            piv = elim(a, z, l, std::make_integer_sequence<int, 16>());
+            piv = elim<DIV>(a, z, l, std::make_integer_sequence<int, 16>());
         }
         if (b == 0) __syncthreads();  // every wave is done with P
         if (w == 0) {
@@ -306,10 +319,14 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
                 for (int c = 0; c < 16; ++c) As[16 * b + c][16 * zb + l] = z[c];
             if (lane < 16) {
                 ls->p[16 * b + l] = piv;
-                ls->r[16 * b + l] = recip(piv);
+                ls->r[16 * b + l] = recip<DIV>(piv);
             }
-            const unsigned long long bad = __ballot(!(piv > 0.0));
-            if (bad && lane == 0 && ls->fail == 64) ls->fail = 16 * b + __ffsll(bad) - 1;
+            // the first pivot that is not positive, or that the fast quotients are not made for
+            const unsigned long long odd = __ballot(DIV ? !(piv > 0.0) : !(piv >= FAST_MIN && piv <= FAST_MAX));
+            if (odd && lane == __ffsll(odd) - 1 && ls->fail == 64 && !ls->again) {
+                if (!DIV && piv > 0.0) ls->again = 1;
+                else ls->fail = 16 * b + lane;
+            }
         } else if (b > 0 && w < 4) {
             // the rest of step b - 1: block columns beyond b, and the column's L
             int q = 0;
@@ -327,6 +344,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
         else if (b == 3 && w > 0 && w < 4) xrow_sum(3, w - 1);
         __syncthreads();
     }
+    if (!DIV && ls->again) return true;
     if (w == 0) xrow_solve(3);
     if (tid == 0 && ls->fail < 64) *info = k0 + ls->fail + 1;
 #pragma unroll
@@ -342,6 +360,7 @@ __device__ void leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
         const int c = w + 8 * u;
         D[lane + 64 * c] = (lane >= c) ? Xs[lane][c] : 0.0;
     }
+    return false;
 }
 
 // Step k of the factorisation of the lower triangle of A (destroyed) into L: workgroup 0
@@ -357,7 +376,10 @@ __global__ __launch_bounds__(CH_THREADS, 2) void chol_step_kernel(int n, T *A, l
     __shared__ int bad;
     if (blockIdx.x == 0) {
         if (k == 0 && threadIdx.x == 0) *info = 0;
-        leaf_role(n, A, lda, L, ldl, Dinv, k, kp, info, P0, P1, &ls);
+        if (leaf_role<T, false>(n, A, lda, L, ldl, Dinv, k, kp, info, P0, P1, &ls)) {
+            __syncthreads();
+            leaf_role<T, true>(n, A, lda, L, ldl, Dinv, k, kp, info, P0, P1, &ls);
+        }
         return;
     }
     const int nb = (n + 63) / 64;

@@ -53,3 +53,23 @@ def test_info_is_the_first_failing_column(potrf, dtype, n, flips):
     """info: the first column whose pivot is not positive, from 1, or 0."""
     _, info = potrf(_spd(n, np.random.default_rng(n), flips).astype(dtype))
     assert info == (min(flips) + 1 if flips else 0)
+
+
+# one block of 16 columns, one tile, several tiles; a subnormal, a normal and a huge scale
+@pytest.mark.parametrize("n", [1, 10, 16, 17, 40, 64])
+@pytest.mark.parametrize("scale", [2.0**-1040, 2.0**-1030, 2.0**-1000, 2.0**1018])
+def test_factor_at_the_ends_of_the_range(potrf, n, scale):
+    """S = scale B B^T for a small-integer B: its factor is sqrt(scale) B.  Every sum of the
+    elimination is a small multiple of scale, exact down to the smallest subnormal (2^-1074);
+    quotients by pivots of 25 scale round to u = 1.1e-16 and sums of n of them to n u of the
+    largest entry, 6, with n steps on the way: 50 n u.  Subnormal sums round to 2^-1074 / scale
+    more per step."""
+    rng = np.random.default_rng(n)
+    B = np.tril(rng.integers(-1, 2, (n, n)).astype(float), -1)
+    B[np.abs(np.subtract.outer(np.arange(n), np.arange(n))) > 3] = 0.0
+    B += 5.0 * np.eye(n)
+    L, info = potrf((B @ B.T) * scale)
+    assert info == 0
+    root = scale**0.5
+    tol = 50.0 * n * (1.1e-16 + 2.0**-1074 / scale)
+    assert np.max(np.abs(np.tril(L) / root - B)) <= tol
