@@ -357,6 +357,8 @@ def test_cg_solve_lower_triangle_product(gpu_lib, oracle, m, monkeypatch):
     assert rel(sols[0], sols[1]) < 1e-7
 
 
+# (these sizes take the step-by-step form; trailing updates on the second stream begin at 3073
+# rows, in test_cholesky_block_edges)
 @pytest.mark.parametrize("n", [257, 300, 520, 777])
 def test_blocked_cholesky_look_ahead(gpu_lib, n):
     """The blocked Cholesky with look-ahead (n > 4 panels of 64): trailing updates of

@@ -3,10 +3,11 @@ to a 1e-6 relative gap.
 
 Two kinds of instance:
   * sparse constraints (MaxCut, theta), and rank-one constraints with r < 32 n:
-    M is built in FP64 and only its preconditioner is FP32 (equilibrated
-    Cholesky); the CG stops on FP64 residuals at the reference's tolerances,
-    so the iterates agree to the solve tolerance: same status and iteration
-    count;
+    M is built in FP64 and only its preconditioner may be FP32 (equilibrated
+    Cholesky; from m = 65536 by itself, below where HDSDP_MIXED_CHOL32_MIN says
+    so, otherwise the run is the FP64 one); the CG stops on FP64 residuals at
+    the reference's tolerances, so the iterates agree to the solve tolerance:
+    same status and iteration count;
   * dense constraints (and rank-one ones when forced onto the bf16 Gram
     path): the Gram blocks of M come from bf16 split products (three terms per
     operand, FP32-equivalent, FP64 accumulation); once the factor preconditioner
@@ -71,7 +72,8 @@ def test_mixed_matches_fp64(gpu_lib, name, monkeypatch):
 
 # The two mixed-precision workloads at their own sizes: the dense random SDP n = 1000,
 # m = 2000 (every Gram block from bf16 planes) and the rank-one SDP n = 2000, m = 20000
-# in factor form (FP64 Gram, FP32 Cholesky preconditioner, lower-triangle CG products).
+# in factor form (FP64 Gram, lower-triangle CG products; its Cholesky preconditioner is FP64
+# by itself and FP32 in test_mixed_full_size_fp32_factor).
 FULL = {
     "dense_n1000_m2000": (lambda: I.dense_random(1000, 2000, 3), True),
     "rankone_n2000_m20000": (lambda: I.rank_one(2000, 20000, 20, 4), False),
@@ -112,6 +114,13 @@ def test_mixed_full_size(gpu_lib, name):
     else:
         assert rmx.iters == r64.iters
         assert abs(rmx.pobj - r64.pobj) <= 1e-8 * max(1.0, abs(r64.pobj))
+
+
+def test_mixed_full_size_fp32_factor(gpu_lib, monkeypatch):
+    """The rank-one instance of test_mixed_full_size, same bounds, with the FP32 Cholesky
+    preconditioner that larger systems take by themselves."""
+    monkeypatch.setenv("HDSDP_MIXED_CHOL32_MIN", "16384")
+    test_mixed_full_size(gpu_lib, "rankone_n2000_m20000")
 
 
 @pytest.mark.parametrize("name", ["dense_n120_m240", "rankone_n60_m500"])

@@ -176,3 +176,60 @@ def test_not_a_number_switches_to_the_direct_solver(gpu_lib, m):
     d.close()
     assert ldl == 1
     assert np.linalg.norm(M @ x - b) <= 1e-9 * np.linalg.norm(b)
+
+
+# diagonal blocks of 2048 rows and of 4096 (m = 10241), outer blocks of the FP32 Cholesky
+@pytest.mark.parametrize("m", [2048, 2049, 3073, 4097, 10241])
+def test_fp32_factor_by_blocks(gpu_lib, monkeypatch, m):
+    """Mixed precision with the FP32 factor of an FP64-built M (from m = 65536 by itself): the
+    factor's CG takes more than one iteration, which the FP64 factor never does, so the last
+    solve was not the fallback's; the residual is confirmed in FP64, 1e-11 |b|, to which numpy's
+    M adds 12 m u as above."""
+    monkeypatch.setenv("HDSDP_MIXED_CHOL32_MIN", "1")
+    rng = np.random.default_rng(m)
+    n = int(np.ceil(np.sqrt(2.2 * m)))
+    d, M = _system(gpu_lib, m, n, _mild(n, rng), rng, precision=1)
+    b = rng.standard_normal(m)
+    rel = 1e-11
+    d.kkt_params(rel, rel * np.linalg.norm(b), 5, -1)
+    assert _jacobi_cg(M, b, rel, rel * np.linalg.norm(b), 5)[0] == "limit"
+    assert d.kkt_factorize() == 0
+    before = _stats(d)
+    sols = []
+    for rhs in (b, -2.0 * b):
+        sols.append(d.kkt_solve(rhs))
+        got = _stats(d)
+        assert got["factored"] == before["factored"] + 1 and d.uses_ldl() == 0
+        assert 1 <= got["last"] < 5
+    d.close()
+    for rhs, x in zip((b, -2.0 * b), sols):
+        assert np.linalg.norm(M @ x - rhs) <= (rel + 12.0 * m * 1.1e-16) * np.linalg.norm(rhs)
+
+
+def test_fp32_factor_by_blocks_of_a_bf16_schur_matrix(gpu_lib):
+    """The same factor of a dense Schur matrix from the bf16 products at m > 2048, where mixed
+    precision takes it by itself: solves refined against the exact operator, to 1e-11 |b| here."""
+    n, m = 70, 2100
+    rng = np.random.default_rng(7)
+    S = _mild(n, rng)
+    C = dt.Coeff(dt.DENSE, n, val=np.concatenate([S[j:, j] for j in range(n)]))
+    d = dt.Dev(gpu_lib, [C] + [dt.rand_dense(rng, n) for _ in range(m)], 1)
+    d.update(1.0, 0.0, np.zeros(m), 0.0, 0)
+    assert d.factorize(0) == 1
+    d.schur(0, 0.0)
+    d.add_diag(0.1 * np.ones(m))
+    W = np.linalg.inv(S)
+    L = np.linalg.cholesky(0.5 * (W + W.T))
+    T = np.array([(L.T @ c.dense() @ L).ravel() for c in d.coeffs[1:]])
+    M = T @ T.T + 0.1 * np.eye(m)
+    b = rng.standard_normal(m)
+    rel = 1e-11
+    d.kkt_params(rel, rel * np.linalg.norm(b), 8, -1)
+    assert _jacobi_cg(M, b, rel, rel * np.linalg.norm(b), 8)[0] == "limit"
+    assert d.kkt_factorize() == 0
+    before = _stats(d)
+    x = d.kkt_solve(b)
+    got, ldl = _stats(d), d.uses_ldl()
+    d.close()
+    assert got["factored"] == before["factored"] + 1 and ldl == 0
+    assert np.linalg.norm(M @ x - b) <= (rel + 12.0 * m * 1.1e-16) * np.linalg.norm(b)
