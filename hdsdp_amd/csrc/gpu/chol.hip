@@ -53,7 +53,7 @@ __device__ inline double row_bcast(double v) {
 // rounded unless a / p lies within some 2^-53 ulp of the middle of two numbers (or |a| below
 // 2^-969 makes the residual underflow: an ulp then).  p and r have to be normal numbers: a tile
 // with a pivot outside FAST_MIN .. FAST_MAX is factored again with divisions (DIV), which
-// takes the step from 20 us to 38.
+// takes the step from 20 us to 27.
 constexpr double FAST_MIN = 0x1p-960, FAST_MAX = 0x1p960;
 
 template <bool DIV>
@@ -339,14 +339,18 @@ __device__ bool leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
             xrow_solve(b - 1);
         }
         __syncthreads();
+        if (ls->fail < 64 || ls->again) break;  // the same for every thread: wave 0 wrote them before the barrier
         if (w < 3 - b) trail(b + 1 + w, b + 1, b);
         else if (w == 4) scale(b, b);
         else if (b == 3 && w > 0 && w < 4) xrow_sum(3, w - 1);
         __syncthreads();
     }
     if (!DIV && ls->again) return true;
+    if (ls->fail < 64) {
+        if (tid == 0) *info = k0 + ls->fail + 1;
+        return false;
+    }
     if (w == 0) xrow_solve(3);
-    if (tid == 0 && ls->fail < 64) *info = k0 + ls->fail + 1;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
         const int c = w + 8 * u;
