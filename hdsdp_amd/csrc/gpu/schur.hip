@@ -727,9 +727,42 @@ __global__ __launch_bounds__(256) void xdots_sum_kernel(int cnt, const double *p
         out[threadIdx.x] = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
 }
 
-// One pass over both lower triangles on up to 256 workgroups; the one workgroup it replaces
-// walked all n^2 entries: n = 250 34 us against 3, n = 2000 1.7 ms.
+// The whole sums of a block of n <= XDOTS_ONE rows in one workgroup
+constexpr int XDOTS_ONE = 64;
+__global__ __launch_bounds__(1024) void xdots_one_kernel(int n, const double *X, const double *S, double *out) {
+    __shared__ double red[2][16];
+    double a = 0.0, t = 0.0;
+#pragma unroll
+    for (int q = 0; q < (XDOTS_ONE * XDOTS_ONE + 1023) / 1024; ++q) {
+        const int e = threadIdx.x + 1024 * q, j = e / n, i = e - j * n;
+        if (j >= n || i < j) continue;
+        const double x = X[e];
+        a += (i > j) ? 2.0 * x * S[e] : x * S[e];
+        if (i == j) t += x;
+    }
+    a = wave_sum(a);
+    t = wave_sum(t);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = a;
+        red[1][threadIdx.x >> 6] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double sum = 0.0;
+        for (int w = 0; w < 16; ++w) sum += red[threadIdx.x][w];
+        out[threadIdx.x] = sum;
+    }
+}
+
+// One pass over both lower triangles on up to 256 workgroups; one workgroup that walks all n^2
+// entries takes 34 us at n = 250 where this takes 3, and 1.7 ms at n = 2000.  On small blocks the
+// second launch costs more than it saves (the call that forms <X, S>, tr(X) and A(X), with
+// one launch here and with two: n = 20 39.0 and 41.4 us, n = 48 39.6 and 41.3).
 void xdots(hipStream_t s, int n, const double *X, const double *S, double *part, double *out) {
+    if (n <= XDOTS_ONE) {
+        xdots_one_kernel<<<1, 1024, 0, s>>>(n, X, S, out);
+        return;
+    }
     const int g = std::min(n, 256);
     xdots_kernel<<<g, 256, 0, s>>>(n, X, S, part);
     xdots_sum_kernel<<<1, 256, 0, s>>>(g, part, out);

@@ -658,3 +658,10 @@ def test_primal_dot_products(gpu_lib, n):
     u = 1.1e-16
     assert abs(xs - np.sum(X * S)) <= (2.0 * n + 600.0) * u * np.sum(np.abs(X * S))
     assert abs(tx - np.trace(X)) <= (n + 300.0) * u * np.sum(np.abs(np.diag(X)))
+
+
+# the edge of the one-workgroup sums (64 rows) and sizes of one to four passes
+@pytest.mark.parametrize("n", [3, 31, 32, 33, 45, 46, 56, 63, 64, 65])
+def test_primal_dot_products_of_small_blocks(gpu_lib, n):
+    """The same sums as above (same bounds) where one workgroup takes them whole."""
+    test_primal_dot_products(gpu_lib, n)
