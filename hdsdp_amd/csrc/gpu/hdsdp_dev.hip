@@ -492,6 +492,21 @@ void schur_apply_exact(hdsdp_dev *d, const double *x, double *y) {
 
 int cg_solve(hdsdp_dev *d);
 
+// Iterations queued before the next look at a Jacobi CG that has done iter of them.  A look
+// costs about 12 us, an iteration beyond the last one its product (m = 2000 20 us, m = 6000 90),
+// so batches grow with the iterations done, and less the larger the system.  Speed-up over
+// four launches and a look per iteration (in brackets: batches of 5 up to m = 2048, of 3
+// beyond), by iterations to convergence:
+//   m = 300:  1 1.38 (0.79), 3 1.48 (1.51), 17 1.91 (1.98), 60 2.34 (2.37)
+//   m = 3000: 1 1.08 (0.92), 4 1.36 (1.04), 14 1.57 (1.46), 71 1.59 (1.63)
+//   m = 6000: 1 1.18 (0.70), 4 1.16 (0.77), 13 1.12 (1.26), 73 1.24 (1.26)
+//   m = 9000: 1 1.06 (0.59), 4 1.05 (0.65), 14 1.04 (0.98), 72 1.04 (1.06)
+int cgj_batch(int m, int iter) {
+    if (m > 8192) return 1;
+    if (m > 4096) return (iter < 8) ? 1 : (iter < 16) ? 2 : 3;
+    return (iter == 0) ? 2 : (iter < 5 || m > 2048) ? 3 : 5;
+}
+
 // The Jacobi-preconditioned part of cg_solve_inner: the iterations are queued in batches
 // and decide on the device whether they go on (cgj_iter), the host looks once per batch.
 // Returns the CgStop reached and the iteration it was reached at, CG_RUNNING after maxIter
@@ -511,14 +526,11 @@ int cg_jacobi_solve(hdsdp_dev *d, int *pIter) {
         d->rhsStaged = false;
         return stop;
     }
-    // iterations queued between two looks: a look costs about two iterations of a small
-    // system, and half a batch runs for nothing at the end
-    const int batch = (m <= 2048) ? 5 : 3;
     hdk::cgj_start(d->st, m, d->crhs, d->jac, d->relTol, d->absTol, d->cr, d->cx, d->cz, d->cp, d->sc_d);
     symv_M(d, d->cp, d->cMp);
     int iter = 0, stop = hdk::CG_RUNNING;
     while (iter < d->maxIter) {
-        for (int left = std::min(batch, d->maxIter - iter); left > 0 || iter % restart == 6; --left) {
+        for (int left = std::min(cgj_batch(m, iter), d->maxIter - iter); left > 0 || iter % restart == 6; --left) {
             // a batch ends with an iteration that reports, never with a restart
             if (iter >= d->maxIter) break;
             if (iter % restart == 5) {

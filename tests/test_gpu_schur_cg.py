@@ -81,9 +81,10 @@ def _jacobi_cg(M, b, rel, absol, maxit):
 
 
 # one workgroup (m <= 256: 64 rows per lane and register, columns in LDS from 193), vector
-# steps in registers (1024 entries each, up to 6144) and the loops beyond
+# steps in registers (1024 entries each, up to 6144) and the loops beyond; queued batches change
+# at 2048, 4096 and 8192
 @pytest.mark.parametrize("m", [1, 2, 63, 64, 65, 128, 129, 192, 193, 255, 256, 257, 1024, 1025, 2048, 2049, 3073, 4097,
-                               6144, 6145])
+                               6144, 6145, 8193])
 def test_converges_as_numpy_does(gpu_lib, m):
     """|r| < 1e-11 |b| after numpy's number of iterations, one more or less where rounding
     decides, past a restart, without a factorisation; the solution is checked to 1e-10 |b|
