@@ -718,10 +718,8 @@ __global__ void place_diag_kernel(int n, int span, const double *Dinv, T *Linv, 
 // shorter last pair is in the same two launches; n = 500 takes 40 us (129 on 64-wide tiles
 // with launches of its own for that pair), n = 2000 172 (442).
 template <typename T>
-void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work, int span) {
-    if (span <= 0 || span > n) span = n;
-    place_diag_kernel<T><<<dim3(n, (span + 255) / 256), 256, 0, s>>>(n, span, Dinv, Linv, ldi);
-    for (int sz = NB; sz < span; sz *= 2) {
+static void trtri_levels(hipStream_t s, int n, const T *L, int ldl, T *Linv, int ldi, T *work, int from, int to) {
+    for (int sz = from; sz < to; sz *= 2) {
         int npair = n / (2 * sz);
         long strideL = 2L * sz * (ldl + 1), strideI = 2L * sz * (ldi + 1), strideW = (long) sz * sz;
         const int o = npair * 2 * sz, sc = std::max(0, n - o - sz);  // rows of a last, shorter pair
@@ -750,6 +748,13 @@ void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Lin
                     sc, 0, (T) 0, Linv + (o + sz) + (long) o * ldi, ldi, 0, 1, 2);
         }
     }
+}
+
+template <typename T>
+void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Linv, int ldi, T *work, int span) {
+    if (span <= 0 || span > n) span = n;
+    place_diag_kernel<T><<<dim3(n, (span + 255) / 256), 256, 0, s>>>(n, span, Dinv, Linv, ldi);
+    trtri_levels<T>(s, n, L, ldl, Linv, ldi, work, NB, span);
 }
 
 template void trtri<double>(hipStream_t, int, const double *, int, const double *, double *, int, double *, int);
@@ -868,10 +873,20 @@ void solve_prepare(hipStream_t s, int m, T *L, int ld, const double *Dinv, T *Li
     if (m > span) mirror_lower<T>(s, m, L, ld);
 }
 
+bool solve_in_blocks(int m) { return m > solve_span(m); }
+
+template <typename T>
+void solve_complete(hipStream_t s, int m, const T *L, int ld, T *Li, T *LiT) {
+    zero_upper<T>(s, m, Li, ld);
+    trtri_levels<T>(s, m, L, ld, Li, ld, LiT, solve_span(m), m);
+    transpose<T>(s, m, Li, ld, LiT, ld);
+}
+
 // z = L^-T L^-1 r; tmp: m entries; r, z and tmp distinct
 template <typename T>
-void solve_apply(hipStream_t s, int m, const T *L, int ld, const T *Li, const T *LiT, const T *r, T *z, T *tmp) {
-    const int span = solve_span(m);
+void solve_apply(hipStream_t s, int m, const T *L, int ld, const T *Li, const T *LiT, const T *r, T *z, T *tmp,
+                 bool complete) {
+    const int span = complete ? m : solve_span(m);
     if (m > span) (void) hipMemcpyAsync(z, r, sizeof(T) * m, hipMemcpyDeviceToDevice, s);
     const T *rhs = (m > span) ? z : r;
     int b0 = 0;
@@ -892,9 +907,10 @@ void solve_apply(hipStream_t s, int m, const T *L, int ld, const T *Li, const T 
 template void solve_prepare<double>(hipStream_t, int, double *, int, const double *, double *, double *);
 template void solve_prepare<float>(hipStream_t, int, float *, int, const double *, float *, float *);
 template void solve_apply<double>(hipStream_t, int, const double *, int, const double *, const double *,
-                                  const double *, double *, double *);
+                                  const double *, double *, double *, bool);
 template void solve_apply<float>(hipStream_t, int, const float *, int, const float *, const float *, const float *,
-                                 float *, float *);
+                                 float *, float *, bool);
+template void solve_complete<double>(hipStream_t, int, const double *, int, double *, double *);
 
 // ---- symmetric product from the lower triangle -----------------------------------
 

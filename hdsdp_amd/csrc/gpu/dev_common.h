@@ -158,7 +158,13 @@ void trtri(hipStream_t s, int n, const T *L, int ldl, const double *Dinv, T *Lin
 template <typename T>
 void solve_prepare(hipStream_t s, int m, T *L, int ld, const double *Dinv, T *Li, T *LiT);
 template <typename T>
-void solve_apply(hipStream_t s, int m, const T *L, int ld, const T *Li, const T *LiT, const T *r, T *z, T *tmp);
+void solve_apply(hipStream_t s, int m, const T *L, int ld, const T *Li, const T *LiT, const T *r, T *z, T *tmp,
+                 bool complete = false);
+// Where prepare inverts diagonal blocks only, solve_complete extends Li and LiT to the whole
+// inverse (m^3 / 3 flops) for apply with complete: half the launches per solve.
+bool solve_in_blocks(int m);
+template <typename T>
+void solve_complete(hipStream_t s, int m, const T *L, int ld, T *Li, T *LiT);
 
 // In-place LU with partial pivoting, P A = L U (L unit lower, U upper, both in A),
 // blocked by 64 columns.  ipiv (device, m ints): row interchanged with row c at step c,

@@ -98,6 +98,8 @@ struct hdsdp_dev {
     // Schur system; mVer counts changes of M, cholVer is the mVer its FP64 factor
     // (Mchol and the inverses of its diagonal blocks, MLi, MLiT) was computed from (-1: none)
     long mVer, cholVer;
+    int exactSolves;  // solve_exact calls that used this factor
+    bool MLiWhole;    // MLi and MLiT hold the whole inverse, not its diagonal blocks alone
     double *M, *Mchol, *MLi, *MLiT, *Md;  // Md: inverses of the diagonal blocks of either factor of M
     float *Mf, *MLif, *MLiTf, *cf1, *cf2, *cf3;
     double *jac, *cr, *crn, *cp, *cz, *cMp, *cx, *crhs, *ctmp;
@@ -380,6 +382,8 @@ hdsdp_retcode build_chol64(hdsdp_dev *d) {
     DCALL(sync(d));
     if (*d->hinfo != 0) return HDSDP_RETCODE_FAILED;
     hdk::solve_prepare<double>(d->st, m, d->Mchol, m, d->Md, d->MLi, d->MLiT);
+    d->exactSolves = 0;
+    d->MLiWhole = false;
     d->precKind = PREC_CHOL64;
     d->cholVer = d->mVer;
     return check_launch();
@@ -461,7 +465,7 @@ void apply_precond(hdsdp_dev *d, const double *r, double *z, double *p) {
         hdk::solve_apply<float>(d->st, m, d->Mf, m, d->MLif, d->MLiTf, d->cf1, d->cf3, d->cf2);
         hdk::f2d_scaled(d->st, m, d->cf3, d->precS, z);
     } else {
-        hdk::solve_apply<double>(d->st, m, d->Mchol, m, d->MLi, d->MLiT, r, z, d->ctmp);
+        hdk::solve_apply<double>(d->st, m, d->Mchol, m, d->MLi, d->MLiT, r, z, d->ctmp, d->MLiWhole);
     }
     if (p) hdk::cg_jacobi(d->st, m, z, nullptr, p, nullptr);
 }
@@ -1741,7 +1745,24 @@ hdsdp_retcode hdsdp_dev_kkt_solve(hdsdp_dev *d, const double *rhs, double *sol) 
 
 // z = (L L^T)^-1 r with the FP64 factor of M; tmp: m-vector.
 void apply_chol64(hdsdp_dev *d, const double *r, double *z, double *tmp) {
-    hdk::solve_apply<double>(d->st, d->m, d->Mchol, d->m, d->MLi, d->MLiT, r, z, tmp);
+    hdk::solve_apply<double>(d->st, d->m, d->Mchol, d->m, d->MLi, d->MLiT, r, z, tmp, d->MLiWhole);
+}
+
+// An exact solve applies the factor three times or more, and by block substitution each takes
+// 1.1 to 1.4 times as long as with the whole inverse (m = 2500 a solve 195 us against 143,
+// m = 8084 913 against 752, m = 20000 3.58 ms against 3.27).  Callers that solve again and again
+// with one factor (the adjoints of many losses at one point) get the whole inverse once
+// the solves have paid a part of it: then no number of them takes longer, the factorisation
+// included, than with the whole inverse from the start (ratio of the totals over 1 .. 120
+// solves: 1.02 at least; the inverse takes 0.2 ms at m = 2500, 4.7 at 8084, 45 at 20000).
+constexpr int WHOLE_AFTER = 400;
+
+void count_exact_solve(hdsdp_dev *d) {
+    const int m = d->m;
+    d->exactSolves += 1;
+    if (d->MLiWhole || !hdk::solve_in_blocks(m) || d->exactSolves <= m / WHOLE_AFTER) return;
+    hdk::solve_complete<double>(d->st, m, d->Mchol, m, d->MLi, d->MLiT);
+    d->MLiWhole = true;
 }
 
 // Direct FP64 solve of M x = rhs (FP64 Gram blocks, FP64 Cholesky, two refinement steps
@@ -1760,6 +1781,7 @@ hdsdp_retcode solve_exact(hdsdp_dev *d, const double *rhs, double *sol, bool reu
     hdk::mirror_lower<double>(d->st, m, d->M, m);
     DCALL(upload(d, d->crhs, rhs, m, d->hvecB));
     if (reuse && d->cholVer >= 0 && d->cholVer != d->mVer) {
+        count_exact_solve(d);
         apply_chol64(d, d->crhs, d->cx, d->ctmp);
         double z0 = -1.0, zprev = HUGE_VAL;
         bool ok = false;
@@ -1791,6 +1813,7 @@ hdsdp_retcode solve_exact(hdsdp_dev *d, const double *rhs, double *sol, bool reu
         DCALL(build_chol64(d));
         DCALL(prof_end(d, HDSDP_PROF_MFACTOR));
     }
+    count_exact_solve(d);
     apply_chol64(d, d->crhs, d->cx, d->ctmp);
     for (int it = 0; it < 2; ++it) {
         symv_M(d, d->cx, d->crn);

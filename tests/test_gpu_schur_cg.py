@@ -234,3 +234,35 @@ def test_fp32_factor_by_blocks_of_a_bf16_schur_matrix(gpu_lib):
     d.close()
     assert got["factored"] == before["factored"] + 1 and ldl == 0
     assert np.linalg.norm(M @ x - b) <= (rel + 12.0 * m * 1.1e-16) * np.linalg.norm(b)
+
+
+# first size in blocks, ragged last pairs of the whole inverse's levels, the wider span
+@pytest.mark.parametrize("m", [2048, 2049, 2500, 4097, 6200, 10241])
+def test_repeated_exact_solves(gpu_lib, m):
+    """kkt_solve_exact again and again with one factor, past the point (m / 400) where the inverse
+    of the factor is completed, then the CG with that factor, then a new factor: 12 m u of
+    |b| for the refined solves as in test_schur_solve_by_blocks, the tolerance for the CG."""
+    rng = np.random.default_rng(m)
+    n = int(np.ceil(np.sqrt(2.2 * m)))
+    d, M = _system(gpu_lib, m, n, _mild(n, rng), rng)
+    x = np.zeros(m)
+
+    def exact(b):
+        assert gpu_lib.hdsdp_dev_kkt_solve_exact(d.h, _capi.dptr(b), _capi.dptr(x)) == 0
+        return np.linalg.norm(M @ x - b) / np.linalg.norm(b)
+
+    for _ in range(m // 400 + 3):
+        assert exact(rng.standard_normal(m)) <= 12.0 * m * 1.1e-16
+    rel = 1e-11
+    b = rng.standard_normal(m)
+    # a Jacobi CG of one iteration, then the factor of the same M
+    d.kkt_params(rel, rel * np.linalg.norm(b), 1, -1)
+    assert d.kkt_factorize() == 0
+    y = d.kkt_solve(b)
+    assert np.linalg.norm(M @ y - b) <= (rel + 12.0 * m * 1.1e-16) * np.linalg.norm(b)
+    d.add_diag(np.ones(m))
+    M[np.diag_indices(m)] += 1.0
+    for _ in range(2):
+        assert exact(rng.standard_normal(m)) <= 12.0 * m * 1.1e-16
+    assert d.uses_ldl() == 0
+    d.close()
