@@ -428,6 +428,13 @@ hdsdp_retcode build_chol32(hdsdp_dev *d, int *ok) {
     return check_launch();
 }
 
+// whether the FP64 factor of M and its inverses fit on the device beside what is there
+bool chol64_fits(hdsdp_dev *d) {
+    size_t left = 0, all = 0;
+    if (d->Mchol || hipMemGetInfo(&left, &all) != hipSuccess) return true;
+    return left >= sizeof(double) * (3 * (size_t) d->m * d->m + hdk::chol_dinv_len(d->m)) + ((size_t) 256 << 20);
+}
+
 hdsdp_retcode build_precond(hdsdp_dev *d) {
     const int m = d->m;
     if (d->useJacobi) {
@@ -439,10 +446,12 @@ hdsdp_retcode build_precond(hdsdp_dev *d) {
     prof_begin(d, HDSDP_PROF_MFACTOR);
     // Mixed precision factors M in FP32 when its Gram blocks are bf16 products (an FP32-
     // accurate matrix), or when M is so large that three FP64 matrices beside it are a
-    // question of memory (m = 65536: 137 GB in all).  Below, the FP64 factor is the faster one:
-    // at m = 20000 the FP32 factorisation saves 1.5 ms per iteration and its coarser
-    // preconditioner costs 22 ms of CG (0.219 s per iteration against 0.197); m = 8084 1.7 and 7.
-    if (d->precision == HDSDP_PRECISION_MIXED && (d->mGramPending || d->m >= d->chol32Min)) {
+    // question of memory (m = 65536: 137 GB in all; from m = 16384, 6.4 GB, where they do not
+    // fit).  Otherwise the FP64 factor is the faster one: at m = 20000 the FP32 factorisation
+    // saves 1.5 ms per iteration and its coarser preconditioner costs 22 ms of CG (0.219 s per
+    // iteration against 0.197); m = 8084 1.7 and 7.
+    if (d->precision == HDSDP_PRECISION_MIXED &&
+        (d->mGramPending || m >= d->chol32Min || (m >= 16384 && !chol64_fits(d)))) {
         int ok = 0;
         DCALL(build_chol32(d, &ok));
         if (!ok) DCALL(build_chol64(d));
