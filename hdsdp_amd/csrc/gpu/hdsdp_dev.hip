@@ -791,6 +791,21 @@ hdsdp_retcode alloc_dense_gram(hdsdp_dev *d) {
     return HDSDP_RETCODE_OK;
 }
 
+// Whether the FP64 build as planned fits on the device with all that is allocated after it: the
+// Gram parts, the primal method's and the Schur factor's matrices and, in mixed precision, the bf16 or
+// FP32 operands.  The padded panels take up to a quarter more than T_p one after the other
+// (n = 8000 with 513 constraints 164 GB against 131) and 1 GB more of batches.
+bool dense_gram_fits(hdsdp_dev *d, bool mixed) {
+    size_t left = 0, all = 0;
+    if (hipMemGetInfo(&left, &all) != hipSuccess) return true;
+    const size_t m = d->m, n = d->n, r = d->nDn, nl = (size_t) d->gramLd * d->gramRows;
+    size_t need = (size_t) d->gramK1 / 16 * d->gramSlab + d->gramLd * r + nl * (2 * (size_t) d->gramBatch + 1);
+    need += r * r * (d->gramParts + 17) + 4 * m * m + 10 * n * n;
+    need *= sizeof(double);
+    if (mixed) need += 6 * (2 * n * n * r + nl * (2 * (size_t) d->gramBatch + 1));
+    return need + ((size_t) 256 << 20) <= left;
+}
+
 // Rebuild the Gram blocks of M in FP64 from the factor of their build, re-apply the
 // diagonal terms added since, and keep later builds in FP64.
 hdsdp_retcode rebuild_gram_fp64(hdsdp_dev *d) {
@@ -1268,7 +1283,6 @@ hdsdp_retcode hdsdp_dev_load(hdsdp_dev *d, const hdsdp_coeff_view *cv) {
     if (d->dnGram) {
         const size_t nn = (size_t) n * n;
         const int r = d->nDn;
-        d->gramBatch = (int) std::max<size_t>(1, std::min<size_t>(r, (size_t) (512u << 20) / (nn * sizeof(double))));
         // FP64 build, from GRAM_HALF_MIN on with enough 128-wide lower tiles: every operand is
         // padded with zeros to whole tiles, so that no slab takes the bounds-checked loads (at
         // n = 1000 a third of the products' work lies in ragged tiles), and the T_p are kept
@@ -1279,30 +1293,35 @@ hdsdp_retcode hdsdp_dev_load(hdsdp_dev *d, const hdsdp_coeff_view *cv) {
         // summation is kept).
         long tiles = (long) ((r + 127) / 128) * ((r + 127) / 128 + 1) / 2;
         long want = std::min<long>(16, std::max<long>(1, (2048 + tiles - 1) / tiles));
-        d->gramK1 = std::max<long>(2, (long) n * (n - 1) / 2);
-        long parts = hdk::splitk_parts(r, r, d->gramK1, true, 16);
-        const bool panels = n >= GRAM_HALF_MIN && tiles * parts >= 192;
-        d->gramRows = panels ? (n + 127) / 128 * 128 : n;
-        d->gramLd = panels ? d->gramRows : (n + 1) & ~1;
-        d->gramSlab = panels ? 16L * ((r + 127) / 128 * 128) : 0;
-        if (panels) {
-            d->gramK1 = (d->gramK1 + 15) / 16 * 16;
-            d->gramChunk = ((d->gramK1 + parts - 1) / parts + 15) / 16 * 16;
-            // a batch of 1 GB: each launch ends with a round of partly filled CUs
+        const long K0 = std::max<long>(2, (long) n * (n - 1) / 2);
+        const long parts0 = hdk::splitk_parts(r, r, K0, true, 16);
+        auto plan = [&](bool panels) {
+            long parts = panels ? parts0 : want;
+            d->gramK1 = panels ? (K0 + 15) / 16 * 16 : K0;
+            d->gramRows = panels ? (n + 127) / 128 * 128 : n;
+            d->gramLd = panels ? d->gramRows : (n + 1) & ~1;
+            d->gramSlab = panels ? 16L * ((r + 127) / 128 * 128) : 0;
+            if (panels) {
+                d->gramChunk = ((K0 + 15) / 16 * 16 + parts - 1) / parts;
+                d->gramChunk = (d->gramChunk + 15) / 16 * 16;
+            } else {
+                for (long p = want; p <= 2 * want; ++p)
+                    if (K0 % p == 0 && K0 / p >= 256) {
+                        parts = p;
+                        break;
+                    }
+                d->gramChunk = (K0 % parts == 0) ? K0 / parts : std::max<long>(256, (K0 + parts - 1) / parts);
+            }
+            // batches of 512 MB, of 1 GB with the panels: each launch ends with a round of partly
+            // filled CUs
+            const size_t each = panels ? (size_t) d->gramLd * d->gramRows : nn;
             d->gramBatch = (int) std::max<size_t>(
-                1, std::min<size_t>(r, ((size_t) 1 << 30) / ((size_t) d->gramLd * d->gramRows * sizeof(double))));
-        } else {
-            parts = want;
-            for (long p = want; p <= 2 * want; ++p)
-                if (d->gramK1 % p == 0 && d->gramK1 / p >= 256) {
-                    parts = p;
-                    break;
-                }
-            d->gramChunk = (d->gramK1 % parts == 0) ? d->gramK1 / parts
-                                                    : std::max<long>(256, (d->gramK1 + parts - 1) / parts);
-        }
-        const long K = d->gramK1;
-        d->gramParts = (int) ((K + d->gramChunk - 1) / d->gramChunk);
+                1, std::min<size_t>(r, ((size_t) (panels ? 1024 : 512) << 20) / (each * sizeof(double))));
+            d->gramParts = (int) ((d->gramK1 + d->gramChunk - 1) / d->gramChunk);
+        };
+        const bool panels = n >= GRAM_HALF_MIN && tiles * parts0 >= 192;
+        plan(panels);
+        if (panels && !dense_gram_fits(d, mixedGram)) plan(false);
         const size_t K1 = std::max<size_t>(1, (size_t) n * (n - 1) / 2);
         if (mixedGram && d->planes) {
             // planes: operands zero outside their true extent (k padding of the products)

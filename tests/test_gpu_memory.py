@@ -68,3 +68,27 @@ def test_mixed_factor_in_fp32_where_fp64_does_not_fit(gpu_lib, leave):
     Y = W @ X @ W
     Mx = np.where(r == c, 1.0, 2.0)[pick] * Y[r[pick], c[pick]] + x
     assert np.linalg.norm(Mx - b) <= 2.0 * rel * np.linalg.norm(b)
+
+
+def test_dense_build_without_panels_where_they_do_not_fit(gpu_lib, leave):
+    """513 dense constraints at n = 900: 1.7 GB of coefficients, then 1.7 GB of T_p and two batches
+    of 0.5 GB laid out plainly, 2.1 GB and two of 1 GB in panels padded to 640 constraints.
+    With 5.2 GB in all the problem loads, and M is that of the panels (25 n u as in
+    test_dense_gram_build)."""
+    n, m = 900, 513
+    rng = np.random.default_rng(2)
+    S = _mild(n, rng)
+    co = [dt.Coeff(dt.DENSE, n, val=np.concatenate([S[j:, j] for j in range(n)]))]
+    co += [dt.rand_dense(rng, n) for _ in range(m)]
+    got = []
+    for free in (None, 5.2 * GB):
+        if free:
+            leave(int(free))
+        d = dt.Dev(gpu_lib, co)
+        d.update(1.0, 0.0, np.zeros(m), 0.0, 0)
+        assert d.factorize(0) == 1
+        d.schur(0, 0.0)
+        got.append(d.get_schur())
+        d.close()
+    assert not np.array_equal(got[0], got[1])  # the two layouts sum in another order
+    assert np.max(np.abs(got[0] - got[1])) <= 25.0 * n * 1.1e-16 * np.max(np.abs(got[0]))
