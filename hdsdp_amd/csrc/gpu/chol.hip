@@ -17,9 +17,9 @@
 //    the products of the block's inverse are 16 x 16 x 16 MFMA products on the other
 //    waves.
 //
-// A block column takes 21 us this way against 52 us as three launches (an eight-wave
+// A block column takes 20 us this way against 52 us as three launches (an eight-wave
 // leaf with an LDS round trip and a barrier per column, a panel product, an update):
-// n = 500: 170 us, n = 1000: 340 us, n = 2000: 705 us (1.8 ms before), m = 8084: 6.7 ms.
+// n = 500: 160 us, n = 1000: 325 us, n = 2000: 680 us (1.8 ms before), m = 8084: 6.5 ms.
 // Results are those of the unblocked leaf bit for bit up to n = 64 CH_FLAT; an elimination
 // with reciprocals instead of correctly rounded quotients took 16 us per block column,
 // but the interior-point path amplifies its rounding into other iterates.
@@ -370,7 +370,7 @@ __device__ bool leaf_role(int n, const T *A, long lda, T *L, long ldl, double *D
 // Step k of the factorisation of the lower triangle of A (destroyed) into L: workgroup 0
 // factors the diagonal tile (k, k); the others apply panel kp = k - 1 to the tiles (i, j),
 // k <= j < jEnd, j <= i, and write L(i, kp).  kp < 0: nothing to apply (grid of one).
-// One workgroup per CU (210 registers); capped at 128 registers, for two per CU, the leaf
+// One workgroup per CU (214 registers); capped at 128 registers, for two per CU, the leaf
 // spills and the step takes 23 us.
 template <typename T>
 __global__ __launch_bounds__(CH_THREADS, 2) void chol_step_kernel(int n, T *A, long lda, T *L, long ldl, double *Dinv,
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(CH_THREADS) void chol_panel_kernel(int n, const T *
 // rank-(64 CH_OUTER) product: the part on the next outer block on s, the rest on the
 // second stream beside the next block's steps.  The line lies where the step by step
 // form's tiles (a rank-64 update each, with its panel blocks formed again) outgrow the
-// chip: m = 2300 takes 1.0 ms in outer blocks and 0.8 ms flat, m = 8084 6.7 ms in outer
+// chip: m = 2300 takes 1.0 ms in outer blocks and 0.8 ms flat, m = 8084 6.5 ms in outer
 // blocks, where one flat step alone would hold 8000 tiles of 7 us on 256 CUs.  At
 // m = 20000 the outer blocks take 55 ms (48 TF; 61 ms with outer blocks of 4, 57 of 6, 56
 // of 8 and of 16), the paired rank-64 updates before them 105 ms.

@@ -733,11 +733,11 @@ int cg_solve(hdsdp_dev *d) {
 // From n = GRAM_HALF_MIN: T(i, j) sums U(i, k) L^-1(j, k) over k <= j <= i, so of
 // U = L^-1 A_p the lower triangle is formed only: n^3 / 3 + n^3 / 6 multiply-adds per
 // constraint (n = 1000, 1000 constraints: 16 and 9 ms; <T_p, T_q> 9 ms, 64 TF).  Below,
-// the full U and T_p = L^-1 U^T, n^3 / 2 + n^3 / 3 (26 and 18 ms at that size): there the products are a small share of the build, and the
-// Lanczos step bound that the Schur solutions feed, run without reorthogonalisation to a
-// good part of n steps, turns a last-bit change of M into one of up to 4e-3 (n = 121;
-// 2e-9 at n = 300, 1e-12 at n = 700).  Where the products run on 128-wide tiles, T_p is stored
-// packed by the product itself.
+// the full U and T_p = L^-1 U^T, n^3 / 2 + n^3 / 3 (26 and 18 ms at that size): there the
+// products are a small share of the build, and the Lanczos step bound that the Schur solutions
+// feed, run without reorthogonalisation to a good part of n steps, turns a last-bit change of M
+// into one of up to 4e-3 (n = 121; 2e-9 at n = 300, 1e-12 at n = 700).  T_p is stored packed by
+// the product itself, whatever its tiles.
 constexpr int GRAM_HALF_MIN = 512;
 
 void dense_gram(hdsdp_dev *d, const double *Li) {

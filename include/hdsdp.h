@@ -162,7 +162,9 @@ hdsdp_retcode HDSDPSetup( hdsdp *HSolver );
 hdsdp_retcode HDSDPGetBarrierPoint( hdsdp *HSolver, double *mu, double *y );
 
 /* Damped Newton from y (in/out, S(y) positive definite) to y_mu, until
- * ||b - mu A(S^-1)|| <= tol (1 + ||b||) or maxIter steps (FAILED then).
+ * ||b - mu A(S^-1)|| <= tol (1 + ||b||) or maxIter steps (FAILED then; steps beyond the
+ * guaranteed one that end so are taken back and the path begun again without them, with
+ * maxIter steps of its own).
  * Leaves the dual factor and Schur matrix of the final y on the device. */
 hdsdp_retcode HDSDPCenter( hdsdp *HSolver, double mu, double *y, int maxIter, double tol,
                            int *nIter, double *relRes );
